@@ -586,7 +586,7 @@ class Ensemble:
 
     def autotune(self, steps=3):
         """Batched ensembles: time each x-pass plane-range plan, then the tile
-        shapes (z-rows per x-pass wavefront, modes per solve wavefront) over
+        shapes (z-rows per x-pass wavefront, rows per solve segment) over
         `steps` replayed steps each (every member's state restored after
         each), keep the fastest; returns its ms per step."""
         ms = C.c_double(0.0)

@@ -492,8 +492,9 @@ FFTPlan make_plan(int n, int tw_offset) {
 // One batched launch: the channels of one transform length (or segment
 // length) and the work list that covers all their workgroups.
 struct BatchLaunch {
-  int len = 0;                 // nz2 (z-transforms), nx2/2 (x-pass) or rows per segment (solve)
+  int len = 0;                 // nz2 (z-transforms), nx2/2 (x-pass) or solve_wg_layout (solve)
   int rw = 1, nxh = 0;         // x-pass: z-rows per wavefront, largest nx/2+1 of the members
+  int ny = 0;                  // solve: largest ny of the members
   void* args = nullptr;        // device array of per-channel arguments
   BatchItem* items = nullptr;  // device work list
   int nitems = 0;
@@ -527,8 +528,8 @@ struct chan_ensemble {
   // spread over its resident workgroups times xmul (0: the number of lengths)
   int xmul = 0;
   // launch-plan overrides the autotuner may choose: one z-row per x-pass
-  // wavefront at every length; 4 modes per solve wavefront everywhere
-  int xrows1 = 0, solve4 = 0;
+  // wavefront at every length; 5 rows per solve segment everywhere
+  int xrows1 = 0, solve5 = 0;
 };
 
 namespace {
@@ -557,7 +558,7 @@ std::string batch_ineligible(const chan_ctx* c, bool lin) {
   if (!zt_batchable(g.nz2)) return "nz2 has no compile-time transform plan";
   if (!xpass_batchable(g.nx2 / 2)) return "nx2/2 has no wavefront x-pass";
   if (g.nz > 192) return "nz above 192";
-  if (!solve_seg_rows(c->prm.ny)) return "ny+1 rows do not fit the segmented solve";
+  if (!solve_batchable(c->prm.ny)) return "ny+1 rows do not fit the segmented solve";
   if (3.0 * c->nyp * (double)c->nmodes * 16.0 >= 4.0e9) return "the segmented solve's 32-bit offsets";
   const Tuning& t = c->tune;
   if (!(t.xpass_wave == 1 && t.zfwd_v2 == 1 && t.zinv_kx == 8 && (t.solve_seg == 1 || t.solve_seg == 3) &&
@@ -694,7 +695,7 @@ void ensemble_plan_batched(chan_ensemble* e) {
   }
   // the segmented solve, one table per substep
   auto layout = [e](chan_ctx* c) {
-    return e->solve4 ? 64 + solve_seg_rows(c->prm.ny) : solve_seg_layout(c->prm.ny, c->tune.solve_seg);
+    return solve_wg_layout(c->prm.ny, e->solve5 ? 2 : c->tune.solve_seg);
   };
   for (int rk = 1; rk <= 3; ++rk) {
     e->solve[rk - 1] = plan_batches<SBatchArgs>(
@@ -711,10 +712,12 @@ void ensemble_plan_batched(chan_ensemble* e) {
           return x;
         },
         [&](chan_ctx* c, unsigned short k, std::vector<BatchItem>& it) {
-          const int modes = layout(c) / 16;
-          push_grid(it, k, (int)((nmodes(c) + modes - 1) / modes), 1);
+          push_grid(it, k, (int)((nmodes(c) + 7) / 8), 1);   // 8 modes per workgroup
         },
         [](chan_ctx* c) { return (long)c->nmodes * c->nyp; });
+    for (BatchLaunch& b : e->solve[rk - 1])
+      for (chan_ctx* c : e->m)
+        if (layout(c) == b.len) b.ny = std::max(b.ny, c->prm.ny);
   }
   std::vector<CflBatchArgs> cf;
   std::vector<FillBatchArgs> fc;
@@ -769,7 +772,7 @@ void ensemble_step_batched(chan_ensemble* e, hipStream_t s) {
     });
     if (rk == 1) launch_cfl_finalize_batched(e->cfl_args, n, 1, s);
     phase(e->solve[rk - 1], [&](const BatchLaunch& b, hipStream_t st) {
-      launch_solve_batched(b.len, (const SBatchArgs*)b.args, b.items, b.nitems, st);
+      launch_solve_batched(b.len, b.ny, (const SBatchArgs*)b.args, b.items, b.nitems, st);
     });
   }
   launch_advance_time_batched(e->scs, n, s);
@@ -1771,9 +1774,8 @@ int chan_autotune(chan_ctx* c, int steps, double* best_ms) {
     // Candidates: the x-pass kernel (the wavefront kernel only when a
     // subgrid closure is configured: it alone adds the stress to the fluxes)
     // and, for the wavefront kernel, its z-rows per wavefront where the
-    // length has them; the z-forward kernel; the segmented solve's layouts
-    // (4, 2 or 8 modes per wavefront where ny + 1 rows fit) or the
-    // sweep-based solves with their block shapes.
+    // length has them; the z-forward kernel; the segmented solve's rows per
+    // segment or the sweep-based solves with their block shapes.
     const int M = c->gd.nx2 / 2;
     const bool pf = c->tune.xpass_prefetch == 1 && M <= 144;
     std::vector<int> rows_c = {0};
@@ -1781,9 +1783,8 @@ int chan_autotune(chan_ctx* c, int steps, double* best_ms) {
       if (xpass_rows(M, c->gd.nz2, r, pf, false) == r && r != xpass_rows(M, c->gd.nz2, 0, pf, false))
         rows_c.push_back(r);
     std::vector<int> seg_c;
-    if (solve_seg_rows(c->prm.ny)) seg_c.push_back(1);
-    if (solve_seg_rows(c->prm.ny, 32) == 5) seg_c.push_back(2);
-    if (solve_seg_rows(c->prm.ny, 8)) seg_c.push_back(3);
+    if (solve_wg_seg(c->prm.ny, 1)) seg_c.push_back(1);
+    if (solve_wg_seg(c->prm.ny, 2) != solve_wg_seg(c->prm.ny, 1)) seg_c.push_back(2);
     std::vector<Tuning> cand;
     for (int w : {1, 0})
       for (int z : {1, 0}) {
@@ -1956,7 +1957,7 @@ int chan_ensemble_autotune(chan_ensemble* e, int steps, double* best_ms) {
   if (!e) return fail(nullptr, "null ensemble");
   std::vector<void*> bk;
   hipEvent_t a = nullptr, b = nullptr;
-  const int xmul0 = e->xmul, xrows0 = e->xrows1, solve0 = e->solve4;  // kept if the tuning fails
+  const int xmul0 = e->xmul, xrows0 = e->xrows1, solve0 = e->solve5;  // kept if the tuning fails
   auto cleanup = [&] {
     for (void* p : bk) dfree(p);
     bk.clear();
@@ -2035,10 +2036,10 @@ int chan_ensemble_autotune(chan_ensemble* e, int steps, double* best_ms) {
     copy_state(false);
     saved = true;
     // the x-pass plane ranges with the default tile shapes, then the tile
-    // shapes (one z-row per x-pass wavefront; 4 modes per solve wavefront)
+    // shapes (one z-row per x-pass wavefront; 5 rows per solve segment)
     // with the best ranges
     e->xrows1 = 0;
-    e->solve4 = 0;
+    e->solve5 = 0;
     for (int m : {0, 1, 2, 4, 8}) {
       e->xmul = m;
       const double ms = trial();
@@ -2047,14 +2048,14 @@ int chan_ensemble_autotune(chan_ensemble* e, int steps, double* best_ms) {
     e->xmul = bestm;
     for (int v : {1, 2, 3}) {
       e->xrows1 = v & 1;
-      e->solve4 = v >> 1;
+      e->solve5 = v >> 1;
       const double ms = trial();
-      if (ms < best) { best = ms; bestr = e->xrows1; bests = e->solve4; }
+      if (ms < best) { best = ms; bestr = e->xrows1; bests = e->solve5; }
     }
     if (!(best < 1e300)) throw chan_error("autotune: every plan's trial steps failed the CFL check");
     e->xmul = bestm;
     e->xrows1 = bestr;
-    e->solve4 = bests;
+    e->solve5 = bests;
     ensemble_release(e);
     cleanup();
     if (best_ms) *best_ms = best;
@@ -2068,7 +2069,7 @@ int chan_ensemble_autotune(chan_ensemble* e, int steps, double* best_ms) {
   cleanup();
   e->xmul = xmul0;
   e->xrows1 = xrows0;
-  e->solve4 = solve0;
+  e->solve5 = solve0;
   ensemble_release(e);  // the next step plans and captures again
   return 1;
 }

@@ -440,39 +440,61 @@ __device__ __forceinline__ double2 shfl2(double2 v, int src) {
 }
 
 // ---------------------------------------------------------------------------
-// Segmented column solve: the whole y column of every mode stays on chip.
+// Segmented column solve (k_solve_wg): the whole y column of every mode stays
+// on chip.
 //
-// A wavefront owns MODES consecutive (kx,kz) modes; lane (s, q) = (lane /
-// MODES, lane % MODES) owns rows s*SEG .. s*SEG+SEG-1 of mode q, all three
-// velocity components and the pressure correction, in registers.  The last
-// segment holds the remaining 3..SEG rows; rows past ny are identity padding.
-// Each tridiagonal system (u and w with D2H, v with D2N, the Neumann Poisson
-// system) is solved by partition (seg_eliminate, seg_separators, seg_backsub):
+// A workgroup owns 8 consecutive (kx,kz) modes; thread (s, q) = (tid / 8,
+// tid % 8) owns rows s*SEG - f .. s*SEG - f + SEG-1 of mode q, all three
+// velocity components and the pressure correction, in registers.  Each
+// tridiagonal system (u and w with D2H, v with D2N, the Neumann Poisson
+// system) is solved by partition (seg_eliminate, sep_row / sep_reduce,
+// seg_backsub):
 //   1. every segment eliminates its interior rows top-down, carrying the
 //      coupling to the separator below it (the previous segment's last row)
 //      as a second right-hand side; the coupling to the separator above it
 //      (its own last row, except in the last segment) stays in c';
 //   2. with the interiors eliminated, the separators form a tridiagonal
-//      system of (active segments - 1) unknowns per mode, solved by parallel
-//      cyclic reduction over lane shuffles;
+//      system of (segments - 1) unknowns per mode, solved by parallel cyclic
+//      reduction through LDS;
 //   3. every segment back-substitutes with both separators known.
-// The state is read once (NL, R and P; the NL and P rows are kept in LDS for
-// the pressure update and the next RK register) and written once (u, P, R):
-// no scratch array.  The arithmetic per row is that
-// of k_solve; only the elimination order of the solves differs, so results
-// agree with it to rounding.
+// The state is read once (NL, R and P) and written once (u, P, R): no scratch
+// array.  The arithmetic per row is that of k_solve; only the elimination
+// order of the solves differs, so results agree with it to rounding.
+//
+// What bounds it, and why this shape (192x129x192, SEG = 5, one substep):
+//  - Row accesses of 8 modes are whole 128-byte lines.  A copy of this
+//    kernel's loads and stores alone takes 109 us with 8 modes per row piece,
+//    147 us with 4 (64-byte pieces), 95 us with 16, whose workgroups are too
+//    large for the arithmetic's registers.  The whole kernel takes 139 us
+//    (3.9 TB/s); a form with 4 modes and 16 nine-row segments in one
+//    wavefront took 206 us.  201 rows (128x200x64) take 75 us, 334 us with
+//    the sweep-based k_solve3 that served columns above 144 rows before.
+//  - Two workgroups of four wavefronts share a compute unit (256 registers,
+//    75 KB of LDS each), so that one's loads and stores run beside the
+//    other's arithmetic: a workgroup spends about 8 us on its loads, 14 us on
+//    the solves and 6 us on its stores.
+//  - Nothing waits for a load before the last load is issued: the NL rows
+//    (needed again for the next RK register) and the operators go straight to
+//    LDS.  From then on no vector load is issued, which on this chip would
+//    wait for the stores in front of it.
+//  - The wall rows and the mean mode are patched behind branches that the
+//    other wavefronts skip; as selects they were a third of the instructions
+//    (181 -> 154 us together with the loads' order and the Newton reciprocal
+//    of the pivots).
 // ---------------------------------------------------------------------------
 
+// 1 / b for a pivot (finite, nonzero): the hardware estimate and two Newton
+// steps, within an ulp; half the instructions of the IEEE division.
+__device__ __forceinline__ double pivot_rcp(double b) {
+  double r = __builtin_amdgcn_rcp(b);
+  r = fma(r, fma(-b, r, 1.0), r);
+  return fma(r, fma(-b, r, 1.0), r);
+}
+
 // Partitioned solve of NC right-hand sides X[c][0..SEG) that share one
-// matrix, in three calls so that independent systems can be interleaved:
-//   seg_eliminate  - step 1 (coef(t, a, b, c) gives row t of this lane's
-//                    segment) and the relation of the segment's row 0 to
-//                    its two separators;
-//   seg_separators - step 2: the separator equations, solved by parallel
-//                    cyclic reduction across the segment lanes of each mode
-//                    (log2 of the segment count steps of lane shuffles);
-//   seg_backsub    - step 3.
-// ns segments are active; lanes past them carry identity rows.
+// matrix, in pieces so that independent systems can be interleaved:
+// seg_eliminate is step 1 (coef(t, a, b, c) gives row t of this thread's
+// segment) and the relation of the segment's row 0 to its two separators.
 template <int SEG, int NC>
 struct SegSys {
   double cp[SEG], gp[SEG];  // c' and the coupling to the separator below
@@ -493,7 +515,7 @@ __device__ __forceinline__ void seg_eliminate(double2 (&X)[NC][SEG], SegSys<SEG,
     coef(t, a_, b_, c_);
     if (t == SEG - 1) { S.aT = a_; S.bT = b_; S.cT = c_; }
     const double bp = (t == 0) ? b_ : b_ - a_ * S.cp[t - 1];
-    const double inv = 1.0 / bp;
+    const double inv = pivot_rcp(bp);
     S.cp[t] = c_ * inv;
     S.gp[t] = (t == 0) ? (-a_) * inv : (-(a_ * S.gp[t - 1])) * inv;
 #pragma unroll
@@ -520,60 +542,6 @@ __device__ __forceinline__ void seg_eliminate(double2 (&X)[NC][SEG], SegSys<SEG,
   }
 }
 
-template <int MODES, int SEG, int NC>
-__device__ __forceinline__ void seg_separators(const double2 (&X)[NC][SEG], const SegSys<SEG, NC>& S, int lane,
-                                               int ns, double2 (&xl)[NC], double2 (&xr)[NC]) {
-  constexpr int SEGS = 64 / MODES;
-  const int s = lane / MODES;
-  const bool eq = (s < ns - 1);  // this lane's segment ends in a separator
-  // separator s couples row SEG-2 of this segment and row 0 of segment s+1
-  const int nb = (s + 1 < SEGS) ? lane + MODES : lane;
-  const double VLn = __shfl(S.VL, nb, 64), VRn = __shfl(S.VR, nb, 64);
-  double A = eq ? S.aT * S.gp[SEG - 2] : 0.0;
-  double B = eq ? S.aT * (-S.cp[SEG - 2]) + S.bT + S.cT * VLn : 1.0;
-  double C = eq ? S.cT * VRn : 0.0;
-  double2 G[NC];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const double2 Yn = shfl2(S.Y[c], nb);
-    const double2 g = csub(csub(S.fT[c], rmul(S.aT, X[c][SEG - 2])), rmul(S.cT, Yn));
-    G[c] = eq ? g : cz();
-  }
-  // parallel cyclic reduction; rows outside 0..ns-2 are identity rows
-#pragma unroll
-  for (int d = 1; d < SEGS - 1; d *= 2) {
-    if (d >= ns - 1) continue;
-    const bool hasl = (s >= d), hash = (s + d < SEGS);
-    const int lo = hasl ? lane - d * MODES : lane, hi = hash ? lane + d * MODES : lane;
-    double Al = __shfl(A, lo, 64), Bl = __shfl(B, lo, 64), Cl = __shfl(C, lo, 64);
-    double Ah = __shfl(A, hi, 64), Bh = __shfl(B, hi, 64), Ch = __shfl(C, hi, 64);
-    double2 Gl[NC], Gh[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) { Gl[c] = shfl2(G[c], lo); Gh[c] = shfl2(G[c], hi); }
-    if (!hasl) { Al = 0.0; Bl = 1.0; Cl = 0.0; }
-    if (!hash) { Ah = 0.0; Bh = 1.0; Ch = 0.0; }
-    const double k1 = hasl ? A / Bl : 0.0;
-    const double k2 = hash ? C / Bh : 0.0;
-    const double An = -(Al * k1), Cn = -(Ch * k2);
-    const double Bn = B - Cl * k1 - Ah * k2;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const double2 gl = hasl ? Gl[c] : cz(), gh = hash ? Gh[c] : cz();
-      G[c] = csub(csub(G[c], rmul(k1, gl)), rmul(k2, gh));
-    }
-    A = An; B = Bn; C = Cn;
-  }
-  const double rB = 1.0 / B;
-  const int pv = (s > 0) ? lane - MODES : lane;
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const double2 x = eq ? rmul(rB, G[c]) : cz();
-    const double2 xp = shfl2(x, pv);
-    xr[c] = x;
-    xl[c] = (s > 0 && s < ns) ? xp : cz();
-  }
-}
-
 template <int SEG, int NC>
 __device__ __forceinline__ void seg_backsub(double2 (&X)[NC][SEG], const SegSys<SEG, NC>& S, const double2 (&xl)[NC],
                                             const double2 (&xr)[NC]) {
@@ -588,326 +556,482 @@ __device__ __forceinline__ void seg_backsub(double2 (&X)[NC][SEG], const SegSys<
   }
 }
 
-// bx: the wavefront's mode group; gx: the number of groups of the launch
-// (0: no XCD pairing, the batched form)
-template <int MODES, int SEG>
-__device__ __forceinline__ void solve_seg_body(const DevOps& ops, const SolveArgs& a, long bx, long gx) {
-  constexpr int SEGS = 64 / MODES;
-  // NL and P rows of this lane's segment, kept from the right-hand-side pass
-  // for the pressure update and the next RK register: [row][comp][lane]
-  __shared__ double2 stash[SEG][4][64];
-  const int lane = threadIdx.x;
-  const int s = lane / MODES, q = lane - (lane / MODES) * MODES;
+#define SOLVE_WG_MODES 8
+#define SOLVE_WG_SLOTS 6
+
+// The equation of a separator: A x(s-1) + B x(s) + C x(s+1) = G, with 1/B.
+// The rows are not normalised to B = 1: rounding A and C against it once more
+// at every step costs the low wavenumbers of the Poisson system half a digit.
+template <int NC>
+struct SepRow {
+  double A, B, C, rB;
+  double2 G[NC];
+};
+
+// this segment's separator row from the relation of the next segment's row 0
+// (Vn = its VL, VR; Yn) and this segment's own elimination
+template <int SEG, int NC>
+__device__ __forceinline__ void sep_row(const double2 (&X)[NC][SEG], const SegSys<SEG, NC>& S, bool eq, double2 Vn,
+                                        const double2 (&Yn)[NC], SepRow<NC>& e) {
+  e.A = eq ? S.aT * S.gp[SEG - 2] : 0.0;
+  e.B = eq ? S.aT * (-S.cp[SEG - 2]) + S.bT + S.cT * Vn.x : 1.0;
+  e.C = eq ? S.cT * Vn.y : 0.0;
+  e.rB = pivot_rcp(e.B);
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const double2 g = csub(csub(S.fT[c], rmul(S.aT, X[c][SEG - 2])), rmul(S.cT, Yn[c]));
+    e.G[c] = eq ? g : cz();
+  }
+}
+
+// one reduction step: substitute the rows at distance d on either side
+// (acl, rbl, Gl and ach, rbh, Gh: their A and C, 1/B and G)
+template <int NC>
+__device__ __forceinline__ void sep_reduce(SepRow<NC>& e, double2 acl, double rbl, const double2 (&Gl)[NC], double2 ach,
+                                           double rbh, const double2 (&Gh)[NC]) {
+  const double k1 = e.A * rbl, k2 = e.C * rbh;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) e.G[c] = csub(csub(e.G[c], rmul(k1, Gl[c])), rmul(k2, Gh[c]));
+  e.B = e.B - acl.y * k1 - ach.x * k2;
+  e.A = -(acl.x * k1);
+  e.C = -(ach.y * k2);
+  e.rB = pivot_rcp(e.B);
+}
+
+template <int SEG>
+__device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs& a, long bx) {
+  extern __shared__ double2 sh[];
+  const int tid = threadIdx.x;
+  const int s = tid / SOLVE_WG_MODES, q = tid % SOLVE_WG_MODES;
   const long nm = (long)a.nxh * a.nz;
   const int ny = a.ny, nyp = ny + 1;
-  const int ns = (nyp + SEG - 1) / SEG;   // active segments
-  const int rl = nyp - (ns - 1) * SEG;    // rows of the last one (3..SEG)
-  // The G = 8 / MODES mode groups whose rows share 128-byte lines (MODES < 8)
-  // go to workgroups b, b+8, .., b+8(G-1), which land on the same XCD one
-  // after the other.
-  long grp = bx;
-  if (MODES < 8 && gx > 0) {
-    constexpr long G = 8 / MODES;
-    const long full = (gx / (8 * G)) * (8 * G);
-    if (grp < full) {
-      const long xcd = grp & 7, k = grp >> 3;
-      grp = 8 * G * (k / G) + G * xcd + (k % G);
-    }
-  }
-  const long mg = grp * MODES + q;
-  const bool valid = (mg < nm) && (s < ns);
+  const int ns = (nyp + SEG - 1) / SEG;   // segments
+  // The ns*SEG - (ny+1) rows too many pad the end of the last segment down to
+  // 3 rows (the one-sided wall stencils stay in one segment), the rest the
+  // start of the first one, whose row 0 is its row f.
+  const int pad = ns * SEG - nyp, f = max(0, pad - (SEG - 3));
+  const int rl = SEG - (pad - f);         // rows of the last segment
+  const int na = ns * SOLVE_WG_MODES;     // threads with rows
+  const bool act = tid < na;
+  double2* const E = sh;                             // exchange slots [6][na]
+  double2* const NLS = sh + SOLVE_WG_SLOTS * na;     // this substep's NL rows [SEG][3][na]
+  double2* const WL = NLS + 3 * SEG * na;            // wall values [u, v, w][bottom, top][8]
+  double2* const KL = WL + 6 * SOLVE_WG_MODES;       // kx, kz [8]
+  double2* const OP = KL + SOLVE_WG_MODES;           // the operators d2h .. dn as they are packed in memory
+  const double* const d2h = reinterpret_cast<const double*>(OP);
+  const double* const d2n = d2h + (ops.d2n - ops.d2h);
+  const double* const dh = d2h + (ops.dh - ops.d2h);
+  const double* const dn = d2h + (ops.dn - ops.d2h);
+  const long mg = bx * SOLVE_WG_MODES + q;
+  const bool valid = act && mg < nm;
   const long m = (mg < nm) ? mg : nm - 1;
   const int ix = (int)(m / a.nz), iz = (int)(m - (long)ix * a.nz);
-  const int j0 = s * SEG;
-  const bool last = (s == ns - 1);
-  const double kxv = ops.kx[ix], kzv = ops.kz[iz];
-  const double k2 = kxv * kxv + kzv * kzv;
-  const bool mean = (k2 == 0.0);
-  const int r = a.rk - 1;
-  const double dt = a.sc->dt;
-  const double re = a.re;
-  const double* d2h = ops.d2h;
-  const double* d2n = ops.d2n;
-  const double* dn = ops.dn;
-  const double* dh = ops.dh;
-  const double* dm = ops.dm;
+  int j0 = s * SEG - f;
+  const bool first = (s == 0), last = (s == ns - 1);
   const double2* __restrict__ NL = a.nl;
   double2* __restrict__ R = a.R;
   double2* __restrict__ P = a.P;
   double2* __restrict__ U = a.vel;
-  auto neg = [](double2 v) { return make_double2(-v.x, -v.y); };
-  auto sel = [](bool c, double2 x, double2 y) { return make_double2(c ? x.x : y.x, c ? x.y : y.y); };
-
   const uint32_t rowB = (uint32_t)(nm * 16), cmpB = rowB * (uint32_t)nyp;
   const uint32_t om0 = (uint32_t)(m * 16);
+  auto rowc = [&](int j) { return min(max(j, 0), ny); };   // padding rows read the wall rows
   auto OM = [&](int j) { return om0 + (uint32_t)j * rowB; };
   auto OC = [&](int c, int j) { return (uint32_t)c * cmpB + om0 + (uint32_t)j * rowB; };
+  auto sel = [](bool c, double2 x, double2 y) { return make_double2(c ? x.x : y.x, c ? x.y : y.y); };
+  auto put = [&](int k, double2 v) { if (act) E[k * na + tid] = v; };
+  const int ti = act ? tid : 0;
+  const int tn = (act && s + 1 < ns) ? tid + SOLVE_WG_MODES : ti;   // the next segment's thread (or this one)
+  const int tp = (act && s > 0) ? tid - SOLVE_WG_MODES : ti;        // the previous segment's
+  auto get = [&](int k, int t) { return E[k * na + t]; };
 
+  // ---------------- every load of the kernel, none waited for before the last is issued ----------------
+  const int wb = __builtin_amdgcn_readfirstlane(tid & ~63);   // the wavefront's first thread
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  {
+    const int nop = (int)(ops.dn - ops.d2h + ny + 1) / 2;     // 16-byte cells (solve_wg_lds)
+    const double2* src = reinterpret_cast<const double2*>(ops.d2h);
+    for (int i = 0; i < nop; i += blockDim.x)
+      if (i + tid < nop) __builtin_amdgcn_global_load_lds((const void*)(src + i + tid), (lds_ptr)(OP + i + wb), 16, 0, 0);
+  }
+  double kxv = ops.kx[ix], kzv = ops.kz[iz];
+  double2 UW[2][SEG], V[1][SEG], PR[SEG];
+#pragma unroll
+  for (int t = 0; t < SEG; ++t) {
+    const int jc = rowc(j0 + t);
+    UW[0][t] = ldo(R, OC(0, jc));
+    V[0][t] = ldo(R, OC(1, jc));
+    UW[1][t] = ldo(R, OC(2, jc));
+    PR[t] = ldo(P, OM(jc));
+  }
+#pragma unroll
+  for (int t = 0; t < SEG; ++t)
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      if (act)
+        __builtin_amdgcn_global_load_lds((const void*)(reinterpret_cast<const char*>(NL) + OC(c, rowc(j0 + t))),
+                                         (lds_ptr)(NLS + (t * 3 + c) * na + wb), 16, 0, 0);
+  auto nls = [&](int c, int t) { return NLS[(t * 3 + c) * na + ti]; };
+  if (first || last) {   // the segments with the wall rows fetch the wall data (cbc: top, then bottom)
+    const double2* w = a.cbc + (first ? 3L : 0L) * nm + m;
+    double2* wl = WL + (first ? 0 : SOLVE_WG_MODES) + q;
+    const double2 w0 = w[0], w1 = w[nm], w2 = w[2 * nm];
+    wl[0] = w0; wl[2 * SOLVE_WG_MODES] = w1; wl[4 * SOLVE_WG_MODES] = w2;
+  }
+  if (first) KL[q] = make_double2(kxv, kzv);
+  auto wall = [&](int c, int top) { return WL[(2 * c + top) * SOLVE_WG_MODES + q]; };
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wavefront's DMA rows are in LDS
+  __syncthreads();                      // and the other wavefronts' operators
+
+  double k2 = kxv * kxv + kzv * kzv;
+  const bool mean = (k2 == 0.0);        // mode 0 only, so only in workgroup 0
+  const int r = a.rk - 1;
+  const double dt = a.sc->dt;
+  const double re = a.re;
+  const double* dm = ops.dm;
   const double vis_imp = c_rkd[r] * (dt / re);
   const double rk_press = (c_rkc[r] + c_rkd[r]) * dt;
   const double coef = c_rkb[r] * dt;
-  const double vis_exp1 = c_rkc[r] * (dt / re);
-  const double alpha = 1.0 + vis_imp * k2;
-
-  // mean-mode pressure gradient (compute_p_grad, :369-373); the mean mode is mode 0
-  double p_grad = a.sc->p_grad;
-  if (grp == 0 && a.fix_mass == 1) {
-    double part = 0.0;
+  double alpha = 1.0 + vis_imp * k2;
+  double2 msh0 = cz(), msh2 = cz();     // mean pressure gradient (:220-221)
+  if (bx == 0) {
+    // mean-mode pressure gradient (compute_p_grad, :369-373)
+    double p_grad = a.sc->p_grad;
+    if (a.fix_mass == 1) {
+      double part = 0.0;
 #pragma unroll
-    for (int t = 0; t < SEG; ++t) {
-      const int j = j0 + t;
-      const int jc = min(j, ny);
-      const double term = ops.dyh[jc] * (-ldo(NL, OC(0, jc)).x);
-      part = (j >= 1 && j <= ny - 1) ? part + term : part;
+      for (int t = 0; t < SEG; ++t) {
+        const int j = j0 + t;
+        const double term = ops.dyh[rowc(j)] * (-nls(0, t).x);
+        part = (j >= 1 && j <= ny - 1) ? part + term : part;
+      }
+      put(0, make_double2(part, 0.0));
+      __syncthreads();
+      double tmp = 0.0;
+      for (int k = 0; k < ns; ++k) tmp += E[k * SOLVE_WG_MODES + q].x;
+      __syncthreads();
+      if (mean) {
+        p_grad = -tmp + 0.5 * (a.dudy[ny - 1] - a.dudy[0]) / re;
+        if (tid == 0) a.sc->p_grad = p_grad;
+      }
     }
-    double tmp = 0.0;
-#pragma unroll
-    for (int k = 0; k < SEGS; ++k) tmp = (k < ns) ? tmp + __shfl(part, k * MODES + q, 64) : tmp;
     if (mean) {
-      p_grad = -tmp + 0.5 * (a.dudy[ny - 1] - a.dudy[0]) / re;
-      if (lane == 0) a.sc->p_grad = p_grad;
+      msh0.x = a.cosb * rk_press * p_grad;
+      msh2.x = a.sinb * rk_press * p_grad;
+      // the mean mode has no pressure: whatever the state holds is not used
+#pragma unroll
+      for (int t = 0; t < SEG; ++t) PR[t] = cz();
     }
   }
-  const double2 msh0 = make_double2(a.cosb * rk_press * p_grad, 0.0);
-  const double2 msh2 = make_double2(a.sinb * rk_press * p_grad, 0.0);
-
-  const double2 top0 = a.cbc[(0L * 3 + 0) * nm + m], top1 = a.cbc[(0L * 3 + 1) * nm + m],
-                top2 = a.cbc[(0L * 3 + 2) * nm + m];
-  const double2 bot0 = a.cbc[(1L * 3 + 0) * nm + m], bot1 = a.cbc[(1L * 3 + 1) * nm + m],
-                bot2 = a.cbc[(1L * 3 + 2) * nm + m];
 
   // ---------------- right-hand sides (rows j0 .. j0+SEG-1) ----------------
-  double2 UW[2][SEG], V[1][SEG];
   auto rhs = [&](auto first_c) {
     constexpr bool FIRST = decltype(first_c)::value;
-    const int jb = min(j0, ny);  // rows clamped for idle lanes
-    double2 Rm0 = cz(), Rm1 = cz(), Rm2 = cz();
-    double2 Pc = ldo(P, OM(jb));
-    double2 Rc0 = ldo(R, OC(0, jb)), Rc1 = ldo(R, OC(1, jb)), Rc2 = ldo(R, OC(2, jb));
-    // The first substep's stencils reach one row into each neighbouring
-    // segment: R at j0-1 (the explicit diffusion of row j0) and R, P at
-    // j0+SEG (those of the last row).  Every lane reads only its own rows from
-    // memory, the rows it overwrites later in this kernel; the neighbours'
-    // rows come from the lanes that own them, through register shuffles.
-    // Wall rows take the wall values, so what the segments at the ends
-    // receive from beyond the walls (their own rows) is never used.
-    double2 Rx0 = cz(), Rx1 = cz(), Rx2 = cz(), Px = cz();
+    double2 Rm0 = cz(), Rm1 = cz(), Rm2 = cz(), Rx0 = cz(), Rx1 = cz(), Rx2 = cz(), Px = cz();
+    const double vis_exp1 = c_rkc[0] * (dt / re);
     if (FIRST) {
-      const int jl = min(j0 + SEG - 1, ny);
-      const double2 L0 = ldo(R, OC(0, jl)), L1 = ldo(R, OC(1, jl)), L2 = ldo(R, OC(2, jl));
-      const int prv = (s == 0) ? lane : lane - MODES;
-      const int nxt = (s + 1 >= SEGS) ? lane : lane + MODES;
-      Rm0 = sel(s == 0, Rc0, shfl2(L0, prv));
-      Rm1 = sel(s == 0, Rc1, shfl2(L1, prv));
-      Rm2 = sel(s == 0, Rc2, shfl2(L2, prv));
-      Rx0 = shfl2(Rc0, nxt);
-      Rx1 = shfl2(Rc1, nxt);
-      Rx2 = shfl2(Rc2, nxt);
-      Px = shfl2(Pc, nxt);
+      // the neighbouring segments' rows at j0-1 and j0+SEG; what the segments
+      // at the walls receive (their own rows) is never used
+      put(0, UW[0][0]); put(1, V[0][0]); put(2, UW[1][0]); put(3, PR[0]); put(4, UW[0][SEG - 1]);
+      __syncthreads();
+      Rx0 = get(0, tn); Rx1 = get(1, tn); Rx2 = get(2, tn); Px = get(3, tn); Rm0 = get(4, tp);
+      __syncthreads();
+      put(0, V[0][SEG - 1]); put(1, UW[1][SEG - 1]);
+      __syncthreads();
+      Rm1 = get(0, tp); Rm2 = get(1, tp);
     }
 #pragma unroll
     for (int t = 0; t < SEG; ++t) {
       const int j = j0 + t;
-      const int jc = min(j, ny), jn = min(j + 1, ny), jv = min(j, ny - 1);
-      const double2 n0 = ldo(NL, OC(0, jc)), n1 = ldo(NL, OC(1, jc)), n2 = ldo(NL, OC(2, jc));
-      stash[t][0][lane] = n0;
-      stash[t][1][lane] = n1;
-      stash[t][2][lane] = n2;
-      stash[t][3][lane] = Pc;
-      double2 r0 = cz(), r1 = cz(), r2 = cz(), pn = cz();
-      if (t + 1 < SEG) {
-        r0 = ldo(R, OC(0, jn)); r1 = ldo(R, OC(1, jn)); r2 = ldo(R, OC(2, jn));
-        pn = ldo(P, OM(jn));
-      } else if (FIRST) {
-        r0 = Rx0; r1 = Rx1; r2 = Rx2;
-        pn = Px;
-      }
-      double2 v0 = cadd(Rc0, rmul(coef, neg(n0)));
-      double2 v1 = cadd(Rc1, rmul(coef, neg(n1)));
-      double2 v2 = cadd(Rc2, rmul(coef, neg(n2)));
+      const double2 Rc0 = UW[0][t], Rc1 = V[0][t], Rc2 = UW[1][t], Pc = PR[t];
+      double2 v0 = csub(Rc0, rmul(coef, nls(0, t)));
+      double2 v1 = csub(Rc1, rmul(coef, nls(1, t)));
+      double2 v2 = csub(Rc2, rmul(coef, nls(2, t)));
       if (FIRST) {
+        const int jc = rowc(j), jv = min(jc, ny - 1);
+        const int tq = t + 1 < SEG ? t + 1 : t;
+        const double2 r0 = t + 1 < SEG ? UW[0][tq] : Rx0, r1 = t + 1 < SEG ? V[0][tq] : Rx1,
+                      r2 = t + 1 < SEG ? UW[1][tq] : Rx2, pn = t + 1 < SEG ? PR[tq] : Px;
         // add_explicit_diffusive_terms(cv, cru) (:339-351)
         const double a0 = d2h[3 * jc], a1 = d2h[3 * jc + 1], a2 = d2h[3 * jc + 2];
         const double b0 = d2n[3 * jv], b1 = d2n[3 * jv + 1], b2 = d2n[3 * jv + 2];
-        const double dnj = dn[jv];
         const double2 du = cadd(cadd(rmul(a0, Rm0), rmul(a1, Rc0)), rmul(a2, r0));
-        v0 = cadd(v0, rmul(vis_exp1, csub(du, rmul(k2, Rc0))));
         const double2 dw = cadd(cadd(rmul(a0, Rm2), rmul(a1, Rc2)), rmul(a2, r2));
-        v2 = cadd(v2, rmul(vis_exp1, csub(dw, rmul(k2, Rc2))));
         const double2 dv = cadd(cadd(rmul(b0, Rm1), rmul(b1, Rc1)), rmul(b2, r1));
-        v1 = sel(j <= ny - 2, cadd(v1, rmul(vis_exp1, csub(dv, rmul(k2, Rc1)))), v1);
+        v0 = cadd(v0, rmul(vis_exp1, csub(du, rmul(k2, Rc0))));
+        v2 = cadd(v2, rmul(vis_exp1, csub(dw, rmul(k2, Rc2))));
+        v1 = cadd(v1, rmul(vis_exp1, csub(dv, rmul(k2, Rc1))));
         // subtract_pressure_gradient(cv, cp, rk_press) (:54-77)
-        v0 = sel(mean, v0, csub(v0, imul(rk_press * kxv, Pc)));
-        v2 = sel(mean, v2, csub(v2, imul(rk_press * kzv, Pc)));
-        v1 = sel(!mean && j <= ny - 2, csub(v1, rmul(rk_press * dnj, csub(pn, Pc))), v1);
+        v0 = csub(v0, imul(rk_press * kxv, Pc));
+        v2 = csub(v2, imul(rk_press * kzv, Pc));
+        v1 = csub(v1, rmul(rk_press * dn[jv], csub(pn, Pc)));
+        Rm0 = Rc0; Rm1 = Rc1; Rm2 = Rc2;
       }
-      // mean pressure gradient (:220-221)
-      v0 = sel(mean, csub(v0, msh0), v0);
-      v2 = sel(mean, csub(v2, msh2), v2);
-      // wall rows carry the wall values (SOLVE_HELMHOLTZ, :174-213); v has no row ny
-      v0 = sel(j == 0, bot0, sel(j == ny, top0, sel(j > ny, cz(), v0)));
-      v2 = sel(j == 0, bot2, sel(j == ny, top2, sel(j > ny, cz(), v2)));
-      v1 = sel(j == 0, bot1, sel(j == ny - 1, top1, sel(j >= ny, cz(), v1)));
       UW[0][t] = v0;
       UW[1][t] = v2;
       V[0][t] = v1;
-      Rm0 = Rc0; Rm1 = Rc1; Rm2 = Rc2;
-      Rc0 = r0; Rc1 = r1; Rc2 = r2;
-      Pc = pn;
     }
   };
   if (r == 0) rhs(std::true_type{});
   else rhs(std::false_type{});
+  // Special rows and modes are patched behind branches that the other
+  // wavefronts skip (the last segment's row count rl is uniform).
+  if (bx == 0 && mean) {
+#pragma unroll
+    for (int t = 0; t < SEG; ++t) {
+      UW[0][t] = csub(UW[0][t], msh0);
+      UW[1][t] = csub(UW[1][t], msh2);
+    }
+  }
+  // wall rows carry the wall values (SOLVE_HELMHOLTZ, :174-213); v has no row
+  // ny; rows past the last are zero
+  auto walls = [&](int vtop) {
+    if (first) {
+      const double2 W0 = wall(0, 0), W1 = wall(1, 0), W2 = wall(2, 0);
+#pragma unroll
+      for (int t = 0; t < SEG - 2; ++t) {
+        if (t == f) { UW[0][t] = W0; UW[1][t] = W2; V[0][t] = W1; }
+        if (t < f) UW[0][t] = UW[1][t] = V[0][t] = cz();
+      }
+    }
+    if (last) {
+      const double2 W0 = wall(0, 1), v1top = wall(1, vtop), W2 = wall(2, 1);
+#pragma unroll
+      for (int t = 1; t < SEG; ++t) {
+        if (t == rl - 1) { UW[0][t] = W0; UW[1][t] = W2; }
+        if (t >= rl) UW[0][t] = UW[1][t] = cz();
+        if (t == rl - 2) V[0][t] = v1top;
+        if (t >= rl - 1) V[0][t] = cz();
+      }
+    }
+  };
+  walls(1);
+  __syncthreads();   // the exchange slots
 
+  const bool eq = s < ns - 1;
   // ---------------- Helmholtz solves (u and w with D2H, v with D2N) ----------------
   {
     SegSys<SEG, 2> SH;
     SegSys<SEG, 1> SN;
     seg_eliminate(UW, SH, [&](int t, double& a_, double& b_, double& c_) {
-      const int j = j0 + t, jc = min(j, ny);
-      const double h0 = d2h[3 * jc], h1 = d2h[3 * jc + 1], h2 = d2h[3 * jc + 2];
-      const bool wall = (j == 0 || j >= ny);
-      a_ = wall ? 0.0 : -vis_imp * h0;
-      b_ = wall ? 1.0 : -vis_imp * h1 + alpha;
-      c_ = wall ? 0.0 : -vis_imp * h2;
-    }, s >= ns - 1);
+      const int j = j0 + t, jc = rowc(j);
+      const bool wall = (j <= 0 || j >= ny);
+      const double w = wall ? 0.0 : vis_imp;
+      a_ = -w * d2h[3 * jc];
+      b_ = -w * d2h[3 * jc + 1] + (wall ? 1.0 : alpha);
+      c_ = -w * d2h[3 * jc + 2];
+    }, !eq);
     seg_eliminate(V, SN, [&](int t, double& a_, double& b_, double& c_) {
-      const int j = j0 + t, jv = min(j, ny - 1);
-      const double h0 = d2n[3 * jv], h1 = d2n[3 * jv + 1], h2 = d2n[3 * jv + 2];
-      const bool wall = (j == 0 || j >= ny - 1);
-      a_ = wall ? 0.0 : -vis_imp * h0;
-      b_ = wall ? 1.0 : -vis_imp * h1 + alpha;
-      c_ = wall ? 0.0 : -vis_imp * h2;
-    }, s >= ns - 1);
-    double2 xlH[2], xrH[2], xlN[1], xrN[1];
-    seg_separators<MODES, SEG, 2>(UW, SH, lane, ns, xlH, xrH);
-    seg_separators<MODES, SEG, 1>(V, SN, lane, ns, xlN, xrN);
-    seg_backsub(UW, SH, xlH, xrH);
-    seg_backsub(V, SN, xlN, xrN);
-  }
+      const int j = j0 + t, jv = min(rowc(j), ny - 1);
+      const bool wall = (j <= 0 || j >= ny - 1);
+      const double w = wall ? 0.0 : vis_imp;
+      a_ = -w * d2n[3 * jv];
+      b_ = -w * d2n[3 * jv + 1] + (wall ? 1.0 : alpha);
+      c_ = -w * d2n[3 * jv + 2];
+    }, !eq);
+    put(0, make_double2(SH.VL, SH.VR)); put(1, SH.Y[0]); put(2, SH.Y[1]);
+    put(3, make_double2(SN.VL, SN.VR)); put(4, SN.Y[0]);
+    __syncthreads();
+    SepRow<2> eh;
+    SepRow<1> en;
+    {
+      const double2 Yh[2] = {get(1, tn), get(2, tn)}, Yn[1] = {get(4, tn)};
+      sep_row(UW, SH, eq, get(0, tn), Yh, eh);
+      sep_row(V, SN, eq, get(3, tn), Yn, en);
+    }
+    for (int d = 1; d < ns - 1; d *= 2) {
+      __syncthreads();
+      put(0, make_double2(eh.A, eh.C)); put(1, eh.G[0]); put(2, eh.G[1]);
+      put(3, make_double2(en.A, en.C)); put(4, en.G[0]); put(5, make_double2(eh.rB, en.rB));
+      __syncthreads();
+      // rows past either end: the first separator's A and the last one's C
+      // are zero, and stay so, so any row stands in for them
+      const int lo = (act && s >= d) ? tid - d * SOLVE_WG_MODES : ti, hi = (act && s + d < ns) ? tid + d * SOLVE_WG_MODES : ti;
+      const double2 rl_ = get(5, lo), rh_ = get(5, hi);
+      const double2 Ghl[2] = {get(1, lo), get(2, lo)}, Ghh[2] = {get(1, hi), get(2, hi)};
+      sep_reduce(eh, get(0, lo), rl_.x, Ghl, get(0, hi), rh_.x, Ghh);
+      const double2 Gnl[1] = {get(4, lo)}, Gnh[1] = {get(4, hi)};
+      sep_reduce(en, get(3, lo), rl_.y, Gnl, get(3, hi), rh_.y, Gnh);
+    }
 #pragma unroll
-  for (int t = 0; t < SEG; ++t)  // mean mode (:261-263)
-    V[0][t] = sel(mean, (j0 + t < ny) ? bot1 : cz(), V[0][t]);
+    for (int c = 0; c < 2; ++c) eh.G[c] = rmul(eh.rB, eh.G[c]);
+    en.G[0] = rmul(en.rB, en.G[0]);
+    __syncthreads();
+    put(0, eh.G[0]); put(1, eh.G[1]); put(2, en.G[0]);
+    __syncthreads();
+    // the first row of segment 0 has no separator below it (gp = 0)
+    const double2 xl[2] = {get(0, tp), get(1, tp)};
+    const double2 xn[1] = {get(2, tp)};
+    seg_backsub(UW, SH, xl, eh.G);
+    seg_backsub(V, SN, xn, en.G);
+  }
+  if (bx == 0 && mean) {  // mean mode (:261-263)
+#pragma unroll
+    for (int t = 0; t < SEG; ++t) V[0][t] = (j0 + t < ny) ? wall(1, 0) : cz();
+  }
 
   // ---------------- Neumann Poisson for the pressure correction ----------------
   double2 PH[1][SEG];
+  put(3, V[0][SEG - 1]);
+  __syncthreads();
   {
-    const int pv = (s == 0) ? lane : lane - MODES;
-    const double2 vprev = shfl2(V[0][SEG - 1], pv);
+    const double2 vprev = get(3, tp);
     const double tmpc = 1.0 / rk_press;
 #pragma unroll
     for (int t = 0; t < SEG; ++t) {
-      const int j = j0 + t, jc = min(j, ny);
-      const double2 vm = (t == 0) ? vprev : V[0][t - 1];
+      const int j = j0 + t, jc = rowc(j);
+      const double2 vm = (t == 0) ? vprev : V[0][t > 0 ? t - 1 : 0];
       // strip_divergence rhs (:28-31)
-      const double2 dv = cadd(cadd(imul(kxv, UW[0][t]), rmul(dh[jc], csub(V[0][t], vm))), imul(kzv, UW[1][t]));
-      PH[0][t] = sel(j >= 1 && j <= ny - 1 && !mean, rmul(tmpc, dv), cz());
+      PH[0][t] = rmul(tmpc, cadd(cadd(imul(kxv, UW[0][t]), rmul(dh[jc], csub(V[0][t], vm))), imul(kzv, UW[1][t])));
+    }
+    if (first) {
+#pragma unroll
+      for (int t = 0; t < SEG - 2; ++t)
+        if (t <= f) PH[0][t] = cz();
+    }
+    if (last) {
+#pragma unroll
+      for (int t = 2; t < SEG; ++t)
+        if (t >= rl - 1) PH[0][t] = cz();
+    }
+    if (bx == 0 && mean) {
+#pragma unroll
+      for (int t = 0; t < SEG; ++t) PH[0][t] = cz();
     }
   }
   const double alp = mean ? -1.0 : -k2;  // the mean mode has no pressure correction
   {
-    const double dn0 = dn[0], dn1 = dn[1], dh1 = dh[1];
-    const double dnt = dn[ny - 1], dnt2 = dn[ny - 2], dht = dh[ny - 1];
     SegSys<SEG, 1> SP;
     seg_eliminate(PH, SP, [&](int t, double& a_, double& b_, double& c_) {
-      const int j = j0 + t, jc = min(j, ny);
-      const double h0 = d2h[3 * jc], h1 = d2h[3 * jc + 1], h2 = d2h[3 * jc + 2];
-      a_ = h0; b_ = h1 + alp; c_ = h2;
-      a_ = (j == 1) ? dh1 * dn0 : a_;
-      b_ = (j == 1) ? -dh1 * dn0 - dh1 * dn1 + alp : b_;
-      c_ = (j == 1) ? dh1 * dn1 : c_;
-      a_ = (j == ny - 1) ? dht * dnt2 : a_;
-      b_ = (j == ny - 1) ? -dht * dnt2 - dht * dnt + alp : b_;
-      c_ = (j == ny - 1) ? dht * dnt : c_;
-      a_ = (j == 0) ? 0.0 : (j == ny) ? -dnt : (j > ny) ? 0.0 : a_;
-      b_ = (j == 0) ? -dn0 : (j == ny) ? dnt : (j > ny) ? 1.0 : b_;
-      c_ = (j == 0) ? dn0 : (j >= ny) ? 0.0 : c_;
-    }, s >= ns - 1);
-    double2 xl[1], xr[1];
-    seg_separators<MODES, SEG, 1>(PH, SP, lane, ns, xl, xr);
-    seg_backsub(PH, SP, xl, xr);
+      const int jc = rowc(j0 + t);
+      a_ = d2h[3 * jc]; b_ = d2h[3 * jc + 1] + alp; c_ = d2h[3 * jc + 2];
+      // the Neumann rows 0, 1 and ny-1, ny, and identity rows beyond them
+      if (t < SEG - 3 && t < f && first) { a_ = 0.0; b_ = 1.0; c_ = 0.0; }
+      if (t < SEG - 2 && t == f && first) { a_ = 0.0; b_ = -dn[0]; c_ = dn[0]; }
+      if (t >= 1 && t < SEG - 1 && t == f + 1 && first) { a_ = dh[1] * dn[0]; b_ = -dh[1] * dn[0] - dh[1] * dn[1] + alp; c_ = dh[1] * dn[1]; }
+      if (t >= 1 && t == rl - 2 && last) {
+        const double dht = dh[ny - 1], dnt = dn[ny - 1], dnt2 = dn[ny - 2];
+        a_ = dht * dnt2; b_ = -dht * dnt2 - dht * dnt + alp; c_ = dht * dnt;
+      }
+      if (t >= 2 && t == rl - 1 && last) { a_ = -dn[ny - 1]; b_ = dn[ny - 1]; c_ = 0.0; }
+      if (t >= 3 && t >= rl && last) { a_ = 0.0; b_ = 1.0; c_ = 0.0; }
+    }, !eq);
+    put(0, make_double2(SP.VL, SP.VR)); put(1, SP.Y[0]);
+    __syncthreads();
+    SepRow<1> ep;
+    {
+      const double2 Yp[1] = {get(1, tn)};
+      sep_row(PH, SP, eq, get(0, tn), Yp, ep);
+    }
+    for (int d = 1; d < ns - 1; d *= 2) {
+      __syncthreads();
+      put(0, make_double2(ep.A, ep.C)); put(1, ep.G[0]); put(2, make_double2(ep.rB, 0.0));
+      __syncthreads();
+      const int lo = (act && s >= d) ? tid - d * SOLVE_WG_MODES : ti, hi = (act && s + d < ns) ? tid + d * SOLVE_WG_MODES : ti;
+      const double2 Gl[1] = {get(1, lo)}, Gh[1] = {get(1, hi)};
+      sep_reduce(ep, get(0, lo), get(2, lo).x, Gl, get(0, hi), get(2, hi).x, Gh);
+    }
+    ep.G[0] = rmul(ep.rB, ep.G[0]);
+    put(3, ep.G[0]);
+    __syncthreads();
+    const double2 xl[1] = {get(3, tp)};
+    seg_backsub(PH, SP, xl, ep.G);
   }
   // wall re-extrapolation (SOLVE_P :335-336, zero wall data)
-  {
-    const double2 pb = make_double2((0.0 - dm[1] * PH[0][1].x - dm[2] * PH[0][2].x) / dm[0],
-                                    (0.0 - dm[1] * PH[0][1].y - dm[2] * PH[0][2].y) / dm[0]);
-    PH[0][0] = sel(s == 0, pb, PH[0][0]);
-    double2 q1 = cz(), q2 = cz();
+  if (first) {
+    const double d0 = 1.0 / dm[0];
 #pragma unroll
-    for (int t = 0; t < SEG; ++t) {
-      q1 = sel(t == rl - 3, PH[0][t], q1);
-      q2 = sel(t == rl - 2, PH[0][t], q2);
-    }
-    const double2 pt = make_double2((0.0 - dm[3] * q1.x - dm[4] * q2.x) / dm[5],
-                                    (0.0 - dm[3] * q1.y - dm[4] * q2.y) / dm[5]);
+    for (int t = 0; t < SEG - 2; ++t)
+      if (t == f)
+        PH[0][t] = make_double2((0.0 - dm[1] * PH[0][t + 1].x - dm[2] * PH[0][t + 2].x) * d0,
+                                (0.0 - dm[1] * PH[0][t + 1].y - dm[2] * PH[0][t + 2].y) * d0);
+  }
+  if (last) {
+    const double d5 = 1.0 / dm[5];
 #pragma unroll
-    for (int t = 0; t < SEG; ++t) PH[0][t] = sel(mean, cz(), sel(last && t == rl - 1, pt, PH[0][t]));
+    for (int t = 2; t < SEG; ++t)
+      if (t == rl - 1)
+        PH[0][t] = make_double2((0.0 - dm[3] * PH[0][t - 2].x - dm[4] * PH[0][t - 1].x) * d5,
+                                (0.0 - dm[3] * PH[0][t - 2].y - dm[4] * PH[0][t - 1].y) * d5);
+  }
+  if (bx == 0 && mean) {
+#pragma unroll
+    for (int t = 0; t < SEG; ++t) PH[0][t] = cz();
   }
 
+  // Row addresses and wavenumbers are formed anew in each of the last phases
+  // (the empty asm hides that they are the old ones): kept in registers over
+  // the whole kernel they are spilled, and a reload waits for the stores
+  // before it (158 -> 139 us at 192x129x192).
+  auto renew = [&]() {
+    asm volatile("" : "+v"(j0));
+    const double2 kk = KL[q];
+    kxv = kk.x; kzv = kk.y;
+    k2 = kxv * kxv + kzv * kzv;
+    alpha = 1.0 + vis_imp * k2;
+  };
   // ---------------- projection and pressure update ----------------
-  const int nxt = (last || s + 1 >= SEGS) ? lane : lane + MODES, prv = (s == 0) ? lane : lane - MODES;
-  const double alpha2 = 1.0 + vis_imp * k2;
-  double2 PN[SEG];
+  put(4, PH[0][0]); put(5, PH[0][SEG - 1]);
+  __syncthreads();
+  renew();
   {
-    const double2 phN = shfl2(PH[0][0], nxt);
-    const double2 phP = shfl2(PH[0][SEG - 1], prv);
+    const double alpha2 = alpha;   // 1 + vis_imp k^2
+    const double2 phN = get(4, tn), phP = get(5, tp);
 #pragma unroll
     for (int t = 0; t < SEG; ++t) {
-      const int j = j0 + t, jc = min(j, ny), jv = min(j, ny - 1);
+      const int j = j0 + t, jc = rowc(j), jv = min(jc, ny - 1);
       const double2 f0 = PH[0][t];
-      const double2 fn = (t + 1 < SEG) ? PH[0][t + 1] : phN;
-      double2 s0 = (t > 0) ? PH[0][t - 1] : phP, s1 = f0, s2 = fn;
-      if (t == 0) { s0 = sel(j == 0, PH[0][0], s0); s1 = sel(j == 0, PH[0][1], s1); s2 = sel(j == 0, PH[0][2], s2); }
-      if (t >= 2) { s0 = sel(j == ny, PH[0][t - 2], s0); s1 = sel(j == ny, PH[0][t - 1], s1); s2 = sel(j == ny, f0, s2); }
-      const double2 Pold = stash[t][3][lane];
-      const double h0 = d2h[3 * jc], h1 = d2h[3 * jc + 1], h2 = d2h[3 * jc + 2];
-      const double dnj = dn[jv];
-      const bool inner = !mean && j >= 1 && j <= ny - 1;
-      const double2 cu = sel(inner, csub(UW[0][t], imul(rk_press * kxv, f0)), UW[0][t]);
-      const double2 cw = sel(inner, csub(UW[1][t], imul(rk_press * kzv, f0)), UW[1][t]);
-      const double2 cv = sel(inner && j <= ny - 2, csub(V[0][t], rmul(rk_press * dnj, csub(fn, f0))), V[0][t]);
-      const double2 d2 = cadd(cadd(rmul(h0, s0), rmul(h1, s1)), rmul(h2, s2));
-      const double2 pn = sel(mean, cz(), csub(cadd(Pold, rmul(alpha2, f0)), rmul(vis_imp, d2)));
-      UW[0][t] = cu;
-      V[0][t] = cv;
-      UW[1][t] = cw;
-      PN[t] = pn;
+      const double2 fn = (t + 1 < SEG) ? PH[0][t + 1 < SEG ? t + 1 : t] : phN;
+      double2 s0 = (t > 0) ? PH[0][t > 0 ? t - 1 : 0] : phP, s1 = f0, s2 = fn;
+      // the one-sided rows: 0 and ny
+      if (t < SEG - 2 && t == f && first) { s0 = f0; s1 = PH[0][t + 1 < SEG ? t + 1 : t]; s2 = PH[0][t + 2 < SEG ? t + 2 : t]; }
+      if (t >= 2 && t == rl - 1 && last) { s0 = PH[0][t >= 2 ? t - 2 : 0]; s1 = PH[0][t >= 1 ? t - 1 : 0]; s2 = f0; }
+      UW[0][t] = csub(UW[0][t], imul(rk_press * kxv, f0));
+      UW[1][t] = csub(UW[1][t], imul(rk_press * kzv, f0));
+      V[0][t] = csub(V[0][t], rmul(rk_press * dn[jv], csub(fn, f0)));
+      const double2 d2 = cadd(cadd(rmul(d2h[3 * jc], s0), rmul(d2h[3 * jc + 1], s1)), rmul(d2h[3 * jc + 2], s2));
+      PR[t] = csub(cadd(PR[t], rmul(alpha2, f0)), rmul(vis_imp, d2));
     }
   }
-  if (valid) {
-#pragma unroll
-    for (int t = 0; t < SEG; ++t) {
-      const int j = j0 + t;
-      if (j <= ny) {
-        sto(U, OC(0, j), UW[0][t]);
-        sto(U, OC(1, j), V[0][t]);
-        sto(U, OC(2, j), UW[1][t]);
-        sto(P, OM(j), PN[t]);
-      }
-    }
-  }
+  walls(mean ? 0 : 1);   // the wall rows are not projected; the mean mode's v is its bottom value (:261-263)
 
   // ---------------- d_um_dy and the next RK register ----------------
-  const double2 uN = shfl2(UW[0][0], nxt), vN = shfl2(V[0][0], nxt), wN = shfl2(UW[1][0], nxt);
-  const double2 uP = shfl2(UW[0][SEG - 1], prv), vP = shfl2(V[0][SEG - 1], prv), wP = shfl2(UW[1][SEG - 1], prv);
-  const double2 pnN = shfl2(PN[0], nxt);
-  if (mean && valid) {  // d_um_dy update from the new mean profile (:84-89)
+  put(0, UW[0][0]); put(1, V[0][0]); put(2, UW[1][0]);
+  __syncthreads();
+  const double2 uN = get(0, tn), vN = get(1, tn), wN = get(2, tn);
+  __syncthreads();
+  put(0, UW[0][SEG - 1]); put(1, V[0][SEG - 1]); put(2, UW[1][SEG - 1]); put(3, PR[0]);
+  __syncthreads();
+  const double2 uP = get(0, tp), vP = get(1, tp), wP = get(2, tp), pnN = get(3, tn);
+  // no barrier from here on, so that no store is waited for
+  renew();
+  if (bx == 0 && mean && valid) {  // d_um_dy update from the new mean profile (:84-89)
 #pragma unroll
     for (int t = 0; t < SEG; ++t) {
       const int j = j0 + t;
-      const double un = (t + 1 < SEG) ? UW[0][t + 1].x : uN.x;
+      const double un = (t + 1 < SEG) ? UW[0][t + 1 < SEG ? t + 1 : t].x : uN.x;
       if (j >= 1 && j <= ny - 2) a.dudy[j] = (dn[j] * (un - UW[0][t].x));
-      if (t == 0 && j == 0) a.dudy[0] = dm[0] * UW[0][0].x + dm[1] * UW[0][1].x + dm[2] * UW[0][2].x;
+      if (t < SEG - 2 && j == 0)
+        a.dudy[0] = dm[0] * UW[0][t].x + dm[1] * UW[0][t + 1 < SEG ? t + 1 : t].x + dm[2] * UW[0][t + 2 < SEG ? t + 2 : t].x;
       if (t >= 2 && j == ny)
-        a.dudy[ny - 1] = dm[3] * UW[0][t - 2].x + dm[4] * UW[0][t - 1].x + dm[5] * UW[0][t].x;
+        a.dudy[ny - 1] = dm[3] * UW[0][t >= 2 ? t - 2 : 0].x + dm[4] * UW[0][t >= 1 ? t - 1 : 0].x + dm[5] * UW[0][t].x;
     }
   }
   if (!valid) return;
+#pragma unroll
+  for (int t = 0; t < SEG; ++t) {
+    const int j = j0 + t;
+    if ((!last || t < rl) && (!first || t >= f)) {
+      sto(U, OC(0, j), UW[0][t]);
+      sto(U, OC(1, j), V[0][t]);
+      sto(U, OC(2, j), UW[1][t]);
+      sto(P, OM(j), PR[t]);
+    }
+  }
   if (a.rk == 3) {
 #pragma unroll
     for (int t = 0; t < SEG; ++t) {
       const int j = j0 + t;
-      if (j <= ny) {
+      if ((!last || t < rl) && (!first || t >= f)) {
         sto(R, OC(0, j), UW[0][t]);
         sto(R, OC(1, j), V[0][t]);
         sto(R, OC(2, j), UW[1][t]);
@@ -920,48 +1044,46 @@ __device__ __forceinline__ void solve_seg_body(const DevOps& ops, const SolveArg
   const double rk_press2 = (c_rkc[r + 1] + c_rkd[r + 1]) * dt;
 #pragma unroll
   for (int t = 0; t < SEG; ++t) {
-    const int j = j0 + t, jc = min(j, ny), jv = min(j, ny - 1);
-    const double2 n0 = stash[t][0][lane], n1 = stash[t][1][lane], n2 = stash[t][2][lane];
-    const double a0 = d2h[3 * jc], a1 = d2h[3 * jc + 1], a2 = d2h[3 * jc + 2];
-    const double b0 = d2n[3 * jv], b1 = d2n[3 * jv + 1], b2 = d2n[3 * jv + 2];
-    const double dnj = dn[jv];
+    const int j = j0 + t, jc = rowc(j), jv = min(jc, ny - 1);
+    const int tm1 = t >= 1 ? t - 1 : 0, tm2 = t >= 2 ? t - 2 : 0, tp1 = t + 1 < SEG ? t + 1 : t;
     // D2H / D2N stencil rows j-1, j, j+1; rows 0..2 at the bottom, the last three at the top
-    double2 u0 = (t > 0) ? UW[0][t - 1] : uP, u1 = UW[0][t], u2 = (t + 1 < SEG) ? UW[0][t + 1] : uN;
-    double2 w0 = (t > 0) ? UW[1][t - 1] : wP, w1 = UW[1][t], w2 = (t + 1 < SEG) ? UW[1][t + 1] : wN;
-    double2 x0 = (t > 0) ? V[0][t - 1] : vP, x1 = V[0][t], x2 = (t + 1 < SEG) ? V[0][t + 1] : vN;
-    if (t == 0) {
-      const bool b = (j == 0);
-      u0 = sel(b, UW[0][0], u0); u1 = sel(b, UW[0][1], u1); u2 = sel(b, UW[0][2], u2);
-      w0 = sel(b, UW[1][0], w0); w1 = sel(b, UW[1][1], w1); w2 = sel(b, UW[1][2], w2);
-      x0 = sel(b, V[0][0], x0); x1 = sel(b, V[0][1], x1); x2 = sel(b, V[0][2], x2);
+    double2 u0 = (t > 0) ? UW[0][tm1] : uP, u1 = UW[0][t], u2 = (t + 1 < SEG) ? UW[0][tp1] : uN;
+    double2 w0 = (t > 0) ? UW[1][tm1] : wP, w1 = UW[1][t], w2 = (t + 1 < SEG) ? UW[1][tp1] : wN;
+    double2 x0 = (t > 0) ? V[0][tm1] : vP, x1 = V[0][t], x2 = (t + 1 < SEG) ? V[0][tp1] : vN;
+    double pg = rk_press2, pgv = rk_press2, vv = vis_exp2;   // zero where the wall rows have no such term
+    if (t < SEG - 2 && t == f && first) {
+      const int tp2 = t + 2 < SEG ? t + 2 : t;
+      u0 = UW[0][t]; u1 = UW[0][tp1]; u2 = UW[0][tp2];
+      w0 = UW[1][t]; w1 = UW[1][tp1]; w2 = UW[1][tp2];
+      x0 = V[0][t]; x1 = V[0][tp1]; x2 = V[0][tp2];
+      pg = pgv = 0.0;
     }
-    if (t >= 2) {
-      const bool b = (j == ny);
-      u0 = sel(b, UW[0][t - 2], u0); u1 = sel(b, UW[0][t - 1], u1); u2 = sel(b, UW[0][t], u2);
-      w0 = sel(b, UW[1][t - 2], w0); w1 = sel(b, UW[1][t - 1], w1); w2 = sel(b, UW[1][t], w2);
+    if (t >= 2 && t == rl - 1 && last) {
+      u0 = UW[0][tm2]; u1 = UW[0][tm1]; u2 = UW[0][t];
+      w0 = UW[1][tm2]; w1 = UW[1][tm1]; w2 = UW[1][t];
+      pg = pgv = vv = 0.0;
     }
-    if (t >= 1) {  // last v row: rows ny-3 .. ny-1
-      const bool b = (j == ny - 1);
-      x0 = sel(b, (t >= 2) ? V[0][t - 2] : vP, x0);
-      x1 = sel(b, V[0][t - 1], x1);
-      x2 = sel(b, V[0][t], x2);
+    if (t >= 1 && t == rl - 2 && last) {  // last v row: rows ny-3 .. ny-1
+      x0 = t >= 2 ? V[0][tm2] : vP; x1 = V[0][tm1]; x2 = V[0][t];
+      pgv = 0.0;
     }
     const double2 cu = UW[0][t], cv = V[0][t], cw = UW[1][t];
-    double2 o0 = cadd(cu, rmul(coef2, neg(n0)));
-    double2 o1 = cadd(cv, rmul(coef2, neg(n1)));
-    double2 o2 = cadd(cw, rmul(coef2, neg(n2)));
+    double2 o0 = csub(cu, rmul(coef2, nls(0, t)));
+    double2 o1 = csub(cv, rmul(coef2, nls(1, t)));
+    double2 o2 = csub(cw, rmul(coef2, nls(2, t)));
+    const double a0 = d2h[3 * jc], a1 = d2h[3 * jc + 1], a2 = d2h[3 * jc + 2];
+    const double b0 = d2n[3 * jv], b1 = d2n[3 * jv + 1], b2 = d2n[3 * jv + 2];
     const double2 du = cadd(cadd(rmul(a0, u0), rmul(a1, u1)), rmul(a2, u2));
     const double2 dw = cadd(cadd(rmul(a0, w0), rmul(a1, w1)), rmul(a2, w2));
+    const double2 dv = cadd(cadd(rmul(b0, x0), rmul(b1, x1)), rmul(b2, x2));
     o0 = cadd(o0, rmul(vis_exp2, csub(du, rmul(k2, cu))));
     o2 = cadd(o2, rmul(vis_exp2, csub(dw, rmul(k2, cw))));
-    const double2 dv = cadd(cadd(rmul(b0, x0), rmul(b1, x1)), rmul(b2, x2));
-    o1 = sel(j < ny, cadd(o1, rmul(vis_exp2, csub(dv, rmul(k2, cv)))), o1);
-    const double2 Pj = PN[t], Pj1 = (t + 1 < SEG) ? PN[t + 1] : pnN;
-    const bool inner = !mean && j >= 1 && j <= ny - 1;
-    o0 = sel(inner, csub(o0, imul(rk_press2 * kxv, Pj)), o0);
-    o2 = sel(inner, csub(o2, imul(rk_press2 * kzv, Pj)), o2);
-    o1 = sel(inner && j <= ny - 2, csub(o1, rmul(rk_press2 * dnj, csub(Pj1, Pj))), o1);
-    if (j <= ny) {
+    o1 = cadd(o1, rmul(vv, csub(dv, rmul(k2, cv))));
+    const double2 Pj = PR[t], Pj1 = (t + 1 < SEG) ? PR[tp1] : pnN;
+    o0 = csub(o0, imul(pg * kxv, Pj));
+    o2 = csub(o2, imul(pg * kzv, Pj));
+    o1 = csub(o1, rmul(pgv * dn[jv], csub(Pj1, Pj)));
+    if ((!last || t < rl) && (!first || t >= f)) {
       sto(R, OC(0, j), o0);
       sto(R, OC(1, j), o1);
       sto(R, OC(2, j), o2);
@@ -969,32 +1091,64 @@ __device__ __forceinline__ void solve_seg_body(const DevOps& ops, const SolveArg
   }
 }
 
-template <int MODES, int SEG>
-__global__ __launch_bounds__(64) void k_solve_seg(DevOps ops, SolveArgs a) {
-  solve_seg_body<MODES, SEG>(ops, a, blockIdx.x, gridDim.x);
+template <int SEG>
+__global__ __launch_bounds__(512) void k_solve_wg(DevOps ops, SolveArgs a) {
+  solve_wg_body<SEG>(ops, a, blockIdx.x);
 }
 
 // Batched form: workgroup i runs mode group it[i].bx of channel it[i].m.
-template <int MODES, int SEG>
-__global__ __launch_bounds__(64) void k_solve_seg_b(const SBatchArgs* __restrict__ args,
+template <int SEG>
+__global__ __launch_bounds__(512) void k_solve_wg_b(const SBatchArgs* __restrict__ args,
                                                     const BatchItem* __restrict__ it) {
   const BatchItem w = it[blockIdx.x];
   const SBatchArgs& x = args[w.m];
-  solve_seg_body<MODES, SEG>(x.ops, x.a, w.bx, 0);
+  solve_wg_body<SEG>(x.ops, x.a, w.bx);
 }
 
-// Rows per segment of the segmented solve for ny+1 rows: the shortest of
-// 5..9 with at most maxsegs segments (64 / modes per wavefront) and 3 or more
-// rows in the last one (the wall rows 0..2 and ny-2..ny each lie in one
-// segment); 0 if none fits.
-int solve_seg_rows(int ny, int maxsegs) {
-  const int nyp = ny + 1;
+// LDS and threads of a k_solve_wg workgroup
+static size_t solve_wg_lds(int ny, int seg) {
+  const int nyp = ny + 1, na = ((nyp + seg - 1) / seg) * SOLVE_WG_MODES;
+  return sizeof(double2) * ((size_t)(SOLVE_WG_SLOTS + 3 * seg) * na + 7 * SOLVE_WG_MODES) +
+         sizeof(double) * (4 * nyp + 4 * ny + 18);  // with dm(3,4) and the even padding between
+}
+static int solve_wg_threads(int ny, int seg) {
+  const int na = ((ny + seg) / seg) * SOLVE_WG_MODES;
+  return (na + 63) / 64 * 64;
+}
+
+// Rows per segment of the workgroup solve for ny+1 rows (0: none): the
+// shortest of 3, 4, 5 that leaves room for two workgroups of at most 256
+// threads on a compute unit, else the longest that fits one.  A shorter
+// segment is a shorter serial chain: 66 rows take 16.4 us with 3 rows, 17.8
+// with 5 (64x65x64), 98 rows 20.5 with 4, 20.8 with 5 (64x97x64).  But 130
+// rows of 4 make 264 threads, one workgroup per compute unit: 197 us against
+// 155 (192x129x192, an earlier form of the kernel; its 6 rows took 233 us,
+// for want of registers).  The padding rows (pad) must leave 3 rows in the
+// first and in the last segment, which 5 rows always do.
+int solve_wg_seg(int ny, int solve_seg) {
   if (ny < 8) return 0;
+  auto fits = [&](int seg) {
+    const int ns = (ny + seg) / seg;
+    return ns * seg - (ny + 1) <= 2 * (seg - 3) && solve_wg_threads(ny, seg) <= 512 && solve_wg_lds(ny, seg) <= 163840;
+  };
+  if (solve_seg == 2 && fits(5)) return 5;
+  for (int seg = 3; seg <= 5; ++seg)
+    if (fits(seg) && solve_wg_threads(ny, seg) <= 256 && solve_wg_lds(ny, seg) <= 81920) return seg;
+  for (int seg = 5; seg >= 3; --seg)
+    if (fits(seg)) return seg;
+  return 0;
+}
+
+// The columns a batched ensemble takes: ny + 1 rows in at most 16 segments of
+// 5..9 rows with 3 or more in the last one.
+bool solve_batchable(int ny) {
+  const int nyp = ny + 1;
+  if (ny < 8) return false;
   for (int seg = 5; seg <= 9; ++seg) {
     const int ns = (nyp + seg - 1) / seg, rl = nyp - (ns - 1) * seg;
-    if (ns <= maxsegs && rl >= 3) return seg;
+    if (ns <= 16 && rl >= 3) return true;
   }
-  return 0;
+  return false;
 }
 
 // ---- direct global-to-LDS row ring (the DMA variant of k_solve3) ----
@@ -1466,43 +1620,16 @@ void launch_solve(const DevOps& ops, const SolveArgs& a, hipStream_t s) {
   // the segmented and component-parallel kernels need the byte offsets of one
   // array to fit 32 bits
   const bool off32 = 3.0 * (a.ny + 1) * (double)nm * 16.0 < 4.0e9;
-  // two modes per wavefront (32 segments): the 5-row segments keep the
-  // wavefront within 256 registers, two wavefronts per SIMD
-  const int seg2 = (a.seg == 2) ? solve_seg_rows(a.ny, 32) : 0;
-  if (seg2 == 5 && off32) {
-    dim3 gs((unsigned)((nm + 1) / 2));
-    hipLaunchKernelGGL((k_solve_seg<2, 5>), gs, dim3(64), 0, s, ops, a);
-    LAUNCH_CHECK("k_solve_seg");
-    return;
-  }
-  // eight modes per wavefront (8 segments) where ny+1 rows fit 8 segments of
-  // 5..9 rows: 128-byte row pieces, and fewer idle segment lanes at ny + 1
-  // just under 8 SEG (66 rows: 8 segments of 9 rows, against 11 of 16 lanes
-  // groups busy with 6-row segments)
-  const int seg8 = (a.seg == 3) ? solve_seg_rows(a.ny, 8) : 0;
-  if (seg8 && off32) {
-    dim3 gs((unsigned)((nm + 7) / 8));
-    switch (seg8) {
-      case 5: hipLaunchKernelGGL((k_solve_seg<8, 5>), gs, dim3(64), 0, s, ops, a); break;
-      case 6: hipLaunchKernelGGL((k_solve_seg<8, 6>), gs, dim3(64), 0, s, ops, a); break;
-      case 7: hipLaunchKernelGGL((k_solve_seg<8, 7>), gs, dim3(64), 0, s, ops, a); break;
-      case 8: hipLaunchKernelGGL((k_solve_seg<8, 8>), gs, dim3(64), 0, s, ops, a); break;
-      default: hipLaunchKernelGGL((k_solve_seg<8, 9>), gs, dim3(64), 0, s, ops, a); break;
-    }
-    LAUNCH_CHECK("k_solve_seg");
-    return;
-  }
-  const int seg = a.seg ? solve_seg_rows(a.ny) : 0;
+  const int seg = a.seg ? solve_wg_seg(a.ny, a.seg) : 0;
   if (seg && off32) {
-    dim3 gs((unsigned)((nm + 3) / 4));
+    const dim3 gs((unsigned)((nm + SOLVE_WG_MODES - 1) / SOLVE_WG_MODES)), bs(solve_wg_threads(a.ny, seg));
+    const size_t lds = solve_wg_lds(a.ny, seg);
     switch (seg) {
-      case 5: hipLaunchKernelGGL((k_solve_seg<4, 5>), gs, dim3(64), 0, s, ops, a); break;
-      case 6: hipLaunchKernelGGL((k_solve_seg<4, 6>), gs, dim3(64), 0, s, ops, a); break;
-      case 7: hipLaunchKernelGGL((k_solve_seg<4, 7>), gs, dim3(64), 0, s, ops, a); break;
-      case 8: hipLaunchKernelGGL((k_solve_seg<4, 8>), gs, dim3(64), 0, s, ops, a); break;
-      default: hipLaunchKernelGGL((k_solve_seg<4, 9>), gs, dim3(64), 0, s, ops, a); break;
+      case 3: hipLaunchKernelGGL((k_solve_wg<3>), gs, bs, lds, s, ops, a); break;
+      case 4: hipLaunchKernelGGL((k_solve_wg<4>), gs, bs, lds, s, ops, a); break;
+      default: hipLaunchKernelGGL((k_solve_wg<5>), gs, bs, lds, s, ops, a); break;
     }
-    LAUNCH_CHECK("k_solve_seg");
+    LAUNCH_CHECK("k_solve_wg");
     return;
   }
   if (lanes == 3 && off32) {
@@ -1803,38 +1930,26 @@ void launch_advance_time_batched(DevScalars* const* sc, int n, hipStream_t s) {
   LAUNCH_CHECK("k_advance_time_b");
 }
 
-// The segmented solve of several channels with the same segment length in one launch.
-// layout = 16 * modes per wavefront + rows per segment (solve_seg_layout)
-void launch_solve_batched(int layout, const SBatchArgs* args, const BatchItem* items, int nitems, hipStream_t s) {
+// The segmented solve of several channels with the same segment length and
+// thread count (solve_wg_layout) in one launch; ny: the largest of them.
+void launch_solve_batched(int layout, int ny, const SBatchArgs* args, const BatchItem* items, int nitems,
+                          hipStream_t s) {
   if (nitems <= 0) return;
-  switch (layout) {
-    case 64 + 5: hipLaunchKernelGGL((k_solve_seg_b<4, 5>), dim3(nitems), dim3(64), 0, s, args, items); break;
-    case 64 + 6: hipLaunchKernelGGL((k_solve_seg_b<4, 6>), dim3(nitems), dim3(64), 0, s, args, items); break;
-    case 64 + 7: hipLaunchKernelGGL((k_solve_seg_b<4, 7>), dim3(nitems), dim3(64), 0, s, args, items); break;
-    case 64 + 8: hipLaunchKernelGGL((k_solve_seg_b<4, 8>), dim3(nitems), dim3(64), 0, s, args, items); break;
-    case 64 + 9: hipLaunchKernelGGL((k_solve_seg_b<4, 9>), dim3(nitems), dim3(64), 0, s, args, items); break;
-    case 128 + 5: hipLaunchKernelGGL((k_solve_seg_b<8, 5>), dim3(nitems), dim3(64), 0, s, args, items); break;
-    case 128 + 6: hipLaunchKernelGGL((k_solve_seg_b<8, 6>), dim3(nitems), dim3(64), 0, s, args, items); break;
-    case 128 + 7: hipLaunchKernelGGL((k_solve_seg_b<8, 7>), dim3(nitems), dim3(64), 0, s, args, items); break;
-    case 128 + 8: hipLaunchKernelGGL((k_solve_seg_b<8, 8>), dim3(nitems), dim3(64), 0, s, args, items); break;
-    case 128 + 9: hipLaunchKernelGGL((k_solve_seg_b<8, 9>), dim3(nitems), dim3(64), 0, s, args, items); break;
+  const int seg = layout & 15, threads = layout >> 4;
+  const size_t lds = solve_wg_lds(ny, seg);
+  if (threads != solve_wg_threads(ny, seg)) throw chan_error("batched solve: layout of another column length");
+  switch (seg) {
+    case 3: hipLaunchKernelGGL((k_solve_wg_b<3>), dim3(nitems), dim3(threads), lds, s, args, items); break;
+    case 4: hipLaunchKernelGGL((k_solve_wg_b<4>), dim3(nitems), dim3(threads), lds, s, args, items); break;
+    case 5: hipLaunchKernelGGL((k_solve_wg_b<5>), dim3(nitems), dim3(threads), lds, s, args, items); break;
     default: throw chan_error("batched solve: no segmented solve of layout " + std::to_string(layout));
   }
-  LAUNCH_CHECK("k_solve_seg_b");
+  LAUNCH_CHECK("k_solve_wg_b");
 }
 
-int solve_seg_layout(int ny, int solve_seg) {
-  // The batched launches take 8 modes per wavefront by default where all 8
-  // segments are busy (66 rows: 8 of 9 rows, against 11 of 16 segments of 6
-  // rows with 4 modes): 179 -> 182 steps/s on the 48-member ensemble, whose
-  // launches keep the GPU full.  Where segments would idle (50 rows: 6 of 8)
-  // it was slower, and so is a single channel with fewer than ~4000 modes,
-  // whose wavefronts are then too few (64x65x64: 21 -> 26 us per solve).
-  int s8 = (solve_seg == 1 || solve_seg == 3) ? solve_seg_rows(ny, 8) : 0;
-  if (s8 && solve_seg == 1 && (ny + 1 + s8 - 1) / s8 < 8) s8 = 0;
-  if (s8) return 128 + s8;
-  const int s4 = solve_seg_rows(ny);
-  return s4 ? 64 + s4 : 0;
+int solve_wg_layout(int ny, int solve_seg) {
+  const int seg = solve_wg_seg(ny, solve_seg);
+  return seg ? 16 * solve_wg_threads(ny, seg) + seg : 0;
 }
 
 // max |ikx u + dh (v_j - v_{j-1}) + ikz w| over non-mean modes, j = 2..ny

@@ -249,11 +249,10 @@ int chan_jet_configure(chan_ctx* ctx, int wall, double amplitude, double radius,
  * 9 planes per x-pass workgroup (2..64; 0, the default: the plane-rows of the
  * pass spread evenly over the workgroups resident at a time), 10 plane
  * ranges the nonlinear pass runs in turn (1..64; 1: every kernel over all
- * planes), 11 segmented column solve (1 on with 4 modes per wavefront, 2
- * with 2 modes per wavefront, 3 with 8 modes per wavefront, 0 off) wherever
- * ny+1 rows fit 16 (32, 8) segments of 5 to 9 (5, 5 to 9) rows (keys 3, 4
- * and 8 then do not apply; value 3 falls back to 1 where 8 segments are too
- * few), 12 z-rows per
+ * planes), 11 segmented column solve (1 on, the y column of a mode in segments
+ * of 3, 4 or 5 rows by its length; 2 on with 5 rows; 3 as 1; 0 off) wherever
+ * the column fits a workgroup (ny up to about 280; keys 3, 4 and 8 then do
+ * not apply), 12 z-rows per
  * wavefront of the wavefront x-pass (0, the default: by length; 1; 2 for
  * nx2/2 <= 72; 4 for nx2/2 <= 24; with the prefetch, where nz2 is a multiple;
  * otherwise the default applies; a batched ensemble takes the fewest rows its
@@ -261,8 +260,8 @@ int chan_jet_configure(chan_ctx* ctx, int wall, double amplitude, double radius,
  * chan_autotune times `steps` timesteps of every candidate (keys 0 and 2,
  * key 0 fixed at 1 while a subgrid closure is configured; with the wavefront
  * x-pass, key 12's row counts the length has; the
- * segmented solve's layouts of key 11 that ny + 1 rows fit, or the
- * sweep-based solves with keys 3, 4 and 8), keeps the fastest whose trial
+ * segmented solve's rows per segment (key 11 = 1, 2), or the sweep-based
+ * solves with keys 3, 4 and 8), keeps the fastest whose trial
  * passed the CFL check and restores the state. */
 int chan_set_tuning(chan_ctx* ctx, int key, int value);
 int chan_get_tuning(chan_ctx* ctx, int key, int* value);
@@ -293,8 +292,8 @@ int chan_ensemble_invalidate(chan_ensemble* ens);
  * plan (each length's planes cut for 1, 2, 4 or 8 times, or as many times as
  * there are lengths, its resident workgroups), then, with the fastest ranges,
  * the tile shapes (one z-row per x-pass wavefront at every length instead of
- * the batched default; 4 modes per solve wavefront everywhere instead of 8
- * where all 8 segments are busy), restores every member's state after each
+ * the batched default; 5 rows per solve segment everywhere instead of 3 to 5
+ * by length), restores every member's state after each
  * trial, keeps the fastest plan and returns its time per step (on failure
  * the state is restored as well and the previous plan kept).  The ranges
  * give every member the same arithmetic; the tile shapes the same to
