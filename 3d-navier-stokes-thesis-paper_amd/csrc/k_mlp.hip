@@ -12,8 +12,8 @@
 // A-operand order (lane l: row l%16, k = 4(l/16)..+3), sit in LDS for the
 // whole persistent workgroup.
 //
-// Training runs in float32 with one tiled GEMM kernel and fused epilogues
-// (bias, GELU, GELU derivative), a mean-squared-error gradient and Adam.
+// Training runs in float32 on the matrix cores: one kernel takes points
+// through the network and back, a second sums the gradients and applies Adam.
 #include "chan_internal.h"
 #include <cmath>
 
@@ -283,106 +283,292 @@ __global__ __launch_bounds__(64 * MLP_WAVES, 2) void k_mlp_infer(const bf16x4* _
 }
 
 // ---------------------------------------------------------------------------
-// float32 training kernels
+// float32 training
+//
+// k_mlp_grad takes 16 points at a time through the whole network and back
+// (forward only without GRAD), on the float32 matrix cores
+// (v_mfma_f32_16x16x4_f32: full float32 products and sums).  The activations
+// and GELU derivatives of the 16 points stay in LDS, the weights in registers
+// (each loaded once, in the order of use; the backward pass takes a layer's
+// from a copy in LDS), and a workgroup's weight gradients stay in accumulators
+// over all its points; it writes them once, as one partial gradient, and
+// k_mlp_update sums the partial gradients in a fixed order (and applies Adam).
+//
+// A mini-batch is small (1024 points: 0.2 GFLOP, 1.4 us of matrix work), so
+// what counts is the number of launches and of workgroups: two launches per
+// batch, one workgroup per 16 points.  One tiled product per layer and
+// direction took 24 launches, its weight gradients on 4 workgroups that ran
+// over all points (175 us each), and a wait for the loss: 835 us a batch of
+// 1024 against 32 us now (22 us in k_mlp_grad, of which 5 us are the weights'
+// first loads, and 6 us in k_mlp_update).
 // ---------------------------------------------------------------------------
-// C(m, n) = sum_k A(m, k) B(k, n), A(m, k) = a[m*as0 + k*as1], B(k, n) = b[k*bs0 + n*bs1],
-// C row-major with row stride ldc.  Epilogue: EPI 0 plain; 1 + bias[n], store
-// the pre-activation in C and GELU of it in act (or C only when act is null,
-// i.e. a linear layer); 2 multiply by gelu'(aux[m*ldc + n]).
-template <int EPI>
-__global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, const float* __restrict__ a, long as0, long as1,
-                                              const float* __restrict__ b, long bs0, long bs1, float* __restrict__ c,
-                                              long ldc, const float* __restrict__ bias, float* __restrict__ act,
-                                              const float* __restrict__ aux) {
-  __shared__ float As[16][65], Bs[16][65];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-      const int kk = e & 15, mm = e >> 4;
-      const int gm = m0 + mm, gk = k0 + kk;
-      As[kk][mm] = (gm < M && gk < K) ? a[gm * as0 + gk * as1] : 0.0f;
-      const int nn = e >> 4;
-      const int gn = n0 + nn;
-      Bs[kk][nn] = (gn < N && gk < K) ? b[gk * bs0 + gn * bs1] : 0.0f;
-    }
-    __syncthreads();
+#define MLP_TP 16              // points per tile
+#define MLP_LD 132             // LDS row of 128 features (16-byte aligned, 4 banks apart)
+#define MLP_LX 20              // LDS row of 16 values
+#define MLP_MAXWG 256          // partial gradients
+
+struct MlpLds {
+  float wt[128][MLP_LD];            // the weights the backward pass is at
+  float x[MLP_TP][MLP_LX];          // inputs, 10 padded to 16
+  float a[3][MLP_TP][MLP_LD];       // activations of the hidden layers
+  float g[3][MLP_TP][MLP_LD];       // their GELU derivatives
+  float d[2][MLP_TP][MLP_LD];       // dL/dz of the current layer
+  float d4[MLP_TP][MLP_LX];         // dL/dy, 6 padded to 16
+  float y4[8][MLP_TP][MLP_LX];      // output layer, one part per wavefront
+};
+
+__device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Operand layout of the 16x16x4 product: lane l = 16 g + r holds row r of A
+// and column r of B at k = g; a k-block of 16 is fed as four products whose
+// k = g stands for element 4g + j.  Result: column r, rows 4g .. 4g+3.
+template <bool GRAD>
+__global__ __launch_bounds__(512) void k_mlp_grad(const float* __restrict__ p, int n, const float* __restrict__ x,
+                                                  const float* __restrict__ t, float* __restrict__ y, float sc,
+                                                  float* __restrict__ part, double* __restrict__ lpart) {
+  extern __shared__ float4 mlp_lds[];
+  MlpLds& L = *reinterpret_cast<MlpLds*>(mlp_lds);
+  const int tid = threadIdx.x, w = tid >> 6, g = (tid & 63) >> 4, r = tid & 15;
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  const int o = 16 * w + r;   // the lane's feature: wavefront w has features 16w .. 16w+15 of every layer
+  // weight-gradient tiles of the wavefront: its output tile of layers 1-3 by
+  // every input tile, its input tile of layer 4
+  f32x4 w1 = zero, w2[8], w3[8], w4 = zero;
+  float b1 = 0.0f, b2 = 0.0f, b3 = 0.0f, b4 = 0.0f;
+  double loss = 0.0;
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float av[4], bv[4];
+  for (int v = 0; v < 8; ++v) w2[v] = w3[v] = zero;
+  // A tile's inputs and targets: threads below 256 = (point, value).  The
+  // first tile's go ahead of the weights, whose loads are issued in the order
+  // of their use and stay in registers over all tiles.
+  const int ti = tid >> 4, tk = tid & 15;
+  auto xload = [&](long base) { return (tid < 256 && tk < 10 && base + ti < n) ? x[(base + ti) * 10 + tk] : 0.0f; };
+  auto tload = [&](long base) {
+    return (GRAD && tid < 256 && tk < 6 && base + ti < n) ? t[(base + ti) * 6 + tk] : 0.0f;
+  };
+  float xv = xload((long)blockIdx.x * MLP_TP), tv = tload((long)blockIdx.x * MLP_TP);
+  __builtin_amdgcn_sched_barrier(0);
+  float q1[4], q4b[4];
+  float4 q2[8], q3[8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) { av[i] = As[kk][ty + 16 * i]; bv[i] = Bs[kk][tx + 16 * i]; }
+  for (int j = 0; j < 4; ++j) q1[j] = 4 * g + j < 10 ? p[MLP_W1 + o * 10 + 4 * g + j] : 0.0f;
+  const float c1 = p[MLP_B1 + o], c2 = p[MLP_B2 + o], c3 = p[MLP_B3 + o];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+  for (int k = 0; k < 8; ++k) q2[k] = *reinterpret_cast<const float4*>(p + MLP_W2 + o * 128 + 16 * k + 4 * g);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
-    }
-    __syncthreads();
+  for (int k = 0; k < 8; ++k) q3[k] = *reinterpret_cast<const float4*>(p + MLP_W3 + o * 128 + 16 * k + 4 * g);
+  const float4 q4 = r < 6 ? *reinterpret_cast<const float4*>(p + MLP_W4 + r * 128 + 16 * w + 4 * g)
+                          : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const float c4 = tk < 6 ? p[MLP_B4 + tk] : 0.0f;
+  if (GRAD) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) q4b[j] = 4 * g + j < 6 ? p[MLP_W4 + (4 * g + j) * 128 + o] : 0.0f;
   }
+  // hidden layer of 128 inputs `in` with weights q and bias b into (a, gelu')
+  auto hidden = [&](const float (*in)[MLP_LD], const float4 (&q)[8], float b, float (*oa)[MLP_LD],
+                    float (*og)[MLP_LD]) {
+    f32x4 c = zero;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int k = 0; k < 8; ++k) {
+      const float4 a = *reinterpret_cast<const float4*>(&in[r][16 * k + 4 * g]);
+      c = mfma_f32(a.x, q[k].x, c); c = mfma_f32(a.y, q[k].y, c);
+      c = mfma_f32(a.z, q[k].z, c); c = mfma_f32(a.w, q[k].w, c);
+    }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gm = m0 + ty + 16 * i, gn = n0 + tx + 16 * j;
-      if (gm >= M || gn >= N) continue;
-      float v = acc[i][j];
-      const long o = (long)gm * ldc + gn;
-      if (EPI == 1) {
-        v += bias[gn];
-        c[o] = v;
-        if (act) act[o] = gelu_f(v);
-      } else if (EPI == 2) {
-        c[o] = v * gelu_grad_f(aux[o]);
-      } else {
-        c[o] = v;
+    for (int i = 0; i < 4; ++i) {
+      const float z = c[i] + b;
+      oa[4 * g + i][o] = gelu_f(z);
+      if (GRAD) og[4 * g + i][o] = gelu_grad_f(z);
+    }
+  };
+  // weights (rows o, as the forward pass holds them) to LDS for the backward
+  // pass, which takes them by columns
+  auto stage = [&](const float4 (&q)[8]) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) *reinterpret_cast<float4*>(&L.wt[o][16 * k + 4 * g]) = q[k];
+  };
+  // dL/dz of the layer below: (D W) gelu', W in L.wt
+  auto back = [&](const float (*D)[MLP_LD], const float (*gp)[MLP_LD], float (*out)[MLP_LD]) {
+    f32x4 c = zero;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float4 a = *reinterpret_cast<const float4*>(&D[r][16 * k + 4 * g]);
+      const float(*W)[MLP_LD] = L.wt + 16 * k + 4 * g;
+      c = mfma_f32(a.x, W[0][o], c); c = mfma_f32(a.y, W[1][o], c);
+      c = mfma_f32(a.z, W[2][o], c); c = mfma_f32(a.w, W[3][o], c);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[4 * g + i][o] = c[i] * gp[4 * g + i][o];
+  };
+  // acc[v] += D^T A over the 16 points, the wavefront's output tile by input tile v
+  auto wgrad = [&](const float (*D)[MLP_LD], const float (*A)[MLP_LD], f32x4 (&acc)[8]) {
+    float dv[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dv[j] = D[4 * g + j][o];
+#pragma unroll
+    for (int v = 0; v < 8; ++v)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[v] = mfma_f32(dv[j], A[4 * g + j][16 * v + r], acc[v]);
+  };
+  auto colsum = [&](const float (*D)[MLP_LD]) {
+    float v = 0.0f;
+#pragma unroll
+    for (int i = 0; i < MLP_TP; ++i) v += D[i][tid & 127];
+    return v;
+  };
+
+  const int ntile = (n + MLP_TP - 1) / MLP_TP;
+  for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+    const long base = (long)tile * MLP_TP;
+    const float target = tv;
+    if (tid < 256) L.x[ti][tk] = xv;
+    __syncthreads();
+    xv = xload(base + (long)gridDim.x * MLP_TP);
+    tv = tload(base + (long)gridDim.x * MLP_TP);
+    {  // layer 1, K = 10 padded to 16
+      const float4 a = *reinterpret_cast<const float4*>(&L.x[r][4 * g]);
+      const float av[4] = {a.x, a.y, a.z, a.w};
+      f32x4 c = zero;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c = mfma_f32(av[j], q1[j], c);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float z = c[i] + c1;
+        L.a[0][4 * g + i][o] = gelu_f(z);
+        if (GRAD) L.g[0][4 * g + i][o] = gelu_grad_f(z);
       }
     }
-}
-
-// d = 2 (y - t)/(n*m); partial sums of (y - t)^2 per workgroup into part.
-__global__ __launch_bounds__(256) void k_mse_grad(long nm, const float* __restrict__ yv, const float* __restrict__ t,
-                                                  float* __restrict__ d, double* __restrict__ part) {
-  __shared__ double red[4];
-  double s = 0.0;
-  const float sc = 2.0f / (float)nm;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < nm; i += (long)gridDim.x * blockDim.x) {
-    const float e = yv[i] - t[i];
-    d[i] = sc * e;
-    s += (double)e * (double)e;
-  }
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
-}
-
-// Column sums: g[j] = sum_i d[i*N + j] (bias gradients).
-__global__ __launch_bounds__(256) void k_colsum(int M, int N, const float* __restrict__ d, float* __restrict__ g) {
-  __shared__ float red[256];
-  const int j = blockIdx.x;
-  float s = 0.0f;
-  for (int i = threadIdx.x; i < M; i += blockDim.x) s += d[(long)i * N + j];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
     __syncthreads();
+    hidden(L.a[0], q2, c2, L.a[1], L.g[1]);
+    __syncthreads();
+    hidden(L.a[1], q3, c3, L.a[2], L.g[2]);
+    if (GRAD) stage(q3);
+    __syncthreads();
+    {  // output layer, 6 padded to 16: wavefront w sums its own features
+      f32x4 c = zero;
+      const float4 a = *reinterpret_cast<const float4*>(&L.a[2][r][16 * w + 4 * g]);
+      c = mfma_f32(a.x, q4.x, c); c = mfma_f32(a.y, q4.y, c);
+      c = mfma_f32(a.z, q4.z, c); c = mfma_f32(a.w, q4.w, c);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) L.y4[w][4 * g + i][r] = c[i];
+    }
+    __syncthreads();
+    if (tid < 256) {
+      const int i = ti, k = tk;
+      const bool ok = k < 6 && base + i < n;
+      float d = 0.0f;
+      if (ok) {
+        const float v = ((L.y4[0][i][k] + L.y4[1][i][k]) + (L.y4[2][i][k] + L.y4[3][i][k])) +
+                        ((L.y4[4][i][k] + L.y4[5][i][k]) + (L.y4[6][i][k] + L.y4[7][i][k])) + c4;
+        const long at = (base + i) * 6 + k;
+        if (GRAD) {
+          const float e = v - target;
+          d = sc * e;
+          loss += (double)e * (double)e;
+        } else {
+          y[at] = v;
+        }
+      }
+      if (GRAD) L.d4[i][k] = d;
+    }
+    if (GRAD) {
+      __syncthreads();
+      {  // layer 4: its weight gradient, and dL/dz of layer 3
+        const float4 a = *reinterpret_cast<const float4*>(&L.d4[r][4 * g]);
+        const float av[4] = {a.x, a.y, a.z, a.w};
+        f32x4 c = zero;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          w4 = mfma_f32(L.d4[4 * g + j][r], L.a[2][4 * g + j][o], w4);
+          c = mfma_f32(av[j], q4b[j], c);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) L.d[0][4 * g + i][o] = c[i] * L.g[2][4 * g + i][o];
+        if (tid < 6) {
+#pragma unroll
+          for (int i = 0; i < MLP_TP; ++i) b4 += L.d4[i][tid];
+        }
+      }
+      __syncthreads();
+      wgrad(L.d[0], L.a[1], w3);
+      b3 += colsum(L.d[0]);
+      back(L.d[0], L.g[1], L.d[1]);
+      __syncthreads();
+      stage(q2);
+      wgrad(L.d[1], L.a[0], w2);
+      b2 += colsum(L.d[1]);
+      __syncthreads();
+      back(L.d[1], L.g[0], L.d[0]);
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w1 = mfma_f32(L.d[0][4 * g + j][o], L.x[4 * g + j][r], w1);
+      b1 += colsum(L.d[0]);
+    }
+    __syncthreads();   // the tile's LDS is free
   }
-  if (threadIdx.x == 0) g[j] = red[0];
+  if (!GRAD) return;
+  float* q = part + (long)blockIdx.x * MLP_NPARAM;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 16 * w + 4 * g + i;
+    if (r < 10) q[MLP_W1 + row * 10 + r] = w1[i];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      q[MLP_W2 + row * 128 + 16 * v + r] = w2[v][i];
+      q[MLP_W3 + row * 128 + 16 * v + r] = w3[v][i];
+    }
+    if (4 * g + i < 6) q[MLP_W4 + (4 * g + i) * 128 + o] = w4[i];
+  }
+  if (tid < 128) {
+    q[MLP_B1 + tid] = b1;
+    q[MLP_B2 + tid] = b2;
+    q[MLP_B3 + tid] = b3;
+  }
+  if (tid < 6) q[MLP_B4 + tid] = b4;
+  __shared__ double red[8];
+  for (int s = 32; s > 0; s >>= 1) loss += __shfl_xor(loss, s, 64);
+  if ((tid & 63) == 0) red[w] = loss;
+  __syncthreads();
+  if (tid == 0) lpart[blockIdx.x] = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
 }
 
-// Adam (Kingma & Ba 2015, Algorithm 1), step t >= 1.
-__global__ void k_adam(int n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+// g = sum of the nw partial gradients (in double, in order), loss = sum of the
+// nw partial losses; with ADAM one step t >= 1 of Adam (Kingma & Ba 2015,
+// Algorithm 1) on the parameters.
+// A workgroup has 64 parameters; wavefront w sums every fourth partial.
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_mlp_update(int nw, const float* __restrict__ part,
+                                                    const double* __restrict__ lpart, float* __restrict__ g,
+                                                    double* __restrict__ loss, float* __restrict__ p,
+                                                    float* __restrict__ m, float* __restrict__ v, float lr, float b1,
+                                                    float b2, float eps, float c1, float c2) {
+  __shared__ double red[4][64];
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i = blockIdx.x * 64 + l, ic = min(i, MLP_NPARAM - 1);
+  const bool own = w == 0 && i < MLP_NPARAM;
+  const float m0 = ADAM && own ? m[i] : 0.0f, v0 = ADAM && own ? v[i] : 0.0f, p0 = ADAM && own ? p[i] : 0.0f;
+  double s = 0.0;
+#pragma unroll 16
+  for (int k = w; k < nw; k += 4) s += (double)part[(long)k * MLP_NPARAM + ic];
+  red[w][l] = s;
+  if (blockIdx.x == 0 && threadIdx.x == 64) {
+    double e = 0.0;
+    for (int k = 0; k < nw; ++k) e += lpart[k];
+    *loss = e;
+  }
+  __syncthreads();
+  if (!own) return;
+  const float gi = (float)((red[0][l] + red[1][l]) + (red[2][l] + red[3][l]));
+  g[i] = gi;
+  if (ADAM) {
+    const float mi = b1 * m0 + (1.0f - b1) * gi;
+    const float vi = b2 * v0 + (1.0f - b2) * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    p[i] = p0 - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -399,16 +585,14 @@ struct chan_mlp {
   int adam_t = 0;
   // work buffers (capacity in points)
   long cap = 0;
-  float *d_x = nullptr, *d_y = nullptr, *d_t = nullptr, *d_d = nullptr;
-  float *d_z[4] = {}, *d_a[3] = {}, *d_e[2] = {};
-  double* d_part = nullptr;
+  float *d_x = nullptr, *d_y = nullptr, *d_t = nullptr;
+  // partial gradients and losses of the training workgroups, and the loss
+  float* d_part = nullptr;
+  double* d_lpart = nullptr;
   std::string last_error;
 };
 
 namespace {
-
-const int kIn[4] = {10, 128, 128, 128}, kOut[4] = {128, 128, 128, 6};
-const int kW[4] = {MLP_W1, MLP_W2, MLP_W3, MLP_W4}, kB[4] = {MLP_B1, MLP_B2, MLP_B3, MLP_B4};
 
 void mchk(hipError_t e, const char* what) {
   if (e != hipSuccess) throw chan_error(std::string(what) + ": " + hipGetErrorString(e));
@@ -422,70 +606,48 @@ void mfree(T*& p) {
 
 void ensure_cap(chan_mlp* m, long n) {
   if (n <= m->cap) return;
-  mfree(m->d_x); mfree(m->d_y); mfree(m->d_t); mfree(m->d_d); mfree(m->d_part);
-  for (auto& z : m->d_z) mfree(z);
-  for (auto& a : m->d_a) mfree(a);
-  for (auto& e : m->d_e) mfree(e);
+  mfree(m->d_x); mfree(m->d_y); mfree(m->d_t);
+  m->cap = 0;
   mchk(hipMalloc(&m->d_x, sizeof(float) * 10 * n), "hipMalloc");
   mchk(hipMalloc(&m->d_y, sizeof(float) * 6 * n), "hipMalloc");
   mchk(hipMalloc(&m->d_t, sizeof(float) * 6 * n), "hipMalloc");
-  mchk(hipMalloc(&m->d_d, sizeof(float) * 6 * n), "hipMalloc");
-  for (int l = 0; l < 4; ++l) mchk(hipMalloc(&m->d_z[l], sizeof(float) * kOut[l] * n), "hipMalloc");
-  for (int l = 0; l < 3; ++l) mchk(hipMalloc(&m->d_a[l], sizeof(float) * 128 * n), "hipMalloc");
-  for (int l = 0; l < 2; ++l) mchk(hipMalloc(&m->d_e[l], sizeof(float) * 128 * n), "hipMalloc");
-  mchk(hipMalloc(&m->d_part, sizeof(double) * 1024), "hipMalloc");
   m->cap = n;
 }
 
-template <int EPI>
-void gemm(chan_mlp* m, int M, int N, int K, const float* a, long as0, long as1, const float* b, long bs0, long bs1,
-          float* c, long ldc, const float* bias = nullptr, float* act = nullptr, const float* aux = nullptr) {
-  dim3 grid((N + 63) / 64, (M + 63) / 64);
-  hipLaunchKernelGGL(k_gemm<EPI>, grid, dim3(256), 0, m->stream, M, N, K, a, as0, as1, b, bs0, bs1, c, ldc, bias,
-                     act, aux);
-  LAUNCH_CHECK("k_gemm");
+void ensure_partials(chan_mlp* m) {
+  if (!m->d_part) mchk(hipMalloc(&m->d_part, sizeof(float) * (size_t)MLP_NPARAM * MLP_MAXWG), "hipMalloc");
+  if (!m->d_lpart) mchk(hipMalloc(&m->d_lpart, sizeof(double) * (MLP_MAXWG + 1)), "hipMalloc");
 }
 
-// Forward pass of n points at d_x: pre-activations d_z[l], activations d_a[l]
-// (layer inputs of layers 2..4), outputs d_z[3].
-void forward32(chan_mlp* m, int n) {
-  const float* in = m->d_x;
-  for (int l = 0; l < 4; ++l) {
-    gemm<1>(m, n, kOut[l], kIn[l], in, kIn[l], 1, m->d_p + kW[l], 1, kIn[l], m->d_z[l], kOut[l], m->d_p + kB[l],
-            l < 3 ? m->d_a[l] : nullptr);
-    if (l < 3) in = m->d_a[l];
+int tile_blocks(long n) { return (int)std::min<long>(MLP_MAXWG, (n + MLP_TP - 1) / MLP_TP); }
+
+// Gradient of the mean squared error of n points (inputs x, targets t on the
+// device) into d_g and its sum of squares into d_lpart[MLP_MAXWG]; with
+// adam_t > 0 that step of Adam on the parameters.  Queued, not waited for.
+void gradient32(chan_mlp* m, int n, const float* x, const float* t, int adam_t, float lr) {
+  const int nw = tile_blocks(n);
+  hipLaunchKernelGGL((k_mlp_grad<true>), dim3(nw), dim3(512), sizeof(MlpLds), m->stream, m->d_p, n, x, t, nullptr,
+                     2.0f / (float)(6L * n), m->d_part, m->d_lpart);
+  LAUNCH_CHECK("k_mlp_grad");
+  const dim3 grid((MLP_NPARAM + 63) / 64);
+  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  if (adam_t > 0) {
+    const float c1 = 1.0f - std::pow(b1, (float)adam_t), c2 = 1.0f - std::pow(b2, (float)adam_t);
+    hipLaunchKernelGGL((k_mlp_update<true>), grid, dim3(256), 0, m->stream, nw, m->d_part, m->d_lpart, m->d_g,
+                       m->d_lpart + MLP_MAXWG, m->d_p, m->d_m, m->d_v, lr, b1, b2, eps, c1, c2);
+  } else {
+    hipLaunchKernelGGL((k_mlp_update<false>), grid, dim3(256), 0, m->stream, nw, m->d_part, m->d_lpart, m->d_g,
+                       m->d_lpart + MLP_MAXWG, m->d_p, m->d_m, m->d_v, lr, b1, b2, eps, 1.0f, 1.0f);
   }
+  LAUNCH_CHECK("k_mlp_update");
 }
 
-// Gradient of the mean squared error of n points (targets at d_t) into d_g;
-// returns the loss.
-double gradient32(chan_mlp* m, int n) {
-  forward32(m, n);
-  const long nm = 6L * n;
-  const int blocks = (int)std::min<long>(1024, (nm + 255) / 256);
-  hipLaunchKernelGGL(k_mse_grad, dim3(blocks), dim3(256), 0, m->stream, nm, m->d_z[3], m->d_t, m->d_d, m->d_part);
-  LAUNCH_CHECK("k_mse_grad");
-  const float* d = m->d_d;  // dL/dz of the current layer, [n][out]
-  for (int l = 3; l >= 0; --l) {
-    const float* xin = l == 0 ? m->d_x : m->d_a[l - 1];
-    // dW[o][i] = sum_b d[b][o] xin[b][i]
-    gemm<0>(m, kOut[l], kIn[l], n, d, 1, kOut[l], xin, kIn[l], 1, m->d_g + kW[l], kIn[l]);
-    hipLaunchKernelGGL(k_colsum, dim3(kOut[l]), dim3(256), 0, m->stream, n, kOut[l], d, m->d_g + kB[l]);
-    LAUNCH_CHECK("k_colsum");
-    if (l > 0) {
-      float* dn = m->d_e[l & 1];
-      // dxin[b][i] = sum_o d[b][o] W[o][i], times gelu'(z[l-1][b][i])
-      gemm<2>(m, n, kIn[l], kOut[l], d, kOut[l], 1, m->d_p + kW[l], kIn[l], 1, dn, kIn[l], nullptr, nullptr,
-              m->d_z[l - 1]);
-      d = dn;
-    }
-  }
-  std::vector<double> part(blocks);
-  mchk(hipMemcpyAsync(part.data(), m->d_part, sizeof(double) * blocks, hipMemcpyDeviceToHost, m->stream), "copy");
-  mchk(hipStreamSynchronize(m->stream), "sync");
+// the loss of the last gradient32 of n points (waits for it)
+double last_loss(chan_mlp* m, int n) {
   double s = 0.0;
-  for (double v : part) s += v;
-  return s / (double)nm;
+  mchk(hipMemcpyAsync(&s, m->d_lpart + MLP_MAXWG, sizeof(double), hipMemcpyDeviceToHost, m->stream), "copy");
+  mchk(hipStreamSynchronize(m->stream), "sync");
+  return s / (double)(6L * n);
 }
 
 void pack(chan_mlp* m) {
@@ -566,10 +728,7 @@ int chan_mlp_destroy(chan_mlp* m) {
   if (!m) return 0;
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   mfree(m->d_p); mfree(m->d_g); mfree(m->d_m); mfree(m->d_v); mfree(m->d_packed);
-  mfree(m->d_x); mfree(m->d_y); mfree(m->d_t); mfree(m->d_d); mfree(m->d_part);
-  for (auto& z : m->d_z) mfree(z);
-  for (auto& a : m->d_a) mfree(a);
-  for (auto& e : m->d_e) mfree(e);
+  mfree(m->d_x); mfree(m->d_y); mfree(m->d_t); mfree(m->d_part); mfree(m->d_lpart);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
   return 0;
@@ -619,8 +778,10 @@ int chan_mlp_forward_fp32(chan_mlp* m, int n, const float* x, float* y) {
     if (n < 1 || !x || !y) throw chan_error("invalid arguments");
     ensure_cap(m, n);
     mchk(hipMemcpyAsync(m->d_x, x, sizeof(float) * 10 * n, hipMemcpyHostToDevice, m->stream), "copy");
-    forward32(m, n);
-    mchk(hipMemcpyAsync(y, m->d_z[3], sizeof(float) * 6 * n, hipMemcpyDeviceToHost, m->stream), "copy");
+    hipLaunchKernelGGL((k_mlp_grad<false>), dim3(tile_blocks(n)), dim3(512), sizeof(MlpLds), m->stream, m->d_p, n,
+                       m->d_x, nullptr, m->d_y, 0.0f, nullptr, nullptr);
+    LAUNCH_CHECK("k_mlp_grad");
+    mchk(hipMemcpyAsync(y, m->d_y, sizeof(float) * 6 * n, hipMemcpyDeviceToHost, m->stream), "copy");
     mchk(hipStreamSynchronize(m->stream), "sync");
   });
 }
@@ -629,13 +790,13 @@ int chan_mlp_gradient(chan_mlp* m, int n, const float* x, const float* t, float*
   return mguard(m, [&] {
     if (n < 1 || !x || !t) throw chan_error("invalid arguments");
     ensure_cap(m, n);
+    ensure_partials(m);
     mchk(hipMemcpyAsync(m->d_x, x, sizeof(float) * 10 * n, hipMemcpyHostToDevice, m->stream), "copy");
     mchk(hipMemcpyAsync(m->d_t, t, sizeof(float) * 6 * n, hipMemcpyHostToDevice, m->stream), "copy");
-    const double l = gradient32(m, n);
-    if (grad) {
+    gradient32(m, n, m->d_x, m->d_t, 0, 0.0f);
+    if (grad)
       mchk(hipMemcpyAsync(grad, m->d_g, sizeof(float) * MLP_NPARAM, hipMemcpyDeviceToHost, m->stream), "copy");
-      mchk(hipStreamSynchronize(m->stream), "sync");
-    }
+    const double l = last_loss(m, n);
     if (loss) *loss = l;
   });
 }
@@ -648,37 +809,17 @@ int chan_mlp_train(chan_mlp* m, int n, const float* x, const float* t, int epoch
   return mguard(m, [&] {
     if (n < 1 || !x || !t || epochs < 1 || batch < 1 || batch > n) throw chan_error("invalid arguments");
     ensure_cap(m, n);
-    float *dx_all = nullptr, *dt_all = nullptr;
-    mchk(hipMalloc(&dx_all, sizeof(float) * 10 * n), "hipMalloc");
-    mchk(hipMalloc(&dt_all, sizeof(float) * 6 * n), "hipMalloc");
-    double l = 0.0;
-    try {
-      mchk(hipMemcpyAsync(dx_all, x, sizeof(float) * 10 * n, hipMemcpyHostToDevice, m->stream), "copy");
-      mchk(hipMemcpyAsync(dt_all, t, sizeof(float) * 6 * n, hipMemcpyHostToDevice, m->stream), "copy");
-      const int nb = n / batch;
-      for (int e = 0; e < epochs; ++e)
-        for (int bi = 0; bi < nb; ++bi) {
-          mchk(hipMemcpyAsync(m->d_x, dx_all + (long)bi * batch * 10, sizeof(float) * 10 * batch,
-                              hipMemcpyDeviceToDevice, m->stream), "copy");
-          mchk(hipMemcpyAsync(m->d_t, dt_all + (long)bi * batch * 6, sizeof(float) * 6 * batch,
-                              hipMemcpyDeviceToDevice, m->stream), "copy");
-          l = gradient32(m, batch);
-          m->adam_t += 1;
-          const float b1 = 0.9f, b2 = 0.999f;
-          const float c1 = 1.0f - std::pow(b1, (float)m->adam_t), c2 = 1.0f - std::pow(b2, (float)m->adam_t);
-          hipLaunchKernelGGL(k_adam, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, m->stream, MLP_NPARAM, m->d_p,
-                             m->d_g, m->d_m, m->d_v, (float)lr, b1, b2, 1e-8f, c1, c2);
-          LAUNCH_CHECK("k_adam");
-        }
-      mchk(hipStreamSynchronize(m->stream), "sync");
-    } catch (...) {
-      (void)hipFree(dx_all);
-      (void)hipFree(dt_all);
-      throw;
-    }
-    (void)hipFree(dx_all);
-    (void)hipFree(dt_all);
+    ensure_partials(m);
+    mchk(hipMemcpyAsync(m->d_x, x, sizeof(float) * 10 * n, hipMemcpyHostToDevice, m->stream), "copy");
+    mchk(hipMemcpyAsync(m->d_t, t, sizeof(float) * 6 * n, hipMemcpyHostToDevice, m->stream), "copy");
     m->packed_ok = false;
+    const int nb = n / batch;
+    for (int e = 0; e < epochs; ++e)
+      for (int bi = 0; bi < nb; ++bi) {
+        m->adam_t += 1;
+        gradient32(m, batch, m->d_x + (long)bi * batch * 10, m->d_t + (long)bi * batch * 6, m->adam_t, (float)lr);
+      }
+    const double l = last_loss(m, batch);
     if (loss_out) *loss_out = l;
   });
 }
