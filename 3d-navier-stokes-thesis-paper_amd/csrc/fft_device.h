@@ -160,16 +160,26 @@ __device__ void fft_batch(double2* lds, int sstride, int B, const FFTPlan& pl,
 // ---------------------------------------------------------------------------
 // Two-pass (four-step) FFT with a compile-time length N = N1 * N2.
 //
-// A sequence is held in LDS as an N1 x N2 array with row stride N2 + 1.
+// A sequence is held in LDS as an N1 x N2 array with row stride N2 | 1.
 // Input x[n], n = a*N2 + b, sits at row a, column b.  Pass 1 transforms each
 // column b over a (length N1, in registers) and multiplies by w_N^{b*k1};
 // pass 2 transforms each row k1 over b (length N2).  Both passes read and
 // write the same LDS cells, so the transform is in place with one barrier
 // between the passes.  The result X[k], k = k1 + N1*k2, ends at row k1,
-// column k2 (fft2_out_pos).  With N2 even the odd row stride keeps the
-// 16-byte row-wise accesses of pass 2 free of bank conflicts.
+// column k2 (fft2_out_pos).  The odd row stride keeps the 16-byte row-wise
+// accesses of pass 2 free of bank conflicts.
 //
-// The in-register DFTs of length L (4, 6, 8, 9, 12, 16, 18, 24) are built the
+// The lengths are 2^a 3^b with both factors short enough for a register DFT:
+// 2^a and 3 * 2^a, and the ones with two or more factors of 3 that 3/2
+// dealiasing of the grid sizes 24, 36, 54, 72, 108, 144 and 162 makes (and
+// the sizes themselves, which the undealiased transforms take).  The
+// runtime-planned transform these ran before makes one LDS round trip and
+// barrier per radix-2/3/4/8 stage and computes its indices by division:
+// a step at 72x81x108 took 893 us with it and takes 362, 144x65x162
+// 2609 and 726, 36x65x36 535 and 138; 288x65x36 (nx2/2 = 216, whose
+// workgroup x-pass spills a few registers) 1532 and 554.
+//
+// The in-register DFTs of length L (3, 4, 6, 8, 9, 12, 16, 18, 27) are built the
 // same way from the radix-2/3/4/8 kernels above; their twiddles w_L^e are read
 // from the length-N root table at the compile-time index e*N/L (uniform
 // scalar loads).
@@ -179,24 +189,40 @@ struct Fft2Split { int n1, n2; };
 __host__ __device__ constexpr Fft2Split fft2_split(int n) {
   switch (n) {
     case 16: return {4, 4};
+    case 18: return {3, 6};
     case 24: return {4, 6};
+    case 27: return {3, 9};
     case 32: return {4, 8};
     case 36: return {6, 6};
     case 48: return {6, 8};
+    case 54: return {6, 9};
     case 64: return {8, 8};
     case 72: return {9, 8};
+    case 81: return {9, 9};
     case 96: return {8, 12};
+    case 108: return {12, 9};
+    case 128: return {8, 16};
     case 144: return {12, 12};
+    case 162: return {18, 9};
     case 192: return {12, 16};
+    case 216: return {12, 18};
+    case 243: return {9, 27};
     case 288: return {18, 16};
     default: return {0, 0};
   }
 }
 
-// LDS cells one sequence occupies: N1*(N2+1) for a compile-time length, n+1
-// for the runtime-planned transform.
+// Row stride of the two-pass layout, and the LDS cells one sequence occupies:
+// N1 rows for a compile-time length, n+1 cells for the runtime-planned transform.
+__host__ __device__ constexpr int fft2_rs(int n) { return fft2_split(n).n2 | 1; }
 __host__ __device__ constexpr int fft_seq_cells(int n) {
-  return fft2_split(n).n1 ? fft2_split(n).n1 * (fft2_split(n).n2 + 1) : n + 1;
+  return fft2_split(n).n1 ? fft2_split(n).n1 * fft2_rs(n) : n + 1;
+}
+
+// Lengths the batched ensemble's launches and the closure's x-pass are built
+// for: powers of two times 1, 3 or 9 up to 9 * 32.
+__host__ __device__ constexpr bool fft2_batched(int n) {
+  return fft2_split(n).n1 > 0 && n % 27 != 0 && n != 18 && n != 128;
 }
 
 __host__ __device__ constexpr int rdft_first(int L) {
@@ -248,18 +274,18 @@ __device__ __forceinline__ void rdft(double2* v, const double2* __restrict__ rt)
 template <int N>
 __device__ __forceinline__ int fft2_in_pos(int n) {
   constexpr int N2 = fft2_split(N).n2;
-  return n + n / N2;
+  return n + (fft2_rs(N) - N2) * (n / N2);
 }
 template <int N>
 __device__ __forceinline__ int fft2_out_pos(int k) {
-  constexpr int N1 = fft2_split(N).n1, N2 = fft2_split(N).n2;
-  return (k % N1) * (N2 + 1) + k / N1;
+  constexpr int N1 = fft2_split(N).n1;
+  return (k % N1) * fft2_rs(N) + k / N1;
 }
 
 // The two passes of the two-pass FFT for one task each.
 template <int N, int SGN>
 __device__ __forceinline__ void fft2_pass1(double2* seq, int b, const double2* rl, const double2* __restrict__ rg) {
-  constexpr int N1 = fft2_split(N).n1, N2 = fft2_split(N).n2, RS = N2 + 1;
+  constexpr int N1 = fft2_split(N).n1, N2 = fft2_split(N).n2, RS = fft2_rs(N);
   double2* p = seq + b;
   double2 v[N1];
 #pragma unroll
@@ -277,7 +303,7 @@ __device__ __forceinline__ void fft2_pass1(double2* seq, int b, const double2* r
 
 template <int N, int SGN>
 __device__ __forceinline__ void fft2_pass2(double2* seq, int k1, const double2* __restrict__ rg) {
-  constexpr int N1 = fft2_split(N).n1, N2 = fft2_split(N).n2, RS = N2 + 1;
+  constexpr int N1 = fft2_split(N).n1, N2 = fft2_split(N).n2, RS = fft2_rs(N);
   double2* p = seq + k1 * RS;
   double2 v[N2];
 #pragma unroll
@@ -316,7 +342,7 @@ __device__ __forceinline__ void fft2p(double2* lds, int sstride, int B, const do
 // beyond the table's), which leaves the workgroup's LDS to the data alone.
 template <int N, int SGN>
 __device__ __forceinline__ void fft2_pass1_rec(double2* seq, int b, const double2* __restrict__ rg) {
-  constexpr int N1 = fft2_split(N).n1, N2 = fft2_split(N).n2, RS = N2 + 1;
+  constexpr int N1 = fft2_split(N).n1, N2 = fft2_split(N).n2, RS = fft2_rs(N);
   double2* p = seq + b;
   const double2 wt = rg[b];
   double2 v[N1];
@@ -439,15 +465,24 @@ __device__ __forceinline__ void load_tw2(double2* dst, const double2* __restrict
 #define FFT_DISPATCH(n, F)        \
   switch (n) {                    \
     case 16: F(16); break;        \
+    case 18: F(18); break;        \
     case 24: F(24); break;        \
+    case 27: F(27); break;        \
     case 32: F(32); break;        \
     case 36: F(36); break;        \
     case 48: F(48); break;        \
+    case 54: F(54); break;        \
     case 64: F(64); break;        \
     case 72: F(72); break;        \
+    case 81: F(81); break;        \
     case 96: F(96); break;        \
+    case 108: F(108); break;      \
+    case 128: F(128); break;      \
     case 144: F(144); break;      \
+    case 162: F(162); break;      \
     case 192: F(192); break;      \
+    case 216: F(216); break;      \
+    case 243: F(243); break;      \
     case 288: F(288); break;      \
     default: F(0); break;         \
   }

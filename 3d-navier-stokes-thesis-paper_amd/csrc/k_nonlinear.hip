@@ -687,7 +687,7 @@ static bool xpass_rw_built(int M, int rw, bool pf) {
 int xpass_rows(int M, int nz2, int req, bool pf, bool batched) {
   auto ok = [&](int r) { return xpass_rw_built(M, r, pf) && nz2 % r == 0; };
   if (req > 0 && ok(req)) return req;
-  const int d = (M <= 24 || (batched && M <= 72)) ? 2 : 1;
+  const int d = (M <= 27 || (batched && M <= 72)) ? 2 : 1;
   return ok(d) ? d : 1;
 }
 
@@ -701,7 +701,9 @@ size_t xpass_w_lds(int M, int rw, int nxh, bool pf) {
 
 template <int N, bool PF, int RW>
 static XPassFn xpass_w_variant(bool les, bool lin) {
-  if (les) return k_xpass_w<false, N, PF, true, RW>;
+  if constexpr (fft2_batched(N)) {
+    if (les) return k_xpass_w<false, N, PF, true, RW>;
+  }
   return lin ? (XPassFn)k_xpass_w<true, N, PF, false, RW> : (XPassFn)k_xpass_w<false, N, PF, false, RW>;
 }
 
@@ -741,7 +743,7 @@ static XPassBFn xpass_wb_fn(bool lin, int rw) {
 static XPassBFn xpass_wb_pick(int M, bool lin, int rw) {
   XPassBFn fn = nullptr;
 #define XPASSB_CASE(N)                                   \
-  if constexpr (N > 0 && N <= 192) fn = xpass_wb_fn<N>(lin, rw);
+  if constexpr (fft2_batched(N) && N <= 192) fn = xpass_wb_fn<N>(lin, rw);
   FFT_DISPATCH(M, XPASSB_CASE)
 #undef XPASSB_CASE
   if (!fn) throw chan_error("batched x-pass: no wavefront kernel for nx2/2 = " + std::to_string(M) + " with " +
@@ -753,7 +755,7 @@ static XPassBFn xpass_wb_pick(int M, bool lin, int rw) {
 // launch (the batched ensemble); the row prefetch is on wherever the single
 // launch uses it (M <= 144).  rw: rows per wavefront (every member's nz2 a
 // multiple of it); nxh: the largest nx/2+1 of the members.
-bool xpass_batchable(int M) { return fft2_split(M).n1 > 0 && M <= 192; }
+bool xpass_batchable(int M) { return fft2_batched(M) && M <= 192; }
 
 void launch_xpass_batched(int M, bool lin, int rw, int nxh, const XBatchArgs* args, const BatchItem* items,
                           int nitems, hipStream_t s) {
@@ -810,7 +812,7 @@ void launch_xpass(const XZGeom& g, const double2* tw, const DevOps& ops, const X
       if (((nbf + nthr - 1) / nthr) * R > 12) throw chan_error("x-pass FFT staging bound");
     }
   const int nplanes = a.kb - a.ka + 1;
-  if (a.tau && !(a.wave && ct && M <= 192))
+  if (a.tau && !(a.wave && fft2_batched(M) && M <= 192))
     throw chan_error("the subgrid closure needs the wavefront x-pass (nx2/2 <= 192 of the form 2^a 3^b)");
   if (a.wave && ct && M <= 192) {
     const bool pf = a.prefetch && M <= 144;

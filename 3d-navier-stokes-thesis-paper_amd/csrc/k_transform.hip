@@ -55,7 +55,8 @@ __device__ __forceinline__ double2 pad_apply(double2 v, const PadSrc& p, bool va
 // for ss = 2 (mod 8) (ss = 306 at nz2 = 288), where the 8 columns of one row
 // meet in pairs (measured: LDS bank-conflict cycles of the z-forward 3.6e7 ->
 // 1.6e7 per step); every 16 lanes still read two whole 128-byte rows of the
-// [z][kx] array.  Needs an even row count.
+// [z][kx] array.  A length-nz2 column with nz2 odd has one row more than it
+// needs in the last group: the caller masks t = nz2.
 __device__ __forceinline__ void tile8_ts(int e, int& t, int& s) {
   const int r = e & 15;
   t = 2 * (e >> 4) + ((r >> 2) & 1);
@@ -387,7 +388,8 @@ __device__ __forceinline__ void zfwd2_body(const XZGeom& g, const double2* __res
   extern __shared__ double2 lds[];
   constexpr int NZ2 = NC, SS = fft_seq_cells(NC);
   constexpr int NT = 32 * KX;
-  constexpr int NLD = (NZ2 * KX + NT - 1) / NT;       // loads per thread per field
+  constexpr int NE = KX == 8 ? (NZ2 + 1) / 2 * 16 : NZ2 * KX;   // elements in whole row pairs (tile8_ts)
+  constexpr int NLD = (NE + NT - 1) / NT;             // loads per thread per field
   const int tid = threadIdx.x;
   const int kx0 = bx * KX;
   const long P = map_plane(pm, by);
@@ -417,7 +419,7 @@ __device__ __forceinline__ void zfwd2_body(const XZGeom& g, const double2* __res
     const int e = tid + NT * k;
     int t = e / KX, s = e - t * KX;
     if constexpr (KX == 8) tile8_ts(e, t, s);
-    const bool ok = e < NZ2 * KX && s < ncol;
+    const bool ok = t < NZ2 && s < ncol;
     const long o = (long)(t < NZ2 ? t : NZ2 - 1) * g.kxpad + kx0 + (s < ncol ? s : ncol - 1);
     const double2 a = Ap[o], b = Bp[o];
     ra[k] = ok ? a : make_double2(0.0, 0.0);
@@ -430,7 +432,7 @@ __device__ __forceinline__ void zfwd2_body(const XZGeom& g, const double2* __res
     const int e = tid + NT * k;
     int t = e / KX, s = e - t * KX;
     if constexpr (KX == 8) tile8_ts(e, t, s);
-    if (e < NZ2 * KX) lds[s * SS + fft2_in_pos<NC>(t)] = ra[k];
+    if (t < NZ2) lds[s * SS + fft2_in_pos<NC>(t)] = ra[k];
   }
   __syncthreads();
   fft2p<NC, -1>(lds, SS, ncol, rl, tw + g.pz.tw, tid, NT);  // the valid columns only
@@ -459,7 +461,7 @@ __device__ __forceinline__ void zfwd2_body(const XZGeom& g, const double2* __res
     const int e = tid + NT * k;
     int t = e / KX, s = e - t * KX;
     if constexpr (KX == 8) tile8_ts(e, t, s);
-    if (e < NZ2 * KX) lds[s * SS + fft2_in_pos<NC>(t)] = rb[k];
+    if (t < NZ2) lds[s * SS + fft2_in_pos<NC>(t)] = rb[k];
   }
   __syncthreads();
   fft2p<NC, -1>(lds, SS, ncol, rl, tw + g.pz.tw, tid, NT);  // the valid columns only
@@ -510,11 +512,11 @@ void launch_zinv(const XZGeom& g, const double2* tw, const double2* in, long in_
                  long out_ps, int nplanes, hipStream_t s, int kx, int pcnt, int pstride, int poff) {
   const PlaneMap pm = pcnt > 0 ? PlaneMap{pcnt, pstride, poff} : PlaneMap{nplanes, 0, 0};
   const bool ct = fft2_split(g.nz2).n1 > 0;
-  if (ct && (kx == 4 || kx == 16)) {
+  if (fft2_batched(g.nz2) && (kx == 4 || kx == 16)) {
     dim3 gk((g.nxh + kx - 1) / kx, nplanes);
     const size_t lk = sizeof(double2) * (kx * fft_seq_cells(g.nz2) + g.nz2);
 #define ZINV2_CASE(N)                                                                                      \
-  if constexpr (N > 0) {                                                                                   \
+  if constexpr (fft2_batched(N)) {                                                                                   \
     if (kx == 4) hipLaunchKernelGGL((k_zinv2<N, 4>), gk, dim3(128), lk, s, g, tw, in, in_ps, out, out_ps, pm); \
     else hipLaunchKernelGGL((k_zinv2<N, 16>), gk, dim3(512), lk, s, g, tw, in, in_ps, out, out_ps, pm);         \
   }
@@ -535,16 +537,16 @@ void launch_zinv(const XZGeom& g, const double2* tw, const double2* in, long in_
 }
 
 // Batched z-transforms: one launch runs the work lists of several channels
-// of the same transform length (the batched ensemble).  Only the
-// compile-time two-pass lengths are batched.
-bool zt_batchable(int nz2) { return fft2_split(nz2).n1 > 0; }
+// of the same transform length (the batched ensemble), at the lengths
+// fft2_batched names.
+bool zt_batchable(int nz2) { return fft2_batched(nz2); }
 
 void launch_zinv_batched(int nz2, const ZBatchArgs* args, const BatchItem* items, int nitems, hipStream_t s) {
   if (nitems <= 0) return;
   if (!zt_batchable(nz2)) throw chan_error("batched z-inverse: length " + std::to_string(nz2) + " has no compile-time plan");
   const size_t lds = sizeof(double2) * ZT_KX * fft_seq_cells(nz2);
 #define ZINVB_CASE(N) \
-  if constexpr (N > 0) hipLaunchKernelGGL(k_zinv_b<N>, dim3(nitems), dim3(256), lds, s, args, items)
+  if constexpr (fft2_batched(N)) hipLaunchKernelGGL(k_zinv_b<N>, dim3(nitems), dim3(256), lds, s, args, items)
   FFT_DISPATCH(nz2, ZINVB_CASE)
 #undef ZINVB_CASE
   LAUNCH_CHECK("k_zinv_b");
@@ -555,7 +557,7 @@ void launch_zfwd_batched(int nz2, const ZBatchArgs* args, const BatchItem* items
   if (!zt_batchable(nz2)) throw chan_error("batched z-forward: length " + std::to_string(nz2) + " has no compile-time plan");
   const size_t lds = sizeof(double2) * (8 * fft_seq_cells(nz2) + nz2);
 #define ZFWDB_CASE(N) \
-  if constexpr (N > 0) hipLaunchKernelGGL((k_zfwd2_b<N, 8>), dim3(nitems), dim3(256), lds, s, args, items)
+  if constexpr (fft2_batched(N)) hipLaunchKernelGGL((k_zfwd2_b<N, 8>), dim3(nitems), dim3(256), lds, s, args, items)
   FFT_DISPATCH(nz2, ZFWDB_CASE)
 #undef ZFWDB_CASE
   LAUNCH_CHECK("k_zfwd2_b");
@@ -614,16 +616,16 @@ void launch_zfwd(const XZGeom& g, const double2* tw, const double2* A, const dou
   const int nthr = 256 * nf;
   const bool ct = fft2_split(g.nz2).n1 > 0;
   if (v2 && ct && B && !g.small && g.nz <= 192) {
-    const int k2 = (kx == 4) ? 4 : 8;
+    const int k2 = (kx == 4 && fft2_batched(g.nz2)) ? 4 : 8;
     dim3 g2((g.nxh + k2 - 1) / k2, nplanes);
     size_t l2 = sizeof(double2) * (k2 * fft_seq_cells(g.nz2) + g.nz2);
 #define ZFWD2_CASE(N)                                                                                       \
-  if constexpr (N > 0) {                                                                                    \
+  if constexpr (fft2_batched(N))                                                                            \
     if (k2 == 4) hipLaunchKernelGGL((k_zfwd2<N, 4>), g2, dim3(128), l2, s, g, tw, A, B, ab_ps, kz, out, out_ps, \
                                     nl_zero_ny, pm);                                                        \
-    else hipLaunchKernelGGL((k_zfwd2<N, 8>), g2, dim3(256), l2, s, g, tw, A, B, ab_ps, kz, out, out_ps,       \
-                            nl_zero_ny, pm);                                                                \
-  }
+  if constexpr (N > 0)                                                                                      \
+    if (k2 == 8) hipLaunchKernelGGL((k_zfwd2<N, 8>), g2, dim3(256), l2, s, g, tw, A, B, ab_ps, kz, out, out_ps, \
+                                    nl_zero_ny, pm)
     FFT_DISPATCH(g.nz2, ZFWD2_CASE)
 #undef ZFWD2_CASE
     LAUNCH_CHECK("k_zfwd2");
