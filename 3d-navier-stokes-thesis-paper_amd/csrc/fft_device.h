@@ -30,6 +30,23 @@ __device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_doub
 __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
+// Half-length packing of a real transform: (a + b) + i w (a - b), and its
+// inverse (a + b) - i w (a - b); x + i k y.  Written as explicit fused
+// multiply-adds so that every kernel (and every inlined copy of one) rounds
+// alike, wherever the compiler places the stores that follow.
+__device__ __forceinline__ double2 c2r_combine(double2 a, double2 b, double2 w) {
+  const double2 s = cadd(a, b), d = csub(a, b);
+  return make_double2(__builtin_fma(-w.x, d.y, __builtin_fma(-w.y, d.x, s.x)),
+                      __builtin_fma(w.x, d.x, __builtin_fma(-w.y, d.y, s.y)));
+}
+__device__ __forceinline__ double2 r2c_combine(double2 a, double2 b, double2 w) {
+  const double2 s = cadd(a, b), d = csub(a, b);
+  return make_double2(__builtin_fma(w.x, d.y, __builtin_fma(w.y, d.x, s.x)),
+                      __builtin_fma(-w.x, d.x, __builtin_fma(w.y, d.y, s.y)));
+}
+__device__ __forceinline__ double2 add_ik(double2 x, double k, double2 y) {
+  return make_double2(__builtin_fma(-k, y.y, x.x), __builtin_fma(k, y.x, x.y));
+}
 __device__ __forceinline__ double2 cconj(double2 a) { return make_double2(a.x, -a.y); }
 __device__ __forceinline__ double2 cscale(double s, double2 a) { return make_double2(s * a.x, s * a.y); }
 // multiply by +i (s=+1) or -i (s=-1)

@@ -18,6 +18,7 @@
 //   4. combines A = F(fy) + i kx F(fx) and B = F(fz) for each component
 //      (PFC/transform.f90:613) and writes them for the z-forward pass.
 // At rk_step == 1 it also accumulates the per-plane CFL maxima (:202-217).
+#include <type_traits>
 #include "chan_internal.h"
 
 __device__ __forceinline__ double2 c2r_pack_nl(const double2* __restrict__ row, int nxh, int M,
@@ -26,18 +27,16 @@ __device__ __forceinline__ double2 c2r_pack_nl(const double2* __restrict__ row, 
   if (n < nxh) { a = row[n]; if (n == 0 || n == M) a.y = 0.0; }
   int m = M - n;
   if (m < nxh) { b = row[m]; if (m == 0 || m == M) b.y = 0.0; b.y = -b.y; }
-  double2 s = cadd(a, b), d = csub(a, b);
-  double2 wd = cmul(wconj, d);
-  return make_double2(s.x - wd.y, s.y + wd.x);
+  return c2r_combine(a, b, wconj);
 }
 
+// Twice the real transform's coefficient k from the half-length transform
+// (Z_k + conj Z_{M-k}) - i w^k (Z_k - conj Z_{M-k}); the z-forward pass halves
+// it with its own scale.
 template <int MC>
 __device__ __forceinline__ double2 r2c_post_nl(const double2* __restrict__ Zs, int M, int k, double2 wk) {
-  double2 a = Zs[fft_out_pos<MC>(k % M)], b = cconj(Zs[fft_out_pos<MC>((M - k) % M)]);
-  double2 E = make_double2(0.5 * (a.x + b.x), 0.5 * (a.y + b.y));
-  double2 d = csub(a, b);
-  double2 O = make_double2(0.5 * d.y, -0.5 * d.x);
-  return cadd(E, cmul(wk, O));
+  const double2 a = Zs[fft_out_pos<MC>(k % M)], b = cconj(Zs[fft_out_pos<MC>((M - k) % M)]);
+  return r2c_combine(a, b, wk);
 }
 
 // elementwise helpers on the pair of points (x = 2n, 2n+1)
@@ -273,7 +272,17 @@ __global__ __launch_bounds__(640) void k_xpass(XZGeom g, const double2* __restri
 // writes cells base + i) as soon as the current rows have been consumed, so
 // their latency overlaps a whole plane of work instead of stalling the
 // wavefront at the start of every plane.  A raw row takes nxh cells (M + 1
-// with one row per wavefront) rounded up to 64.
+// with one row per wavefront, or below 64 pairs) rounded up to 64.
+//
+// What bounds it: LDS round trips and vector issue in turn (M = 144: two
+// wavefronts per SIMD, a forward transform phase of 2900 cycles of which
+// 1280 issue vector instructions; LDS 48 % busy), so the steps are laid out
+// for few waits: lanes without work run along and only their stores are
+// masked, which lets every load of a step issue before the first wait, and
+// the wait for the next raw rows leaves the stores behind them in flight.
+// x-pass at 256x193x192 (M = 192, rows read in place): 796 us with a branch
+// per cell and one wavefront per SIMD, 442 now; 32x65x32 16.6 and 14.8.
+//
 // (bx, by): the workgroup's group of 4*RW z-rows and its plane range
 // (blockIdx, or a work-list entry of the batched form)
 template <bool LIN, int M, bool PF, bool LES = false, int RW = 1>
@@ -286,9 +295,9 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
   // offsets on the scalar unit
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nz2 = g.nz2, kxp = g.kxpad, nxh = g.nxh;
-  // one row per wavefront keeps the raw-row stride a constant (M + 1 cells
-  // rounded up), so the LDS offsets of its three raw rows fold into the reads
-  const int rawn = RW == 1 ? xpass_raw_cells(M + 1) : xpass_raw_cells(nxh);
+  // a constant raw-row stride (M + 1 cells rounded up) where it costs no LDS, so that the
+  // LDS offsets of the raw rows fold into the reads
+  const int rawn = (RW == 1 || M < 64) ? xpass_raw_cells(M + 1) : xpass_raw_cells(nxh);
   double2* rl = lds;
   load_tw2<M>(rl, tw + g.px.tw, tid, 256);
   __syncthreads();
@@ -305,7 +314,9 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
   const bool hasbuf = ops.buffer != nullptr;
 
   // pair q of the lane: point nq[q] of row rq(q); pin/pout carry the row's
-  // sequence offset
+  // sequence offset.  A lane past the last pair works on point 0 of row 0 and
+  // its values are not stored: everything but the stores runs without a
+  // branch, so that the loads of a step are all issued before the first wait.
   int nq[PPL], pin[PPL], pout[PPL];
   bool vq[PPL];
   double2 wc[PPL];
@@ -313,11 +324,11 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
 #pragma unroll
   for (int q = 0; q < PPL; ++q) {
     const int v = lane + 64 * q;
-    vq[q] = v < NP;
+    vq[q] = 64 * (q + 1) <= NP || v < NP;
     const int vv = vq[q] ? v : 0;
     const int r = RW == 1 ? 0 : vv / M, n = vv - r * M;
     nq[q] = n;
-    wc[q] = cconj(rootx[n]);
+    wc[q] = cconj(rootx[RW == 1 ? min(v, M) : n]);   // one row: also the root of output column v <= M
     pin[q] = r * SEQ + fft2_in_pos<M>(n);
     pout[q] = r * SEQ + fft2_out_pos<M>(n);
   }
@@ -332,7 +343,9 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
 #pragma unroll
         for (int r = 0; r < RW; ++r) {
           const double2* row = a.Z + ((long)(c * nyp + (p - 1)) * nz2 + r) * kxp + rowoff;
-          for (int i = 0; 64 * i < nxh; ++i) {
+#pragma unroll
+          for (int i = 0; i < (M + 64) / 64; ++i) {   // nxh <= M + 1
+            if (64 * i >= nxh) break;
             const int idx = min(64 * i + lane, nxh - 1);
             __builtin_amdgcn_global_load_lds((const void*)(row + idx),
                                              (__attribute__((address_space(3))) void*)(RAW + (c * RW + r) * rawn + 64 * i),
@@ -342,31 +355,61 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
       }
     }
   };
-  auto ready = [&]() {
+  // The raw rows have landed.  Vector memory operations complete in the order
+  // they were issued, so the `later` stores issued since the fetch need not
+  // have: waiting for them too would add their latency to every plane.
+  auto ready = [&](int later) {
     if constexpr (PF) {
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the raw rows have landed
+      switch (later) {
+        case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
+        case 12: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
+        case 18: asm volatile("s_waitcnt vmcnt(18)" ::: "memory"); break;
+        default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
+      }
       wave_sync();
     }
   };
-  // c2r of plane p (1-based) into U, V, Wv at the owned points
-  auto c2r_plane = [&](int p, double2* U, double2* V, double2* Wv, bool needv) {
+  // c2r of plane p (1-based) into U, V, Wv at the owned points; the raw rows
+  // of plane pnext (0: none) are fetched as soon as those of p are in registers.
+  // The half-length packing (c2r_pack_nl) with the cells of both modes clamped
+  // into the row and their parts zeroed by selects.
+  auto c2r_plane = [&](int p, double2* U, double2* V, double2* Wv, int pnext) {
+    constexpr int CB = RW == 1 ? 3 : 1;   // components whose cells are in flight together
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
+    for (int c0 = 0; c0 < 3; c0 += CB) {
+      double2 ya[CB][PPL], yb[CB][PPL];
+#pragma unroll
+      for (int c = 0; c < CB; ++c) {
+#pragma unroll
+        for (int q = 0; q < PPL; ++q) {
+          const double2* row = PF ? RAW + ((c0 + c) * RW + rq(q)) * rawn
+                                  : a.Z + ((long)((c0 + c) * nyp + (p - 1)) * nz2 + rq(q)) * kxp + rowoff;
+          ya[c][q] = row[min(nq[q], nxh - 1)];
+          yb[c][q] = row[min(M - nq[q], nxh - 1)];
+        }
+      }
+      if (c0 + CB == 3 && pnext) fetch(pnext);
 #pragma unroll
       for (int q = 0; q < PPL; ++q) {
-        if (!vq[q]) continue;
-        const double2* row = PF ? RAW + (c * RW + rq(q)) * rawn
-                                : a.Z + ((long)(c * nyp + (p - 1)) * nz2 + rq(q)) * kxp + rowoff;
-        double2 v = make_double2(0.0, 0.0);
-        if (c != 1 || needv) v = c2r_pack_nl(row, nxh, M, nq[q], wc[q]);
-        W[c * FS + pin[q]] = v;
+        const int n = nq[q];
+        const bool ha = n < nxh, hb = M - n < nxh, im = n != 0;
+        double2 z[CB];
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+          const double2 A = make_double2(ha ? ya[c][q].x : 0.0, ha && im ? ya[c][q].y : 0.0);
+          const double2 B = make_double2(hb ? yb[c][q].x : 0.0, hb && im ? -yb[c][q].y : 0.0);
+          z[c] = c2r_combine(A, B, wc[q]);
+        }
+        if (vq[q]) {
+#pragma unroll
+          for (int c = 0; c < CB; ++c) W[(c0 + c) * FS + pin[q]] = z[c];
+        }
       }
     }
     wave_sync();
     fft2p_wave<M, 1>(W, SEQ, 3 * RW, rl, rg, lane);
 #pragma unroll
     for (int q = 0; q < PPL; ++q) {
-      if (!vq[q]) continue;
       U[q] = W[0 * FS + pout[q]];
       V[q] = W[1 * FS + pout[q]];
       Wv[q] = W[2 * FS + pout[q]];
@@ -381,7 +424,6 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
     const long cs = (long)nyp * nz2 * g.nx2;
 #pragma unroll
     for (int q = 0; q < PPL; ++q) {
-      if (!vq[q]) continue;
       const long o = (long)(p - 1) * nz2 * g.nx2 + poff(q);
       U[q] = *reinterpret_cast<const double2*>(b + o);
       V[q] = *reinterpret_cast<const double2*>(b + cs + o);
@@ -393,11 +435,13 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
   // would make its consumer wait for the in-flight prefetch as well.
   // The output columns of the rows: output u = lane + 64i is column
   // u mod nxh of row u / nxh.  The columns of the first KP iterations (all of
-  // them with 3/2 dealiasing, nxh = 2M/3 + 1) have their root and wavenumber
-  // in registers; wider rows load the rest in place.
+  // them with 3/2 dealiasing, nxh = 2M/3 + 1) have their root (with one row,
+  // that of the pair with the same index) and wavenumber in registers; wider
+  // rows load the rest in place.
   constexpr int KQ = (RW * (M + 1) + 63) / 64;              // nxh <= M + 1
   constexpr int KPD = (RW * ((2 * M) / 3 + 1) + 63) / 64;
   constexpr int KP = KPD < KQ ? KPD : KQ;
+  constexpr int G0 = RW == 1 && KP > 1 ? 2 : 1;             // columns of the first output group
   const int nout = RW * nxh;
   auto orow = [&](int i) {
     const int u = min(lane + 64 * i, nout - 1);
@@ -407,14 +451,19 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
     return r;
   };
   auto ocol = [&](int i) { return min(lane + 64 * i, nout - 1) - orow(i) * nxh; };
-  double2 rxl[KP];
+  static_assert(RW > 1 || KP <= PPL, "the columns' roots are those of the pairs");
+  double2 rxl[RW == 1 ? 1 : KP];
   double kxl[KP];
 #pragma unroll
   for (int i = 0; i < KP; ++i) {
     const int kq = ocol(i);
-    rxl[i] = rootx[kq];
+    if (RW > 1) rxl[i] = rootx[kq];
     kxl[i] = ops.kx[kq];
   }
+  auto root_of = [&](int i, int kq) {
+    if (i >= KP) return rootx[kq];
+    return RW == 1 ? cconj(wc[i < PPL ? i : 0]) : rxl[RW > 1 && i < KP ? i : 0];
+  };
   auto bufv = [&](int q) { return *reinterpret_cast<const double2*>(ops.buffer + poff(q)); };
   // Subgrid stress (LES): tau_ij is added to the flux u_i u_j wherever the
   // flux is formed, so the divergence of the fluxes carries -div(tau) with the
@@ -438,14 +487,12 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
 
   // prologue: planes ka-1 and ka, fluxes at y(ka-1) and yh(ka)
   fetch(ka - 1);
-  ready();
-  c2r_plane(ka - 1, U0, V0, W0, true);
-  fetch(ka);
+  ready(0);
+  c2r_plane(ka - 1, U0, V0, W0, ka);
   load_base(ka - 1, BU0, BV0, BW0);
   load_base(ka, BU1, BV1, BW1);
-  ready();
-  c2r_plane(ka, U1, V1, W1, true);
-  fetch(ka + 1);
+  ready(0);
+  c2r_plane(ka, U1, V1, W1, ka + 1);
 #pragma unroll
   for (int q = 0; q < PPL; ++q) {
     if (!LIN) {
@@ -467,7 +514,7 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
       double2 t = psc(half, padd(V0[q], V1[q])), tb = psc(half, padd(BV0[q], BV1[q]));
       GV[q] = pmul(psc(two, t), tb);
     }
-    if (les && vq[q]) {
+    if (les) {
       const int k0 = ka - 2;  // 0-based plane ka-1
       if (ka - 1 != 1) {      // the bottom wall carries no subgrid stress
         const double j1 = ldro(ops.iu, 2 * k0), j2 = ldro(ops.iu, 2 * k0 + 1);
@@ -480,6 +527,9 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
     BU0[q] = BU1[q]; BV0[q] = BV1[q]; BW0[q] = BW1[q];
   }
 
+  // stores of a plane below the top one: two batches of three per 64 columns
+  const int nst = 6 * ((nout + 63) / 64);
+  int later = 0;   // stores issued since the last fetch, at least
   for (int k = ka; k <= kb; ++k) {
     const bool top = (k == ny);
     const int kk = k - 1;  // 0-based plane index
@@ -489,9 +539,9 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
     double tgu = 0.0, tgv = 0.0, tgw = 0.0;
     if (hasbuf) { tgu = ldro(ops.target, 0 * nyp + kk); tgv = ldro(ops.target, 1 * nyp + kk); tgw = ldro(ops.target, 2 * nyp + kk); }
     load_base(k + 1, BU1, BV1, BW1);
-    ready();
-    c2r_plane(k + 1, U1, V1, W1, !top);
-    if (k < kb) fetch(k + 2);
+    ready(later);
+    later = nst;
+    c2r_plane(k + 1, U1, V1, W1, k < kb ? k + 2 : 0);
     double2 Fu[PPL], Fw[PPL], G1[PPL];
     // batch 1: u^2, d/dy flux_u, w u, d/dy flux_w (:138-155)
 #pragma unroll
@@ -513,7 +563,6 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
           Fw[q] = padd(pmul(BV0[q], W1[q]), pmul(V0[q], BW1[q]));
         }
       }
-      if (!vq[q]) continue;
       if (les && !top) {
         Fu[q] = padd(Fu[q], padd(psc(i1, tauv(1, kk, q)), psc(i2, tauv(1, kk + 1, q))));
         Fw[q] = padd(Fw[q], padd(psc(i1, tauv(4, kk, q)), psc(i2, tauv(4, kk + 1, q))));
@@ -530,17 +579,18 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
       if (!LIN) { f0 = pmul(U0[q], U0[q]); f2 = pmul(W0[q], U0[q]); }
       else { f0 = pmul(psc(two, BU0[q]), U0[q]); f2 = padd(pmul(BW0[q], U0[q]), pmul(W0[q], BU0[q])); }
       if (les) { f0 = padd(f0, tauv(0, kk, q)); f2 = padd(f2, tauv(2, kk, q)); }
-      W[0 * FS + pin[q]] = f0;
-      W[1 * FS + pin[q]] = yfu;
-      W[2 * FS + pin[q]] = f2;
-      W[3 * FS + pin[q]] = yfw;
+      if (vq[q]) {
+        W[0 * FS + pin[q]] = f0;
+        W[1 * FS + pin[q]] = yfu;
+        W[2 * FS + pin[q]] = f2;
+        W[3 * FS + pin[q]] = yfw;
+      }
     }
     // CFL maxima for this plane (check_cfl :211-213)
     if (a.cflbits) {
       double au = 0.0, av = 0.0, aw = 0.0;
 #pragma unroll
       for (int q = 0; q < PPL; ++q) {
-        if (!vq[q]) continue;
         au = fmax(au, pabsmax(padd(U0[q], U1[q])));
         av = fmax(av, pabsmax(V0[q]));
         aw = fmax(aw, pabsmax(padd(W0[q], W1[q])));
@@ -564,20 +614,36 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
     const long ab0 = ((long)((0 * nyp + kk) * 2) * nz2) * kxp + rowoff;
     const long ab1 = ((long)((1 * nyp + kk) * 2) * nz2) * kxp + rowoff;
     const long ab2 = ((long)((2 * nyp + kk) * 2) * nz2) * kxp + rowoff;
+    // The columns i0 .. i1-1 (x 64) of the first batch: the loads of all of
+    // them (in groups, for the registers), then the stores
+    auto out1 = [&](auto i0_, auto i1_) {
+      constexpr int i0 = decltype(i0_)::value, i1 = decltype(i1_)::value;
+      double2 Au[i1 - i0], Bu[i1 - i0], Aw[i1 - i0];
 #pragma unroll
-    for (int i = 0; i < KQ; ++i) {
-      if (lane + 64 * i >= nout) break;
-      const int kq = RW == 1 ? lane + 64 * i : ocol(i);
-      const long oo = (long)orow(i) * kxp + kq;
-      const double2* S = W + orow(i) * SEQ;
-      const double2 wk = i < KP ? rxl[i] : rootx[kq];
-      const double kxv = i < KP ? kxl[i] : ops.kx[kq];
-      auto ikxm = [&](double2 v) { return make_double2(-kxv * v.y, kxv * v.x); };
-      const double2 X0 = r2c_post_nl<M>(S + 0 * FS, M, kq, wk), X1 = r2c_post_nl<M>(S + 1 * FS, M, kq, wk);
-      const double2 X2 = r2c_post_nl<M>(S + 2 * FS, M, kq, wk), X3 = r2c_post_nl<M>(S + 3 * FS, M, kq, wk);
-      a.AB[ab0 + oo] = cadd(X1, ikxm(X0));
-      a.AB[ab0 + bst + oo] = X2;
-      a.AB[ab2 + oo] = cadd(X3, ikxm(X2));
+      for (int i = i0; i < i1; ++i) {
+        const int kq = ocol(i);
+        const double2* S = W + orow(i) * SEQ;
+        const double2 wk = root_of(i, kq);
+        const double kxv = i < KP ? kxl[i < KP ? i : 0] : ops.kx[kq];
+        const double2 X0 = r2c_post_nl<M>(S + 0 * FS, M, kq, wk), X1 = r2c_post_nl<M>(S + 1 * FS, M, kq, wk);
+        const double2 X2 = r2c_post_nl<M>(S + 2 * FS, M, kq, wk), X3 = r2c_post_nl<M>(S + 3 * FS, M, kq, wk);
+        Au[i - i0] = add_ik(X1, kxv, X0);
+        Bu[i - i0] = X2;
+        Aw[i - i0] = add_ik(X3, kxv, X2);
+      }
+#pragma unroll
+      for (int i = i0; i < i1; ++i) {
+        if (lane + 64 * i >= nout) break;
+        const long oo = (long)orow(i) * kxp + ocol(i);
+        a.AB[ab0 + oo] = Au[i - i0];
+        a.AB[ab0 + bst + oo] = Bu[i - i0];
+        a.AB[ab2 + oo] = Aw[i - i0];
+      }
+    };
+    out1(std::integral_constant<int, 0>{}, std::integral_constant<int, G0>{});
+    if constexpr (KP > G0) out1(std::integral_constant<int, G0>{}, std::integral_constant<int, KP>{});
+    if constexpr (KQ > KP) {
+      if (64 * KP < nout) out1(std::integral_constant<int, KP>{}, std::integral_constant<int, KQ>{});
     }
     wave_sync();
     // batch 2: w^2 and, below the top plane, the v fluxes (:183-195)
@@ -595,11 +661,10 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
           G1[q] = z2;
         }
       }
-      if (!vq[q]) continue;
       if (les && !top) G1[q] = padd(G1[q], tauv(3, kk + 1, q));
       double2 f4 = LIN ? pmul(psc(two, BW0[q]), W0[q]) : pmul(W0[q], W0[q]);
       if (les) f4 = padd(f4, tauv(5, kk, q));
-      W[0 * FS + pin[q]] = f4;
+      if (vq[q]) W[0 * FS + pin[q]] = f4;
       if (!top) {
         double2 f5, f7;
         if (!LIN) {
@@ -620,29 +685,44 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
           const double tv = tgv;
           yfv = padd(yfv, pmul(bufv(q), make_double2(V0[q].x - tv, V0[q].y - tv)));
         }
-        W[1 * FS + pin[q]] = f5;
-        W[2 * FS + pin[q]] = yfv;
-        W[3 * FS + pin[q]] = f7;
+        if (vq[q]) {
+          W[1 * FS + pin[q]] = f5;
+          W[2 * FS + pin[q]] = yfv;
+          W[3 * FS + pin[q]] = f7;
+        }
       }
     }
     wave_sync();
     fft2p_wave<M, -1>(W, SEQ, nb2 * RW, rl, rg, lane);
+    auto out2 = [&](auto i0_, auto i1_) {
+      constexpr int i0 = decltype(i0_)::value, i1 = decltype(i1_)::value;
+      double2 Bw[i1 - i0], Av[i1 - i0], Bv[i1 - i0];
 #pragma unroll
-    for (int i = 0; i < KQ; ++i) {
-      if (lane + 64 * i >= nout) break;
-      const int kq = RW == 1 ? lane + 64 * i : ocol(i);
-      const long oo = (long)orow(i) * kxp + kq;
-      const double2* S = W + orow(i) * SEQ;
-      const double2 wk = i < KP ? rxl[i] : rootx[kq];
-      const double kxv = i < KP ? kxl[i] : ops.kx[kq];
-      auto ikxm = [&](double2 v) { return make_double2(-kxv * v.y, kxv * v.x); };
-      a.AB[ab2 + bst + oo] = r2c_post_nl<M>(S + 0 * FS, M, kq, wk);
-      if (!top) {
+      for (int i = i0; i < i1; ++i) {
+        const int kq = ocol(i);
+        const double2* S = W + orow(i) * SEQ;
+        const double2 wk = root_of(i, kq);
+        const double kxv = i < KP ? kxl[i < KP ? i : 0] : ops.kx[kq];
+        Bw[i - i0] = r2c_post_nl<M>(S + 0 * FS, M, kq, wk);
         const double2 X5 = r2c_post_nl<M>(S + 1 * FS, M, kq, wk), X6 = r2c_post_nl<M>(S + 2 * FS, M, kq, wk);
-        const double2 X7 = r2c_post_nl<M>(S + 3 * FS, M, kq, wk);
-        a.AB[ab1 + oo] = cadd(X6, ikxm(X5));
-        a.AB[ab1 + bst + oo] = X7;
+        Av[i - i0] = add_ik(X6, kxv, X5);
+        Bv[i - i0] = r2c_post_nl<M>(S + 3 * FS, M, kq, wk);   // at the top plane Av and Bv are not stored
       }
+#pragma unroll
+      for (int i = i0; i < i1; ++i) {
+        if (lane + 64 * i >= nout) break;
+        const long oo = (long)orow(i) * kxp + ocol(i);
+        a.AB[ab2 + bst + oo] = Bw[i - i0];
+        if (!top) {
+          a.AB[ab1 + oo] = Av[i - i0];
+          a.AB[ab1 + bst + oo] = Bv[i - i0];
+        }
+      }
+    };
+    out2(std::integral_constant<int, 0>{}, std::integral_constant<int, G0>{});
+    if constexpr (KP > G0) out2(std::integral_constant<int, G0>{}, std::integral_constant<int, KP>{});
+    if constexpr (KQ > KP) {
+      if (64 * KP < nout) out2(std::integral_constant<int, KP>{}, std::integral_constant<int, KQ>{});
     }
     wave_sync();
     // slide the window (:81, :170-171, :198)
@@ -655,15 +735,23 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
   }
 }
 
+// Wavefronts per SIMD the registers are held to: two (a few of them go to
+// scratch at M = 192 and two rows of 72), but one for the linearized pass of
+// 128 and more pairs, whose base flow would go there.  Three at two rows of
+// 36 or 48 cost 20 registers of scratch: 337 against 334 ms for 60 steps of
+// the 48-member ensemble.
+template <bool LIN, int M, int RW>
+constexpr int xpass_w_waves() { return LIN && RW * M >= 128 ? 1 : 2; }
+
 template <bool LIN, int M, bool PF, bool LES = false, int RW = 1>
-__global__ __launch_bounds__(256) void k_xpass_w(XZGeom g, const double2* __restrict__ tw, DevOps ops,
+__global__ __launch_bounds__(256, (xpass_w_waves<LIN, M, RW>())) void k_xpass_w(XZGeom g, const double2* __restrict__ tw, DevOps ops,
                                                   XPassArgs a) {
   xpass_w_body<LIN, M, PF, LES, RW>(g, tw, ops, a, blockIdx.x, blockIdx.y);
 }
 
 // Batched form: workgroup i runs work-list entry it[i] of channel it[i].m.
 template <bool LIN, int M, bool PF, int RW>
-__global__ __launch_bounds__(256) void k_xpass_w_b(const XBatchArgs* __restrict__ args,
+__global__ __launch_bounds__(256, (xpass_w_waves<LIN, M, RW>())) void k_xpass_w_b(const XBatchArgs* __restrict__ args,
                                                     const BatchItem* __restrict__ it) {
   const BatchItem w = it[blockIdx.x];
   const XBatchArgs& x = args[w.m];
@@ -679,23 +767,26 @@ static bool xpass_rw_built(int M, int rw, bool pf) {
   return rw == 1 || (pf && ((rw == 2 && M <= 72) || (rw == 4 && M <= 24)));
 }
 
-// The default: two rows per wavefront where a row's pairs fill at most 36
-// lanes; the batched launches also at the lengths where that halves the
-// wavefronts per SIMD (their lengths share the GPU, so fewer idle lanes count
-// for more than latency hiding: 163 -> 178 steps/s on the 48-member
-// ensemble, where a single 64x65x64 channel's x-pass loses 1 %).
-int xpass_rows(int M, int nz2, int req, bool pf, bool batched) {
+// The default: two rows per wavefront wherever that kernel is built.  The
+// pass issues vector instructions most of the time at these lengths (three
+// wavefronts per SIMD at 64x97x64 finish at 43, 54 and 66 thousand cycles in
+// the order of their age), and the transform tasks of one row of 24 to 72
+// pairs leave half of the lanes or more idle in every one of them.  A whole
+// step with one row and two: 32x129x64 238 and 198 us, 64x97x64 244 and 238,
+// 72x81x108 356 and 335, 96x193x96 811 and 739.
+int xpass_rows(int M, int nz2, int req, bool pf) {
   auto ok = [&](int r) { return xpass_rw_built(M, r, pf) && nz2 % r == 0; };
   if (req > 0 && ok(req)) return req;
-  const int d = (M <= 27 || (batched && M <= 72)) ? 2 : 1;
+  const int d = M <= 72 ? 2 : 1;
   return ok(d) ? d : 1;
 }
 
 // LDS of a wavefront x-pass workgroup: the root table and, per wavefront, 4*rw
 // sequences and (with the prefetch) 3*rw raw rows (of M + 1 cells rounded up
-// to 64 for one row per wavefront, of nxh cells rounded up otherwise)
+// to 64 for one row per wavefront and below 64 pairs, of nxh cells rounded up
+// otherwise)
 size_t xpass_w_lds(int M, int rw, int nxh, bool pf) {
-  const int rawn = rw == 1 ? xpass_raw_cells(M + 1) : xpass_raw_cells(nxh);
+  const int rawn = rw == 1 || M < 64 ? xpass_raw_cells(M + 1) : xpass_raw_cells(nxh);
   return sizeof(double2) * (M + 4 * (4 * rw * fft_seq_cells(M) + (pf ? 3 * rw * rawn : 0)));
 }
 
@@ -817,7 +908,7 @@ void launch_xpass(const XZGeom& g, const double2* tw, const DevOps& ops, const X
   if (a.wave && ct && M <= 192) {
     const bool pf = a.prefetch && M <= 144;
     if (a.tau && a.base) throw chan_error("the subgrid closure is not defined for the linearized pass");
-    const int rw = xpass_rows(M, g.nz2, a.rows, pf, false);
+    const int rw = xpass_rows(M, g.nz2, a.rows, pf);
     const size_t ldw = xpass_w_lds(M, rw, g.nxh, pf);
     XPassFn fn = nullptr;
 #define XPASSW_CASE(N)                                                                  \

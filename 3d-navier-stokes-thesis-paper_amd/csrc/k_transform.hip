@@ -160,19 +160,7 @@ __device__ __forceinline__ double2 c2r_pack(const double2* __restrict__ row, int
     return v;
   };
   double2 a = Y(n), b = cconj(Y(M - n));
-  double2 s = cadd(a, b), d = csub(a, b);
-  double2 wd = cmul(wn_conjroot, d);  // w^n * d
-  return make_double2(s.x - wd.y, s.y + wd.x);
-}
-
-// Post-processing of a half-length forward FFT Z (length M) into the real
-// transform X_k = E_k + w^-k O_k, E = (Z_k + conj Z_{M-k})/2, O = -i (Z_k - conj Z_{M-k})/2.
-__device__ __forceinline__ double2 r2c_post(const double2* __restrict__ Zs, int M, int k, double2 wk) {
-  double2 a = Zs[k % M], b = cconj(Zs[(M - k) % M]);
-  double2 E = make_double2(0.5 * (a.x + b.x), 0.5 * (a.y + b.y));
-  double2 d = csub(a, b);
-  double2 O = make_double2(0.5 * d.y, -0.5 * d.x);
-  return cadd(E, cmul(wk, O));
+  return c2r_combine(a, b, wn_conjroot);
 }
 
 template <int NC>
@@ -235,14 +223,11 @@ __global__ __launch_bounds__(512) void k_xr2c(XZGeom g, const double2* __restric
   }
   __syncthreads();
   fft_run<NC, -1, FFT_MAXV>(lds, ss, nf * rows, g.px, tw, rl, tid, nthr);
-  // X_k = E_k + w^-k O_k from the half-length transform (r2c_post), read
-  // through the two-pass output order
+  // twice the real transform's coefficient k from the half-length transform,
+  // read through the two-pass output order (the z-forward pass halves it)
   auto post = [&](const double2* Zs, int k, double2 wk) {
-    double2 a = Zs[fft_out_pos<NC>(k % M)], b = cconj(Zs[fft_out_pos<NC>((M - k) % M)]);
-    double2 E = make_double2(0.5 * (a.x + b.x), 0.5 * (a.y + b.y));
-    double2 d = csub(a, b);
-    double2 O = make_double2(0.5 * d.y, -0.5 * d.x);
-    return cadd(E, cmul(wk, O));
+    const double2 a = Zs[fft_out_pos<NC>(k % M)], b = cconj(Zs[fft_out_pos<NC>((M - k) % M)]);
+    return r2c_combine(a, b, wk);
   };
   for (int e = tid; e < nr * g.nxh; e += nthr) {
     int r = e / g.nxh, k = e - r * g.nxh;
@@ -250,8 +235,7 @@ __global__ __launch_bounds__(512) void k_xr2c(XZGeom g, const double2* __restric
     double2 X = post(lds + r * ss, k, wk);
     if (fx) {
       double2 Xx = post(lds + (rows + r) * ss, k, wk);
-      double kk = kxv[k];
-      X = make_double2(X.x - kk * Xx.y, X.y + kk * Xx.x);
+      X = add_ik(X, kxv[k], Xx);
     }
     out[P * out_ps + (long)(z0 + r) * g.kxpad + k] = X;
   }
@@ -304,10 +288,10 @@ __global__ __launch_bounds__(512) void k_zfwd(XZGeom g, const double2* __restric
     const double2* a = lds + s * ss;
     double2 val;
     if (g.small) {
-      double sc = 1.0 / (double)(g.nx * g.nz);
+      double sc = 0.5 / (double)(g.nx * g.nz);   // the x transform gives twice its coefficients
       val = cscale(sc, at(a, q));
     } else {
-      const double scale = 1.0 / (double)(g.nx2 * g.nz2);
+      const double scale = 0.5 / (double)(g.nx2 * g.nz2);
       const double f = (kx0 + s == g.nxh - 1) ? 2.0 * scale : scale;
       double2 fa;
       if (q < h) fa = at(a, q);
@@ -437,7 +421,7 @@ __device__ __forceinline__ void zfwd2_body(const XZGeom& g, const double2* __res
   __syncthreads();
   fft2p<NC, -1>(lds, SS, ncol, rl, tw + g.pz.tw, tid, NT);  // the valid columns only
   const int h = nz / 2, off = NZ2 - nz;
-  const double scale = 1.0 / (double)(g.nx2 * NZ2);
+  const double scale = 0.5 / (double)(g.nx2 * NZ2);   // the x transform gives twice its coefficients
   auto fold = [&](const double2* a, int q) {
     if (q < h) return a[fft2_out_pos<NC>(q)];
     if (q == h) return cadd(a[fft2_out_pos<NC>(h)], cconj(a[fft2_out_pos<NC>(off + h)]));
