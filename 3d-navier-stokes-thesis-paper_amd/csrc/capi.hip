@@ -189,8 +189,9 @@ void nl_pass(chan_ctx* c, int step, int rk, bool lin, bool cfl) {
     xpass(2, ny);
     {
       KTimer t(c, KT_ZFWD);
+      const CflTail tail{CflBatchArgs{c->ops, c->prm, c->d_cfl, c->d_sc}, step, 1};
       launch_zfwd(g, c->d_tw, c->d_AB, c->d_AB + zps, 2 * zps, c->ops.kz, c->d_nl, nmodes(c), 3 * nyp, ny,
-                  c->stream, c->tune.zfwd_v2, c->tune.zfwd_kx);
+                  c->stream, c->tune.zfwd_v2, c->tune.zfwd_kx, 0, 0, 0, cfl ? &tail : nullptr);
     }
   } else {
     // plane ranges in turn, so that each range's intermediates are re-read
@@ -215,11 +216,32 @@ void nl_pass(chan_ctx* c, int step, int rk, bool lin, bool cfl) {
                     ny, c->stream, c->tune.zfwd_v2, c->tune.zfwd_kx, f1 - f0 + 1, nyp, f0);
       }
     }
+    if (cfl) launch_cfl_finalize(c->ops, c->prm, c->d_cfl, c->d_sc, step, c->stream);
   }
-  if (cfl) launch_cfl_finalize(c->ops, c->prm, c->d_cfl, c->d_sc, step, c->stream);
 }
 
-void solve_pass(chan_ctx* c, int rk) {
+// Wall data zero but for what the feedback law writes at every step and the
+// profile of a jet without forcing: cleared when they may hold anything else.
+// A clear per step was one of 14 launches, and 4.6 us of 252 at 64x97x64.
+void zero_walls(chan_ctx* c) {
+  if (c->cbc_holds != chan_ctx::CBC_ZERO) launch_fill_zero(c->d_cbc, sizeof(double2) * 6 * nmodes(c), c->stream);
+  c->cbc_holds = chan_ctx::CBC_ZERO;
+}
+void clear_walls(chan_ctx* c) {
+  if (c->d_jet && c->cbc_holds == chan_ctx::CBC_JET) c->cbc_cleared = true;   // the next substep wants it again
+  else zero_walls(c);
+}
+// The jet's part of the wall data, and the clear of it that was left out, where
+// the wall data or the jet are about to change.
+double2* jet_walls(chan_ctx* c) { return c->d_cbc + ((c->jet_wall == 0 ? 1L : 0L) * 3 + 1) * nmodes(c); }
+void settle_walls(chan_ctx* c) {
+  if (c->cbc_cleared) launch_fill_zero(jet_walls(c), sizeof(double2) * nmodes(c), c->stream);
+  c->cbc_cleared = false;
+  c->cbc_holds = chan_ctx::CBC_ANY;
+}
+
+// advance: t_total += dt behind the substep
+void solve_pass(chan_ctx* c, int rk, bool advance = false) {
   KTimer t(c, KT_SOLVE);
   SolveArgs a{};
   a.nl = c->d_nl; a.vel = c->d_vel; a.R = c->d_R; a.P = c->d_P; a.cbc = c->d_cbc; a.dudy = c->d_dudy;
@@ -228,23 +250,25 @@ void solve_pass(chan_ctx* c, int rk) {
   a.fix_mass = c->prm.fix_mass;
   a.lanes = c->tune.solve_lanes; a.bl = c->tune.solve_bl; a.dma = c->tune.solve_dma;
   a.seg = c->tune.solve_seg;
-  if (c->d_jet) {  // the jet overwrites the wall-normal velocity at its wall (PFC/pass2.f90:42-43)
+  a.advance = advance;
+  c->cbc_cleared = false;
+  // the jet overwrites the wall-normal velocity at its wall (PFC/pass2.f90:42-43);
+  // without forcing its profile stays as the last substep left it
+  if (c->d_jet && c->cbc_holds != chan_ctx::CBC_JET) {
     const long nm = nmodes(c);
-    launch_jet_bc(c->d_sc, rk, c->jet_forcing, c->jet_freq, c->d_jet,
-                  c->d_cbc + ((c->jet_wall == 0 ? 1L : 0L) * 3 + 1) * nm, nm, c->stream);
+    const bool keep = c->jet_forcing == 0.0 && c->cbc_holds == chan_ctx::CBC_ZERO;
+    c->cbc_holds = chan_ctx::CBC_ANY;
+    launch_jet_bc(c->d_sc, rk, c->jet_forcing, c->jet_freq, c->d_jet, jet_walls(c), nm, c->stream);
+    if (keep) c->cbc_holds = chan_ctx::CBC_JET;
   }
   launch_solve(c->ops, a, c->stream);
-}
-
-__global__ void k_advance_time(DevScalars* sc) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) sc->t_total = sc->t_total + sc->dt;
 }
 
 // boundary (PFC/read_write.f90:1465-1532)
 void boundary_dev(chan_ctx* c) {
   KTimer t(c, KT_OTHER);
   const long nm = nmodes(c);
-  launch_fill_zero(c->d_cbc, sizeof(double2) * 6 * nm, c->stream);
+  clear_walls(c);
   const double gains[2] = {c->prm.ctrlu, c->prm.ctrlw};
   if (gains[0] == 0.0 && gains[1] == 0.0) return;
   const XZGeom& g = c->gd;
@@ -380,10 +404,18 @@ void step_body(chan_ctx* c, int step, bool lin) {
   boundary_dev(c);
   for (int rk = 1; rk <= 3; ++rk) {
     nl_pass(c, step, rk, lin, rk == 1);
-    solve_pass(c, rk);
+    solve_pass(c, rk, rk == 3);
   }
-  hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(64), 0, c->stream, c->d_sc);
-  LAUNCH_CHECK("k_advance_time");
+}
+
+// The wall data ahead of the capture or a replay of a step: a step captured
+// without jet and feedback (plain) has no clear of its own, so they must be
+// zero before it; any other is captured with the clear and the jet's launch.
+bool plain_walls(const chan_ctx* c) { return !c->d_jet && c->prm.ctrlu == 0.0 && c->prm.ctrlw == 0.0; }
+void graph_walls(chan_ctx* c, bool plain) {
+  c->cbc_cleared = false;
+  if (plain) zero_walls(c);
+  else c->cbc_holds = chan_ctx::CBC_ANY;
 }
 
 // Everything step_body may allocate or synchronise for, done ahead of a capture.
@@ -393,6 +425,7 @@ void prepare_capture(chan_ctx* c) {
   if (c->prm.ctrlu != 0.0 || c->prm.ctrlw != 0.0) (void)stage(c, sizeof(double) * 6 * (size_t)c->gd.nz2 * c->gd.nx2);
   if (c->timing) throw chan_error("disable timing before batching or tuning");
   les_prepare_capture(c);
+  graph_walls(c, plain_walls(c));
   CHAN_CHECK(hipStreamSynchronize(c->stream));
 }
 
@@ -515,9 +548,7 @@ struct chan_ensemble {
   bool batched = false;
   std::vector<BatchLaunch> zinv, zfwd, xpass[2], solve[3];  // xpass[1]: with the CFL maxima; solve[rk-1]
   CflBatchArgs* cfl_args = nullptr;
-  FillBatchArgs* fill_cbc = nullptr;
-  DevScalars** scs = nullptr;
-  size_t cbc_words = 0;
+  std::vector<char> plain;   // member captured without a clear of its wall data (graph_walls)
   std::vector<void*> dmem;     // device tables of the batched launches
   // the launches of one phase touch disjoint members: they run as parallel
   // branches of the graph (fork from the master stream, join back)
@@ -709,6 +740,7 @@ void ensemble_plan_batched(chan_ensemble* e) {
           a.re = c->prm.re; a.cosb = std::cos(c->prm.beta); a.sinb = std::sin(c->prm.beta);
           a.fix_mass = c->prm.fix_mass;
           a.lanes = c->tune.solve_lanes; a.bl = c->tune.solve_bl; a.dma = c->tune.solve_dma; a.seg = 1;
+          a.advance = rk == 3;
           return x;
         },
         [&](chan_ctx* c, unsigned short k, std::vector<BatchItem>& it) {
@@ -720,22 +752,15 @@ void ensemble_plan_batched(chan_ensemble* e) {
         if (layout(c) == b.len) b.ny = std::max(b.ny, c->prm.ny);
   }
   std::vector<CflBatchArgs> cf;
-  std::vector<FillBatchArgs> fc;
-  std::vector<DevScalars*> sc;
   for (chan_ctx* c : e->m) {
     cf.push_back(CflBatchArgs{c->ops, c->prm, c->d_cfl, c->d_sc});
-    const size_t cw = 6 * (size_t)nmodes(c) * sizeof(double2) / 8;
-    fc.push_back(FillBatchArgs{(unsigned long long*)c->d_cbc, cw});
-    e->cbc_words = std::max(e->cbc_words, cw);
-    sc.push_back(c->d_sc);
   }
   e->cfl_args = (CflBatchArgs*)upload_table(e, cf);
-  e->fill_cbc = (FillBatchArgs*)upload_table(e, fc);
-  e->scs = (DevScalars**)upload_table(e, sc);
 }
 
 // One timestep of every member as batched launches (PFC/main_mpi.f90:73-90
-// for all of them at once): boundary with zero gains (wall data cleared),
+// for all of them at once): boundary with zero gains (the wall data are zero,
+// graph_walls),
 // three substeps of z-inverse, x-pass, z-forward (CFL and dt at the first)
 // and solve, then t_total += dt.
 void ensemble_step_batched(chan_ensemble* e, hipStream_t s) {
@@ -759,7 +784,6 @@ void ensemble_step_batched(chan_ensemble* e, hipStream_t s) {
       CHAN_CHECK(hipStreamWaitEvent(s, e->bjoin[j % e->bjoin.size()], 0));
     }
   };
-  launch_fill_zero_batched(e->fill_cbc, n, e->cbc_words, s);
   for (int rk = 1; rk <= 3; ++rk) {
     phase(e->zinv, [&](const BatchLaunch& b, hipStream_t st) {
       launch_zinv_batched(b.len, (const ZBatchArgs*)b.args, b.items, b.nitems, st);
@@ -775,7 +799,6 @@ void ensemble_step_batched(chan_ensemble* e, hipStream_t s) {
       launch_solve_batched(b.len, b.ny, (const SBatchArgs*)b.args, b.items, b.nitems, st);
     });
   }
-  launch_advance_time_batched(e->scs, n, s);
 }
 
 // Capture one timestep of every member: the members are spread round-robin
@@ -783,7 +806,11 @@ void ensemble_step_batched(chan_ensemble* e, hipStream_t s) {
 // stream, so independent members run concurrently inside one graph.  In
 // batched mode the step is the batched launches on the master stream.
 void ensemble_capture(chan_ensemble* e) {
-  for (chan_ctx* c : e->m) prepare_capture(c);
+  e->plain.clear();
+  for (chan_ctx* c : e->m) {
+    prepare_capture(c);
+    e->plain.push_back(plain_walls(c));
+  }
   if (e->batched) {
     if (e->zinv.empty()) ensemble_plan_batched(e);
     for (chan_ctx* c : e->m) c->data1_is_nl = false;
@@ -811,14 +838,17 @@ void ensemble_capture(chan_ensemble* e) {
       c->stream = e->streams[i % e->streams.size()];
       step_body(c, 1, e->lin != 0);
       c->stream = saved[i];
+      if (!e->plain[i]) graph_walls(c, false);   // recorded, not run
     }
     for (size_t k = 0; k < e->streams.size(); ++k) {
       CHAN_CHECK(hipEventRecord(e->done[k], e->streams[k]));
       CHAN_CHECK(hipStreamWaitEvent(e->master, e->done[k], 0));
     }
   } catch (...) {
-    for (size_t i = 0; i < e->m.size(); ++i)
+    for (size_t i = 0; i < e->m.size(); ++i) {
       if (saved[i]) e->m[i]->stream = saved[i];
+      e->m[i]->cbc_holds = chan_ctx::CBC_ANY;
+    }
     hipGraph_t g = nullptr;
     (void)hipStreamEndCapture(e->master, &g);
     if (g) (void)hipGraphDestroy(g);
@@ -894,6 +924,7 @@ int chan_create(const chan_params* prm, chan_ctx** out) {
     CHAN_CHECK(hipMemset(c->d_R, 0, vel_bytes(c)));
     CHAN_CHECK(hipMemset(c->d_P, 0, p_bytes(c)));
     CHAN_CHECK(hipMemset(c->d_cbc, 0, sizeof(double2) * 6 * nm));
+    c->cbc_holds = chan_ctx::CBC_ZERO;
     CHAN_CHECK(hipMemset(c->d_dudy, 0, sizeof(double) * p.ny));
     // the CFL maxima start at zero here; the finalize kernel clears them
     // after each read
@@ -1113,6 +1144,7 @@ int chan_get_scalars(chan_ctx* c, double* dt, double* t_total, double* p_grad, d
 int chan_set_wall_bc(chan_ctx* c, const double* top, const double* bot) {
   return guarded(c, [&] {
     const size_t b = sizeof(double2) * 3 * nmodes(c);
+    settle_walls(c);
     if (top) h2d(c, c->d_cbc, top, b);
     if (bot) h2d(c, c->d_cbc + 3 * nmodes(c), bot, b);
     CHAN_CHECK(hipStreamSynchronize(c->stream));
@@ -1179,6 +1211,7 @@ int chan_jet_configure(chan_ctx* c, int wall, double amplitude, double radius, d
   return guarded(c, [&] {
     check_ops(c);
     if (wall != 0 && wall != 1) throw chan_error("jet wall must be 0 (bottom) or 1 (top)");
+    settle_walls(c);
     if (amplitude == 0.0) {
       dfree(c->d_jet);
       c->d_jet = nullptr;
@@ -1558,7 +1591,9 @@ int chan_linearized_matvec(chan_ctx* c, const double* v, double* w, int tend, do
     launch_arnoldi_scale(ny, plane_c, c->d_vel, c->ops.dy, c->ops.dyh, vmax, 1.0e-8, 0, c->stream);
     c->data1_is_nl = false;
     d2d(c, c->d_R, c->d_vel, vel_bytes(c));
-    launch_fill_zero(c->d_cbc, sizeof(double2) * 6 * plane_c, c->stream);
+    c->cbc_holds = chan_ctx::CBC_ANY;
+    c->cbc_cleared = false;
+    zero_walls(c);
     DevScalars sc;
     d2h(c, &sc, c->d_sc, sizeof(sc));
     const double dt = sc.dt;
@@ -1920,6 +1955,12 @@ int chan_ensemble_step(chan_ensemble* e, int nsteps) {
       CHAN_CHECK(hipStreamSynchronize(c->stream));
     }
     if (!e->exec) ensemble_capture(e);
+    for (size_t i = 0; i < e->m.size(); ++i) {
+      chan_ctx* c = e->m[i];
+      const bool wait = e->plain[i] && c->cbc_holds != chan_ctx::CBC_ZERO;
+      graph_walls(c, e->plain[i]);
+      if (wait) CHAN_CHECK(hipStreamSynchronize(c->stream));
+    }
     for (int s = 0; s < nsteps; ++s) CHAN_CHECK(hipGraphLaunch(e->exec, e->master));
     CHAN_CHECK(hipStreamSynchronize(e->master));
     std::string errs;

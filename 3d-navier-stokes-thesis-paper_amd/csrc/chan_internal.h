@@ -99,6 +99,48 @@ struct PlaneMap {
   int cnt, stride, off;
 };
 
+// check_cfl (PFC/pass1.f90:202-250) and the dt adaptation (:106-124), by the
+// first wavefront of a workgroup
+__device__ __forceinline__ void cfl_finalize_body(const DevOps& ops, const chan_params& prm,
+                                                  unsigned long long* cfl, DevScalars* sc, int step) {
+  // one wavefront: lane l takes the planes k = 2 + l, 2 + l + 64, ...; the
+  // maximum and the abort flag do not depend on the order of the planes.
+  // Each lane clears the maxima it has read, so the next pass starts from zero.
+  const int lane = threadIdx.x;
+  const int ny = prm.ny;
+  const double dt = sc->dt;
+  double cmax = 0.0;   // every plane's CFL number is >= 0
+  int err = 0;
+  for (int k = 2 + lane; k <= ny; k += 64) {
+    const int kk = k - 1;
+    double amax = __longlong_as_double((long long)cfl[3 * kk + 0]);
+    double vmax = __longlong_as_double((long long)cfl[3 * kk + 1]);
+    double wmax = __longlong_as_double((long long)cfl[3 * kk + 2]);
+    cfl[3 * kk + 0] = 0ull;
+    cfl[3 * kk + 1] = 0ull;
+    cfl[3 * kk + 2] = 0ull;
+    double tempa = 0.5 * amax * (double)prm.nx / (0.55 * prm.lx);
+    double tempb = vmax / (1.73 * fmin(ops.hn[k - 1], ops.hn[k - 2]));
+    double tempc = 0.5 * wmax * (double)prm.nz / (0.55 * prm.lz);
+    double c = (tempa + tempb + tempc) * dt;
+    if (prm.dt_flag == 1) { if (c >= 3.0e2) err = 2; }
+    else if (c >= 1.15) err = 1;
+    if (!(c <= cmax)) cmax = c;   // a NaN plane makes the maximum NaN
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    const double oc = __shfl_xor(cmax, o, 64);
+    if (!(oc <= cmax)) cmax = oc;
+    err = max(err, __shfl_xor(err, o, 64));
+  }
+  if (lane != 0) return;
+  sc->cfl = cmax;
+  if (err && !sc->err) sc->err = err;
+  if (step >= 0 && prm.dt_flag == 1) {
+    double dt_temp = dt * prm.cfl_max / cmax;
+    sc->dt = fmin(dt_temp, dt + (dt_temp - dt) * dt / (1.0 + dt));
+  }
+}
+
 // Batched launches (the batched ensemble): workgroup i of a launch runs entry
 // i of a work list, the workgroup (bx, by) of channel m's own grid.
 struct BatchItem {
@@ -198,6 +240,10 @@ struct chan_ctx {
   LesState* les = nullptr;       // subgrid closure (chan_les_configure)
   double2* d_jet = nullptr;      // wall jet: spectral v profile [nxh][nz] (chan_jet_configure)
   int jet_wall = 0;              // 0 bottom, 1 top
+  // What d_cbc holds besides the components the feedback law writes at every
+  // step: anything, zeros, or zeros and the profile of a jet without forcing.
+  enum { CBC_ANY, CBC_ZERO, CBC_JET } cbc_holds = CBC_ANY;
+  bool cbc_cleared = false;      // boundary has run since: the jet's profile counts as cleared
   double jet_forcing = 0.0, jet_freq = 0.0;
   // options
   Tuning tune;
@@ -225,9 +271,21 @@ void launch_xc2r(const XZGeom& g, const double2* tw, const double2* Z, long z_ps
                  long out_ps, int nplanes, hipStream_t s);
 void launch_xr2c(const XZGeom& g, const double2* tw, const double* fy, const double* fx,
                  const double* kx, long in_ps, double2* out, long out_ps, int nplanes, hipStream_t s);
+// The CFL number and dt of one channel (cfl_finalize_body); on = 0: nothing to do
+struct CflBatchArgs {
+  DevOps ops;
+  chan_params prm;
+  unsigned long long* cfl;
+  DevScalars* sc;
+};
+struct CflTail {
+  CflBatchArgs x;
+  int step, on;
+};
 void launch_zfwd(const XZGeom& g, const double2* tw, const double2* A, const double2* B, long ab_ps,
                  const double* kz, double2* out, long out_ps, int nplanes, int nl_zero_ny,
-                 hipStream_t s, int v2 = 1, int kx = 8, int pcnt = 0, int pstride = 0, int poff = 0);
+                 hipStream_t s, int v2 = 1, int kx = 8, int pcnt = 0, int pstride = 0, int poff = 0,
+                 const CflTail* cfl = nullptr);
 bool zt_batchable(int nz2);
 void launch_zinv_batched(int nz2, const ZBatchArgs* args, const BatchItem* items, int nitems, hipStream_t s);
 void launch_zfwd_batched(int nz2, const ZBatchArgs* args, const BatchItem* items, int nitems, hipStream_t s);
@@ -258,22 +316,14 @@ struct SolveArgs {
   int lanes, bl;      // kernel variant (Tuning::solve_lanes, solve_bl)
   int dma;            // 3-lane variant: rows streamed through an LDS ring (Tuning::solve_dma)
   int seg;            // segmented column solve where the row count allows (Tuning::solve_seg)
+  int advance;        // 1: t_total += dt behind this substep
 };
 void launch_solve(const DevOps& ops, const SolveArgs& a, hipStream_t s);
+void launch_advance_time(DevScalars* sc, hipStream_t s);
 // batched forms (the batched ensemble)
 struct SBatchArgs {
   DevOps ops;
   SolveArgs a;
-};
-struct CflBatchArgs {
-  DevOps ops;
-  chan_params prm;
-  unsigned long long* cfl;
-  DevScalars* sc;
-};
-struct FillBatchArgs {
-  unsigned long long* p;
-  size_t n;   // 8-byte words
 };
 void launch_solve_batched(int layout, int ny, const SBatchArgs* args, const BatchItem* items, int nitems, hipStream_t s);
 // Rows per segment of the workgroup solve (0: the sweep-based solve), and its
@@ -281,8 +331,6 @@ void launch_solve_batched(int layout, int ny, const SBatchArgs* args, const Batc
 int solve_wg_seg(int ny, int solve_seg);
 int solve_wg_layout(int ny, int solve_seg);
 void launch_cfl_finalize_batched(const CflBatchArgs* args, int n, int step, hipStream_t s);
-void launch_fill_zero_batched(const FillBatchArgs* args, int n, size_t max_words, hipStream_t s);
-void launch_advance_time_batched(DevScalars* const* sc, int n, hipStream_t s);
 bool solve_batchable(int ny);  // ny+1 rows a batched ensemble's solve takes
 void launch_jet_bc(const DevScalars* sc, int rk, double forcing, double freq, const double2* prof, double2* cbcv,
                    long nm, hipStream_t s);

@@ -694,6 +694,7 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
   double alpha = 1.0 + vis_imp * k2;
   double2 msh0 = cz(), msh2 = cz();     // mean pressure gradient (:220-221)
   if (bx == 0) {
+    if (a.advance && tid == 0) a.sc->t_total = a.sc->t_total + dt;   // no solve reads the time
     // mean-mode pressure gradient (compute_p_grad, :369-373)
     double p_grad = a.sc->p_grad;
     if (a.fix_mass == 1) {
@@ -1630,7 +1631,7 @@ void launch_solve(const DevOps& ops, const SolveArgs& a, hipStream_t s) {
       default: hipLaunchKernelGGL((k_solve_wg<5>), gs, bs, lds, s, ops, a); break;
     }
     LAUNCH_CHECK("k_solve_wg");
-    return;
+    return;   // it advances the time itself
   }
   if (lanes == 3 && off32) {
     dim3 g3((unsigned)((nm + 19) / 20));
@@ -1639,12 +1640,14 @@ void launch_solve(const DevOps& ops, const SolveArgs& a, hipStream_t s) {
     else if (bl == 16) hipLaunchKernelGGL((k_solve3<16, false>), g3, dim3(64), 0, s, ops, a);
     else hipLaunchKernelGGL((k_solve3<8, false>), g3, dim3(64), 0, s, ops, a);
     LAUNCH_CHECK("k_solve3");
+    if (a.advance) launch_advance_time(a.sc, s);
     return;
   }
   if (bl == 4) hipLaunchKernelGGL(k_solve<4>, grid, dim3(64), 0, s, ops, a);
   else if (bl == 16) hipLaunchKernelGGL(k_solve<16>, grid, dim3(64), 0, s, ops, a);
   else hipLaunchKernelGGL(k_solve<8>, grid, dim3(64), 0, s, ops, a);
   LAUNCH_CHECK("k_solve");
+  if (a.advance) launch_advance_time(a.sc, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1823,48 +1826,8 @@ void launch_subtract_grad_cols(const DevOps& ops, int ny, double2* crhs, const d
 }
 
 // ---------------------------------------------------------------------------
-// CFL number and dt adaptation (check_cfl PFC/pass1.f90:202-250, :106-124)
+// CFL number and dt adaptation by a launch of their own (cfl_finalize_body)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void cfl_finalize_body(const DevOps& ops, const chan_params& prm,
-                                                  unsigned long long* cfl, DevScalars* sc, int step) {
-  // one wavefront: lane l takes the planes k = 2 + l, 2 + l + 64, ...; the
-  // maximum and the abort flag do not depend on the order of the planes.
-  // Each lane clears the maxima it has read, so the next pass starts from zero.
-  const int lane = threadIdx.x;
-  const int ny = prm.ny;
-  const double dt = sc->dt;
-  double cmax = 0.0;   // every plane's CFL number is >= 0
-  int err = 0;
-  for (int k = 2 + lane; k <= ny; k += 64) {
-    const int kk = k - 1;
-    double amax = __longlong_as_double((long long)cfl[3 * kk + 0]);
-    double vmax = __longlong_as_double((long long)cfl[3 * kk + 1]);
-    double wmax = __longlong_as_double((long long)cfl[3 * kk + 2]);
-    cfl[3 * kk + 0] = 0ull;
-    cfl[3 * kk + 1] = 0ull;
-    cfl[3 * kk + 2] = 0ull;
-    double tempa = 0.5 * amax * (double)prm.nx / (0.55 * prm.lx);
-    double tempb = vmax / (1.73 * fmin(ops.hn[k - 1], ops.hn[k - 2]));
-    double tempc = 0.5 * wmax * (double)prm.nz / (0.55 * prm.lz);
-    double c = (tempa + tempb + tempc) * dt;
-    if (prm.dt_flag == 1) { if (c >= 3.0e2) err = 2; }
-    else if (c >= 1.15) err = 1;
-    if (!(c <= cmax)) cmax = c;   // a NaN plane makes the maximum NaN
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    const double oc = __shfl_xor(cmax, o, 64);
-    if (!(oc <= cmax)) cmax = oc;
-    err = max(err, __shfl_xor(err, o, 64));
-  }
-  if (lane != 0) return;
-  sc->cfl = cmax;
-  if (err && !sc->err) sc->err = err;
-  if (step >= 0 && prm.dt_flag == 1) {
-    double dt_temp = dt * prm.cfl_max / cmax;
-    sc->dt = fmin(dt_temp, dt + (dt_temp - dt) * dt / (1.0 + dt));
-  }
-}
-
 __global__ __launch_bounds__(64) void k_cfl_finalize(DevOps ops, chan_params prm,
                                                      unsigned long long* cfl, DevScalars* sc,
                                                      int step) {
@@ -1903,31 +1866,14 @@ void launch_fill_zero(void* p, size_t bytes, hipStream_t s) {
   LAUNCH_CHECK("k_fill_zero");
 }
 
-// Zero fill of several buffers in one launch (the batched ensemble): y-row i
-// of the grid clears buffer i (8-byte words).
-__global__ void k_fill_zero_b(const FillBatchArgs* __restrict__ args) {
-  const FillBatchArgs f = args[blockIdx.y];
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < f.n; i += (size_t)gridDim.x * blockDim.x)
-    f.p[i] = 0ull;
+// t_total += dt, behind a solve that does not do it itself
+__global__ void k_advance_time(DevScalars* sc) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) sc->t_total = sc->t_total + sc->dt;
 }
 
-void launch_fill_zero_batched(const FillBatchArgs* args, int n, size_t max_words, hipStream_t s) {
-  if (n <= 0 || max_words == 0) return;
-  const unsigned bx = (unsigned)std::min<size_t>((max_words + 255) / 256, 256);
-  hipLaunchKernelGGL(k_fill_zero_b, dim3(bx, n), dim3(256), 0, s, args);
-  LAUNCH_CHECK("k_fill_zero_b");
-}
-
-// t_total += dt of every channel of a batch
-__global__ void k_advance_time_b(DevScalars* const* __restrict__ sc, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) sc[i]->t_total = sc[i]->t_total + sc[i]->dt;
-}
-
-void launch_advance_time_batched(DevScalars* const* sc, int n, hipStream_t s) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_advance_time_b, dim3((n + 63) / 64), dim3(64), 0, s, sc, n);
-  LAUNCH_CHECK("k_advance_time_b");
+void launch_advance_time(DevScalars* sc, hipStream_t s) {
+  hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(64), 0, s, sc);
+  LAUNCH_CHECK("k_advance_time");
 }
 
 // The segmented solve of several channels with the same segment length and

@@ -468,7 +468,14 @@ __global__ __launch_bounds__(32 * KX) void k_zfwd2(XZGeom g, const double2* __re
                                                const double2* __restrict__ B, long ab_ps,
                                                const double* __restrict__ kzv,
                                                double2* __restrict__ out, long out_ps,
-                                               int nl_zero_ny, PlaneMap pm) {
+                                               int nl_zero_ny, PlaneMap pm, CflTail cfl) {
+  // One workgroup behind the planes' takes the CFL number and dt, which the
+  // x-pass before has left its maxima for and the solve after waits for: a
+  // launch of its own took 3.3 us of 123 per step at 32x65x32.
+  if (cfl.on && blockIdx.y == gridDim.y - 1) {
+    if (blockIdx.x == 0 && threadIdx.x < 64) cfl_finalize_body(cfl.x.ops, cfl.x.prm, cfl.x.cfl, cfl.x.sc, cfl.step);
+    return;
+  }
   zfwd2_body<NC, KX>(g, tw, A, B, ab_ps, kzv, out, out_ps, nl_zero_ny, pm, blockIdx.x, blockIdx.y);
 }
 
@@ -593,7 +600,7 @@ void launch_xr2c(const XZGeom& g, const double2* tw, const double* fy, const dou
 
 void launch_zfwd(const XZGeom& g, const double2* tw, const double2* A, const double2* B, long ab_ps,
                  const double* kz, double2* out, long out_ps, int nplanes, int nl_zero_ny,
-                 hipStream_t s, int v2, int kx, int pcnt, int pstride, int poff) {
+                 hipStream_t s, int v2, int kx, int pcnt, int pstride, int poff, const CflTail* cfl) {
   const PlaneMap pm = pcnt > 0 ? PlaneMap{pcnt, pstride, poff} : PlaneMap{nplanes, 0, 0};
   dim3 grid((g.nxh + ZT_KX - 1) / ZT_KX, nplanes);
   const int nf = B ? 2 : 1;
@@ -601,15 +608,16 @@ void launch_zfwd(const XZGeom& g, const double2* tw, const double2* A, const dou
   const bool ct = fft2_split(g.nz2).n1 > 0;
   if (v2 && ct && B && !g.small && g.nz <= 192) {
     const int k2 = (kx == 4 && fft2_batched(g.nz2)) ? 4 : 8;
-    dim3 g2((g.nxh + k2 - 1) / k2, nplanes);
+    const CflTail tail = cfl ? *cfl : CflTail{};
+    dim3 g2((g.nxh + k2 - 1) / k2, nplanes + (cfl ? 1 : 0));
     size_t l2 = sizeof(double2) * (k2 * fft_seq_cells(g.nz2) + g.nz2);
 #define ZFWD2_CASE(N)                                                                                       \
   if constexpr (fft2_batched(N))                                                                            \
     if (k2 == 4) hipLaunchKernelGGL((k_zfwd2<N, 4>), g2, dim3(128), l2, s, g, tw, A, B, ab_ps, kz, out, out_ps, \
-                                    nl_zero_ny, pm);                                                        \
+                                    nl_zero_ny, pm, tail);                                                  \
   if constexpr (N > 0)                                                                                      \
     if (k2 == 8) hipLaunchKernelGGL((k_zfwd2<N, 8>), g2, dim3(256), l2, s, g, tw, A, B, ab_ps, kz, out, out_ps, \
-                                    nl_zero_ny, pm)
+                                    nl_zero_ny, pm, tail)
     FFT_DISPATCH(g.nz2, ZFWD2_CASE)
 #undef ZFWD2_CASE
     LAUNCH_CHECK("k_zfwd2");
@@ -623,4 +631,5 @@ void launch_zfwd(const XZGeom& g, const double2* tw, const double2* A, const dou
   FFT_DISPATCH(g.nz2, ZFWD_CASE)
 #undef ZFWD_CASE
   LAUNCH_CHECK("k_zfwd");
+  if (cfl) launch_cfl_finalize(cfl->x.ops, cfl->x.prm, cfl->x.cfl, cfl->x.sc, cfl->step, s);
 }
