@@ -1657,17 +1657,23 @@ int chan_l2_norm(chan_ctx* c, double* l2, double* drag) {
       const double yy = c->h_y[std::min(j, ny - 1)];
       lam[j] = 1.0 - yy * yy;
     }
-    char* s = (char*)stage(c, sizeof(double) * (nyp + 3 * nyp + 2) + 64);
+    const bool modes = g.nx2 > c->prm.nx && g.nz2 > c->prm.nz;   // Parseval on a dealiased grid (k_l2_modes)
+    const int np = modes ? l2_modes_parts(nyp) : 3 * nyp;
+    char* s = (char*)stage(c, sizeof(double) * (nyp + np + 2) + 64);
     double* d_lam = (double*)s;
     double* part = d_lam + nyp;
-    double* res = part + 3 * nyp;
+    double* res = part + np;
     h2d(c, d_lam, lam.data(), sizeof(double) * nyp);
-    double* phys = (double*)c->d_AB;
-    for (int comp = 0; comp < 3; ++comp) {
-      dev_c2r(c, g, c->d_vel + (long)comp * nyp * nmodes(c), nyp, phys);
-      launch_l2_planes(phys, ps, nyp, comp == 0 ? d_lam : nullptr, c->ops.dy, part + (long)comp * nyp, c->stream);
+    if (modes) {
+      launch_l2_modes(g, c->d_vel, nyp, d_lam, c->ops.dy, part, c->stream);
+    } else {
+      double* phys = (double*)c->d_AB;
+      for (int comp = 0; comp < 3; ++comp) {
+        dev_c2r(c, g, c->d_vel + (long)comp * nyp * nmodes(c), nyp, phys);
+        launch_l2_planes(phys, ps, nyp, comp == 0 ? d_lam : nullptr, c->ops.dy, part + (long)comp * nyp, c->stream);
+      }
     }
-    launch_l2_final(part, 3 * nyp, (double)ps, c->d_dudy, ny, res, c->stream);
+    launch_l2_final(part, np, (double)ps, c->d_dudy, ny, res, c->stream);
     double h[2];
     d2h(c, h, res, sizeof(h));
     if (l2) *l2 = h[0];
@@ -1695,11 +1701,18 @@ int chan_plane_moments(chan_ctx* c, double* out) {
     const long ps = (long)g.nx2 * g.nz2, cs = (long)nyp * ps;
     if ((size_t)3 * cs * sizeof(double) > (size_t)2 * 3 * nyp * c->gd.nz2 * c->gd.kxpad * sizeof(double2))
       throw chan_error("plane_moments: physical planes do not fit the transform buffer");
-    double* phys = (double*)c->d_AB;
-    dev_c2r(c, g, c->d_vel, 3 * nyp, phys);
     const size_t b = sizeof(double) * 15 * nyp;
-    double* d = (double*)stage(c, b);
-    launch_plane_moments(phys, ps, cs, nyp, d, c->stream);
+    if (!plane_moments_fused(g)) {
+      double* d = (double*)stage(c, b);
+      dev_c2r(c, g, c->d_vel, 3 * nyp, (double*)c->d_AB);
+      launch_plane_moments_points((const double*)c->d_AB, ps, cs, nyp, d, c->stream);
+      d2h(c, out, d, b);
+      return;
+    }
+    double* d = (double*)stage(c, b + sizeof(double) * plane_moments_part(g, nyp));
+    const long zps = (long)g.nz2 * g.kxpad;
+    launch_zinv(g, c->d_tw, c->d_vel, nmodes(c), c->d_Z, zps, 3 * nyp, c->stream);
+    launch_plane_moments(g, c->d_tw, c->d_Z, zps, nyp, c->d_vel, d + 15 * nyp, d, c->stream);
     d2h(c, out, d, b);
   });
 }
@@ -1729,18 +1742,9 @@ int chan_mass_flux(chan_ctx* c, double* out) {
   return guarded(c, [&] {
     check_ops(c);
     const int nyp = c->nyp;
-    std::vector<double2> col(nyp);
-    std::vector<double> dyh(nyp);
-    const double2* src = c->data1_is_nl ? c->d_nl : c->d_vel;
-    double2* pc = (double2*)pinned(c, sizeof(double2) * nyp);
-    CHAN_CHECK(hipMemcpy2DAsync(pc, sizeof(double2), src, sizeof(double2) * nmodes(c), sizeof(double2), nyp,
-                                hipMemcpyDeviceToHost, c->stream));
-    CHAN_CHECK(hipStreamSynchronize(c->stream));
-    std::memcpy(col.data(), pc, sizeof(double2) * nyp);
-    d2h(c, dyh.data(), c->ops.dyh, sizeof(double) * nyp);
-    double q = 0.0;
-    for (int j = 0; j < nyp; ++j) q += col[j].x * dyh[j];
-    *out = q;
+    double* d = (double*)stage(c, sizeof(double));
+    launch_mass_flux(c->data1_is_nl ? c->d_nl : c->d_vel, nmodes(c), nyp, c->ops.dyh, d, c->stream);
+    d2h(c, out, d, sizeof(double));
   });
 }
 

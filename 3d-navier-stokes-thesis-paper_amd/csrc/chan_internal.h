@@ -36,6 +36,16 @@ struct XZGeom {
   int twx;            // root-table offset for length nx2 (real pre/post twiddles)
 };
 
+// A batch of nseq transforms of the runtime-planned kind must fit the values a thread stages.
+inline void check_stage_fit(const FFTPlan& p, int nseq, int nthr) {
+  for (int i = 0; i < p.nst; ++i) {
+    int R = p.rad[i];
+    long nbf = (long)nseq * (p.n / R);
+    long per = (nbf + nthr - 1) / nthr;
+    if (per * R > FFT_MAXV) throw chan_error("FFT batch too large for workgroup");
+  }
+}
+
 // Device-resident scalars of one channel instance.
 struct DevScalars {
   double dt;
@@ -336,9 +346,17 @@ void launch_jet_bc(const DevScalars* sc, int rk, double forcing, double freq, co
                    long nm, hipStream_t s);
 void launch_l2_planes(const double* phys, long ps, int nplanes, const double* lam, const double* dy, double* part,
                       hipStream_t s);
+int l2_modes_parts(int nyp);
+void launch_l2_modes(const XZGeom& g, const double2* vel, int nyp, const double* lam, const double* dy, double* part,
+                     hipStream_t s);
 void launch_l2_final(const double* part, int n, double npts, const double* dudy, int ny, double* out, hipStream_t s);
+void launch_mass_flux(const double2* vel, long nm, int nyp, const double* dyh, double* out, hipStream_t s);
 void launch_mode_energy(const DevOps& ops, int ny, int nxh, int nz, const double2* vel, double* ke, hipStream_t s);
-void launch_plane_moments(const double* phys, long ps, long cs, int nyp, double* out, hipStream_t s);
+bool plane_moments_fused(const XZGeom& g);
+long plane_moments_part(const XZGeom& g, int nyp);
+void launch_plane_moments_points(const double* phys, long ps, long cs, int nyp, double* out, hipStream_t s);
+void launch_plane_moments(const XZGeom& g, const double2* tw, const double2* Z, long z_ps, int nyp, const double2* vel,
+                          double* part, double* out, hipStream_t s);
 void launch_vtk_field(int ny, long nm, const double2* vel, double2* out, hipStream_t s);
 // cols == nullptr: every (kx, kz) of a [3][ny+1][nxh][nz] field; else ncols
 // columns complex(ny+1, 3, ncols) with 0-based mode indices cols[2m], cols[2m+1]

@@ -490,15 +490,6 @@ __global__ __launch_bounds__(32 * KX) void k_zfwd2_b(const ZBatchArgs* __restric
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
-static void check_stage_fit(const FFTPlan& p, int nseq, int nthr) {
-  for (int i = 0; i < p.nst; ++i) {
-    int R = p.rad[i];
-    long nbf = (long)nseq * (p.n / R);
-    long per = (nbf + nthr - 1) / nthr;
-    if (per * R > FFT_MAXV) throw chan_error("FFT batch too large for workgroup");
-  }
-}
-
 void launch_zinv(const XZGeom& g, const double2* tw, const double2* in, long in_ps, double2* out,
                  long out_ps, int nplanes, hipStream_t s, int kx, int pcnt, int pstride, int poff) {
   const PlaneMap pm = pcnt > 0 ? PlaneMap{pcnt, pstride, poff} : PlaneMap{nplanes, 0, 0};
