@@ -98,118 +98,140 @@ __device__ __forceinline__ double contract(const double* a, const double* b) {
 }
 
 // Dynamic procedure with the trapezoidal test filter (1/4, 1/2, 1/4) along x,
-// then along z, of the closure fields on the dealiased grid, fused: a
-// workgroup takes a 16 x 16 tile of one interior plane with a one-point
-// (periodic) halo in LDS, holding the 12 closure fields and the 12 products
-// u_i u_j, |S| S_ij at every halo point; every point of the tile filters
-// them, forms L_ij = T(u_i u_j) - T(u_i) T(u_j),
-// M_ij = 2 D^2 (T(|S| S_ij) - 4 |S^| S^_ij), and the workgroup sums L:M and
-// M:M (partials per tile, reduced per plane by k_les_cs2).  With FEAT it also
-// writes the network inputs of its tile's points from the gradients it holds
-// in LDS, as k_les_feat does (same arithmetic), so that the learned closure
-// needs no separate pass over the gradients where C(y) is recomputed.
-#define DYN_T 16
-#define DYN_H (DYN_T + 2)
+// then along z, of the closure fields on the dealiased grid, fused.  A
+// wavefront takes a segment of at most 62 points along x with a one-point
+// (periodic) halo and walks DYN_Z rows of it in z: at every row it forms the
+// 12 closure fields and the 12 products u_i u_j, |S| S_ij, filters them along
+// x through its LDS slice, and from the x-filtered values of the last three
+// rows, which stay in registers, forms L_ij = T(u_i u_j) - T(u_i) T(u_j) and
+// M_ij = 2 D^2 (T(|S| S_ij) - 4 |S^| S^_ij) of the middle one.  The workgroup
+// sums L:M and M:M (partials per workgroup, reduced per plane by k_les_cs2).
+// With FEAT it also writes the network inputs of its points from the
+// gradients in registers, as k_les_feat does (same arithmetic), so that the
+// learned closure needs no separate pass over the gradients where C(y) is
+// recomputed.  Bounded by vector issue: a 16 x 16 tile with its halo and all
+// 24 fields in LDS read 9 values per field and point where this reads 3, at
+// two workgroups per compute unit: 45 us at 64x65x64, 32 now.
+#define DYN_Z 8
+#define DYN_X 62
 template <bool FEAT>
-__global__ __launch_bounds__(256) void k_les_dyn(int ny, int nz2, int nx2, const double* __restrict__ Ph,
-                                                 const double* __restrict__ delta2, double* __restrict__ part,
-                                                 const double* __restrict__ ydist, float* __restrict__ X,
-                                                 double* __restrict__ scale) {
-  __shared__ double F[24][DYN_H * DYN_H];
-  __shared__ double red[2][256];
+__global__ __launch_bounds__(256, 2) void k_les_dyn(int ny, int nz2, int nx2, int nseg, const double* __restrict__ Ph,
+                                                    const double* __restrict__ delta2, double* __restrict__ part,
+                                                    const double* __restrict__ ydist, float* __restrict__ X,
+                                                    double* __restrict__ scale) {
+  __shared__ double F[4][24][64];
+  __shared__ double red[2][4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int kk = blockIdx.y, nyp = ny + 1;
-  const long ps = (long)nz2 * nx2;
-  const int ntx = (nx2 + DYN_T - 1) / DYN_T;
-  const int tz0 = (blockIdx.x / ntx) * DYN_T, tx0 = (blockIdx.x % ntx) * DYN_T;
-  const bool inner = (kk > 0 && kk < ny);
+  const long ps = (long)nz2 * nx2, cs = (long)nyp * ps;
+  const int seg = blockIdx.x % nseg, sw = (nx2 + nseg - 1) / nseg;
+  const int x0 = seg * sw, xe = min(nx2, x0 + sw);
+  const int z0 = ((blockIdx.x / nseg) * 4 + wv) * DYN_Z, ze = min(nz2, z0 + DYN_Z);
+  const int xo = min(x0 - 1 + lane, xe);          // lanes past the right halo repeat it
+  const int x = xo < 0 ? nx2 - 1 : (xo >= nx2 ? 0 : xo);
+  const bool own = lane >= 1 && x0 - 1 + lane < xe;
   double lm = 0.0, mm = 0.0;
-  if (inner) {
-    for (int p = threadIdx.x; p < DYN_H * DYN_H; p += blockDim.x) {
-      const int hz = p / DYN_H, hx = p - hz * DYN_H;
-      int z = tz0 + hz - 1, x = tx0 + hx - 1;
-      z = (z < 0) ? z + nz2 : (z >= nz2 ? z - nz2 : z);
-      x = (x < 0) ? x + nx2 : (x >= nx2 ? x - nx2 : x);
-      const double* src = Ph + (long)kk * ps + (long)z * nx2 + x;
+  if (kk > 0 && kk < ny && z0 < ze) {
+    const double* plane = Ph + (long)kk * ps + x;
+    const double d2 = delta2[kk];
+    const int ll = max(lane - 1, 0), lr = min(lane + 1, 63);
+    auto row = [&](int z) { return plane + (long)(z < 0 ? z + nz2 : (z >= nz2 ? z - nz2 : z)) * nx2; };
+    double nx[LES_NF];   // the next row's fields
+    {
+      const double* src = row(z0 - 1);
+#pragma unroll
+      for (int f = 0; f < LES_NF; ++f) nx[f] = src[f * cs];
+    }
+    // row z, whose x-filtered fields go to r2 behind those of the two rows before
+    auto step = [&](int z, const double (&r0)[24], const double (&r1)[24], double (&r2)[24]) {
       double g[9], u[3];
 #pragma unroll
-      for (int f = 0; f < 9; ++f) g[f] = src[(long)f * nyp * ps];
+      for (int f = 0; f < 9; ++f) g[f] = nx[f];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) u[c] = src[(long)(9 + c) * nyp * ps];
-      const Strain S = strain(g);
+      for (int c = 0; c < 3; ++c) u[c] = nx[9 + c];
+      if (z < ze) {
+        const double* src = row(z + 1);
 #pragma unroll
-      for (int f = 0; f < 9; ++f) F[f][p] = g[f];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) F[9 + c][p] = u[c];
-#pragma unroll
-      for (int t = 0; t < 6; ++t) {
-        F[12 + t][p] = u[c_ti[t]] * u[c_tj[t]];
-        F[18 + t][p] = S.mag * S.s[t];
+        for (int f = 0; f < LES_NF; ++f) nx[f] = src[f * cs];
       }
-    }
-  }
-  __syncthreads();
-  if (inner) {
-    const int lz = threadIdx.x / DYN_T, lx = threadIdx.x - lz * DYN_T;
-    if (tz0 + lz < nz2 && tx0 + lx < nx2) {
-      auto filt = [&](int f) {
-        const double* a = F[f] + lz * DYN_H + lx;
-        const double r0 = 0.25 * a[0] + 0.5 * a[1] + 0.25 * a[2];
-        const double r1 = 0.25 * a[DYN_H] + 0.5 * a[DYN_H + 1] + 0.25 * a[DYN_H + 2];
-        const double r2 = 0.25 * a[2 * DYN_H] + 0.5 * a[2 * DYN_H + 1] + 0.25 * a[2 * DYN_H + 2];
-        return 0.25 * r0 + 0.5 * r1 + 0.25 * r2;
-      };
+      {
+        const Strain S = strain(g);
+#pragma unroll
+        for (int f = 0; f < 9; ++f) r2[f] = g[f];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) r2[9 + c] = u[c];
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+          r2[12 + t] = u[c_ti[t]] * u[c_tj[t]];
+          r2[18 + t] = S.mag * S.s[t];
+        }
+      }
+      if (FEAT && own && z >= z0 && z < ze) {
+        double n2 = 0.0;
+#pragma unroll
+        for (int f = 0; f < 9; ++f) n2 += g[f] * g[f];
+        const double gn = sqrt(n2);
+        const double inv = gn > 0.0 ? 1.0 / gn : 0.0;
+        const long p = (long)(kk - 1) * ps + (long)z * nx2 + x;
+#pragma unroll
+        for (int f = 0; f < 9; ++f) X[p * 10 + f] = (float)(g[f] * inv);
+        X[p * 10 + 9] = (float)ydist[kk];
+        scale[p] = d2 * n2;
+      }
+#pragma unroll
+      for (int f = 0; f < 24; ++f) F[wv][f][lane] = r2[f];
+      wave_sync();
+#pragma unroll
+      for (int f = 0; f < 24; ++f) r2[f] = 0.25 * F[wv][f][ll] + 0.5 * r2[f] + 0.25 * F[wv][f][lr];
+      wave_sync();
+      if (z <= z0) return;
+      auto filt = [&](int f) { return 0.25 * r0[f] + 0.5 * r1[f] + 0.25 * r2[f]; };
       double tg[9], tu[3], L[6], M[6];
 #pragma unroll
       for (int f = 0; f < 9; ++f) tg[f] = filt(f);
 #pragma unroll
       for (int c = 0; c < 3; ++c) tu[c] = filt(9 + c);
       const Strain St = strain(tg);
-      const double d2 = delta2[kk];
 #pragma unroll
       for (int t = 0; t < 6; ++t) {
         L[t] = filt(12 + t) - tu[c_ti[t]] * tu[c_tj[t]];
         M[t] = 2.0 * d2 * (filt(18 + t) - 4.0 * St.mag * St.s[t]);
       }
-      lm = contract(L, M);
-      mm = contract(M, M);
-      if (FEAT) {
-        const int hp = (lz + 1) * DYN_H + lx + 1;
-        double gp[9], n2 = 0.0;
+      lm += own ? contract(L, M) : 0.0;
+      mm += own ? contract(M, M) : 0.0;
+    };
+    double a[24], b[24], c[24];
 #pragma unroll
-        for (int f = 0; f < 9; ++f) {
-          gp[f] = F[f][hp];
-          n2 += gp[f] * gp[f];
-        }
-        const double gn = sqrt(n2);
-        const double inv = gn > 0.0 ? 1.0 / gn : 0.0;
-        const long p = (long)(kk - 1) * ps + (long)(tz0 + lz) * nx2 + tx0 + lx;
-#pragma unroll
-        for (int f = 0; f < 9; ++f) X[p * 10 + f] = (float)(gp[f] * inv);
-        X[p * 10 + 9] = (float)ydist[kk];
-        scale[p] = delta2[kk] * n2;
-      }
+    for (int f = 0; f < 24; ++f) a[f] = b[f] = c[f] = 0.0;
+    for (int z = z0 - 1; z <= ze; z += 3) {
+      step(z, a, b, c);
+      if (z + 1 <= ze) step(z + 1, b, c, a);
+      if (z + 2 <= ze) step(z + 2, c, a, b);
     }
   }
-  red[0][threadIdx.x] = lm;
-  red[1][threadIdx.x] = mm;
+  for (int o = 32; o > 0; o >>= 1) {
+    lm += __shfl_xor(lm, o, 64);
+    mm += __shfl_xor(mm, o, 64);
+  }
+  if (lane == 0) {
+    red[0][wv] = lm;
+    red[1][wv] = mm;
+  }
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      red[0][threadIdx.x] += red[0][threadIdx.x + o];
-      red[1][threadIdx.x] += red[1][threadIdx.x + o];
-    }
-    __syncthreads();
-  }
   if (threadIdx.x == 0) {
-    part[((long)kk * gridDim.x + blockIdx.x) * 2 + 0] = red[0][0];
-    part[((long)kk * gridDim.x + blockIdx.x) * 2 + 1] = red[1][0];
+    part[((long)kk * gridDim.x + blockIdx.x) * 2 + 0] = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+    part[((long)kk * gridDim.x + blockIdx.x) * 2 + 1] = red[1][0] + red[1][1] + red[1][2] + red[1][3];
   }
 }
+// x segments of a row, and workgroups per plane
+int dyn_segments(int nx2) { return (nx2 + DYN_X - 1) / DYN_X; }
+int dyn_blocks(int nz2, int nx2) { return dyn_segments(nx2) * (((nz2 + DYN_Z - 1) / DYN_Z + 3) / 4); }
 
 __global__ void k_les_cs2(int ny, int nblk, const double* __restrict__ part, double* __restrict__ cs2) {
   const int kk = blockIdx.x * blockDim.x + threadIdx.x;
   if (kk > ny) return;
   double lm = 0.0, mm = 0.0;
+#pragma unroll 4
   for (int b = 0; b < nblk; ++b) {
     lm += part[((long)kk * nblk + b) * 2 + 0];
     mm += part[((long)kk * nblk + b) * 2 + 1];
@@ -306,7 +328,7 @@ struct LesState {
   double beta = 1.0;
   chan_mlp* net = nullptr;
   long ps = 0, nm = 0, npts = 0;
-  int nblk = 0;                // Germano partial sums per plane (tiles of k_les_dyn)
+  int nblk = 0;                // Germano partial sums per plane (workgroups of k_les_dyn)
   double2* G = nullptr;        // [12][nyp][nm]
   double2* Zl = nullptr;       // [12 nyp][nz2][kxpad] transform intermediate
   double* Ph = nullptr;        // [12][nyp][ps]
@@ -356,11 +378,11 @@ void les_fields(chan_ctx* c, LesState* L, bool dynamic, bool feat = false) {
   if (!dynamic) return;
   const XZGeom& g = c->gd;
   if (feat)
-    hipLaunchKernelGGL(k_les_dyn<true>, dim3(L->nblk, nyp), dim3(256), 0, c->stream, ny, g.nz2, g.nx2, L->Ph,
-                       L->delta2, L->part, L->ydist, L->X, L->scale);
+    hipLaunchKernelGGL(k_les_dyn<true>, dim3(L->nblk, nyp), dim3(256), 0, c->stream, ny, g.nz2, g.nx2,
+                       dyn_segments(g.nx2), L->Ph, L->delta2, L->part, L->ydist, L->X, L->scale);
   else
-    hipLaunchKernelGGL(k_les_dyn<false>, dim3(L->nblk, nyp), dim3(256), 0, c->stream, ny, g.nz2, g.nx2, L->Ph,
-                       L->delta2, L->part, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL(k_les_dyn<false>, dim3(L->nblk, nyp), dim3(256), 0, c->stream, ny, g.nz2, g.nx2,
+                       dyn_segments(g.nx2), L->Ph, L->delta2, L->part, nullptr, nullptr, nullptr);
   LAUNCH_CHECK("k_les_dyn");
   hipLaunchKernelGGL(k_les_cs2, dim3((nyp + 63) / 64), dim3(64), 0, c->stream, ny, L->nblk, L->part, L->cs2);
   LAUNCH_CHECK("k_les_cs2");
@@ -454,7 +476,7 @@ int chan_les_configure(chan_ctx* c, int mode, chan_mlp* net, double beta, int ev
     L->ps = (long)g.nz2 * g.nx2;
     L->nm = (long)c->nxh * c->prm.nz;
     L->npts = (long)(ny - 1) * L->ps;
-    L->nblk = (int)(((g.nz2 + DYN_T - 1) / DYN_T) * ((g.nx2 + DYN_T - 1) / DYN_T));
+    L->nblk = dyn_blocks(g.nz2, g.nx2);
     const long zps = (long)g.nz2 * g.kxpad;
     lalloc(L->G, (size_t)LES_NF * nyp * L->nm);
     lalloc(L->Zl, (size_t)12 * nyp * zps);
