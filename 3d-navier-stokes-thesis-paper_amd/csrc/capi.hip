@@ -685,7 +685,7 @@ void ensemble_plan_batched(chan_ensemble* e) {
   std::map<int, int> xrw, xnxh;  // per length: rows per wavefront, largest nx/2+1
   for (chan_ctx* c : e->m) {
     const int M = c->gd.nx2 / 2;
-    const int r = e->xrows1 ? 1 : xpass_rows(M, c->gd.nz2, c->tune.xpass_rows, M <= 144);
+    const int r = e->xrows1 ? 1 : xpass_rows(M, c->gd.nz2, c->tune.xpass_rows, M <= 144, false, false, 0);
     xrw[M] = xrw.count(M) ? std::min(xrw[M], r) : r;
     xnxh[M] = std::max(xnxh[M], c->nxh);
   }
@@ -1819,7 +1819,8 @@ int chan_autotune(chan_ctx* c, int steps, double* best_ms) {
     const bool pf = c->tune.xpass_prefetch == 1 && M <= 144;
     std::vector<int> rows_c = {0};
     for (int r : {1, 2, 4})
-      if (xpass_rows(M, c->gd.nz2, r, pf) == r && r != xpass_rows(M, c->gd.nz2, 0, pf))
+      if (xpass_rows(M, c->gd.nz2, r, pf, false, c->les != nullptr, c->prm.ny - 1) == r &&
+          r != xpass_rows(M, c->gd.nz2, 0, pf, false, c->les != nullptr, c->prm.ny - 1))
         rows_c.push_back(r);
     std::vector<int> seg_c;
     if (solve_wg_seg(c->prm.ny, 1)) seg_c.push_back(1);

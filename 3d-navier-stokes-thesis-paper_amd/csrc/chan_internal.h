@@ -304,8 +304,9 @@ void launch_xpass(const XZGeom& g, const double2* tw, const DevOps& ops, const X
                   hipStream_t s);
 bool xpass_batchable(int M);
 // z-rows per wavefront of the wave x-pass: `req` (1, 2, 4) where the length
-// has that kernel and nz2 is a multiple of it, otherwise the default
-int xpass_rows(int M, int nz2, int req, bool pf);
+// has that kernel and nz2 is a multiple of it, otherwise the default for a
+// launch of nplanes planes
+int xpass_rows(int M, int nz2, int req, bool pf, bool lin, bool les, int nplanes);
 void launch_xpass_batched(int M, bool lin, int rw, int nxh, const XBatchArgs* args, const BatchItem* items,
                           int nitems, hipStream_t s);
 long xpass_batched_resident(int M, bool lin, int rw, int nxh);

@@ -297,7 +297,7 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
   const int nz2 = g.nz2, kxp = g.kxpad, nxh = g.nxh;
   // a constant raw-row stride (M + 1 cells rounded up) where it costs no LDS, so that the
   // LDS offsets of the raw rows fold into the reads
-  const int rawn = (RW == 1 || M < 64) ? xpass_raw_cells(M + 1) : xpass_raw_cells(nxh);
+  const int rawn = (RW == 1 || M < 64) ? xpass_raw_cells(M + 1) : nxh;
   double2* rl = lds;
   load_tw2<M>(rl, tw + g.px.tw, tid, 256);
   __syncthreads();
@@ -347,6 +347,7 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
           for (int i = 0; i < (M + 64) / 64; ++i) {   // nxh <= M + 1
             if (64 * i >= nxh) break;
             const int idx = min(64 * i + lane, nxh - 1);
+            if (RW > 1 && M >= 64 && 64 * i + lane >= nxh) continue;   // the next row's cells follow
             __builtin_amdgcn_global_load_lds((const void*)(row + idx),
                                              (__attribute__((address_space(3))) void*)(RAW + (c * RW + r) * rawn + 64 * i),
                                              16, 0, 0);
@@ -761,24 +762,29 @@ __global__ __launch_bounds__(256, (xpass_w_waves<LIN, M, RW>())) void k_xpass_w_
 using XPassFn = void (*)(XZGeom, const double2*, DevOps, XPassArgs);
 using XPassBFn = void (*)(const XBatchArgs*, const BatchItem*);
 
-// Rows per wavefront with a kernel: 1 at every length, 2 for M <= 72 and 4
-// for M <= 24, the last two with the row prefetch only.
+// Rows per wavefront with a kernel: 1 at every length, 2 for M <= 72 and 96,
+// 4 for M <= 24, the last two with the row prefetch only.
 static bool xpass_rw_built(int M, int rw, bool pf) {
-  return rw == 1 || (pf && ((rw == 2 && M <= 72) || (rw == 4 && M <= 24)));
+  return rw == 1 || (pf && ((rw == 2 && (M <= 72 || M == 96)) || (rw == 4 && M <= 24)));
 }
 
-// The default: two rows per wavefront wherever that kernel is built.  The
-// pass issues vector instructions most of the time at these lengths (three
-// wavefronts per SIMD at 64x97x64 finish at 43, 54 and 66 thousand cycles in
-// the order of their age), and the transform tasks of one row of 24 to 72
-// pairs leave half of the lanes or more idle in every one of them.  A whole
-// step with one row and two: 32x129x64 238 and 198 us, 64x97x64 244 and 238,
-// 72x81x108 356 and 335, 96x193x96 811 and 739.
-int xpass_rows(int M, int nz2, int req, bool pf) {
+// The default.  The pass issues vector instructions most of the time at the
+// short lengths (three wavefronts per SIMD at 64x97x64 finish at 43, 54 and 66
+// thousand cycles in the order of their age), and the transform tasks of one
+// row leave half of the lanes or more idle in every one of them.  A whole step
+// with one row and two: 32x129x64 238 and 198 us, 64x97x64 244 and 238,
+// 72x81x108 356 and 335, 96x193x96 811 and 739.  Two rows of 96 pairs leave one
+// workgroup's registers and LDS twice per compute unit and pay where they
+// leave its plane ranges four planes or more: 128x65x64 296 and 304,
+// 128x200x64 724 and 713, 128x129x128 912 and 852.  With base-flow loads (lin)
+// the registers set the line, 64x65x64 188 and 183, 96x97x96 421 and 426; with
+// the stress loads (les), which wait behind the prefetch, one row and its four
+// wavefronts per SIMD hide more: 48x65x48 234 and 240, 64x97x64 388 and 406.
+int xpass_rows(int M, int nz2, int req, bool pf, bool lin, bool les, int nplanes) {
   auto ok = [&](int r) { return xpass_rw_built(M, r, pf) && nz2 % r == 0; };
   if (req > 0 && ok(req)) return req;
-  const int d = M <= 72 ? 2 : 1;
-  return ok(d) ? d : 1;
+  const bool two = les ? M <= 27 : lin ? M <= 48 : M <= 72 || (M == 96 && (long)nz2 / 8 * nplanes >= 4 * 512);
+  return two && ok(2) ? 2 : 1;
 }
 
 // LDS of a wavefront x-pass workgroup: the root table and, per wavefront, 4*rw
@@ -786,7 +792,7 @@ int xpass_rows(int M, int nz2, int req, bool pf) {
 // to 64 for one row per wavefront and below 64 pairs, of nxh cells rounded up
 // otherwise)
 size_t xpass_w_lds(int M, int rw, int nxh, bool pf) {
-  const int rawn = rw == 1 || M < 64 ? xpass_raw_cells(M + 1) : xpass_raw_cells(nxh);
+  const int rawn = rw == 1 || M < 64 ? xpass_raw_cells(M + 1) : nxh;
   return sizeof(double2) * (M + 4 * (4 * rw * fft_seq_cells(M) + (pf ? 3 * rw * rawn : 0)));
 }
 
@@ -805,7 +811,7 @@ static XPassFn xpass_w_fn(bool les, bool lin, bool pf, int rw) {
       if constexpr (N <= 24) {
         if (rw == 4) return xpass_w_variant<N, true, 4>(les, lin);
       }
-      if constexpr (N <= 72) {
+      if constexpr (N <= 72 || N == 96) {
         if (rw == 2) return xpass_w_variant<N, true, 2>(les, lin);
       }
       return rw == 1 ? xpass_w_variant<N, true, 1>(les, lin) : nullptr;
@@ -908,7 +914,7 @@ void launch_xpass(const XZGeom& g, const double2* tw, const DevOps& ops, const X
   if (a.wave && ct && M <= 192) {
     const bool pf = a.prefetch && M <= 144;
     if (a.tau && a.base) throw chan_error("the subgrid closure is not defined for the linearized pass");
-    const int rw = xpass_rows(M, g.nz2, a.rows, pf);
+    const int rw = xpass_rows(M, g.nz2, a.rows, pf, a.base != nullptr, a.tau != nullptr, nplanes);
     const size_t ldw = xpass_w_lds(M, rw, g.nxh, pf);
     XPassFn fn = nullptr;
 #define XPASSW_CASE(N)                                                                  \
