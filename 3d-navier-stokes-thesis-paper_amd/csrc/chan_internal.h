@@ -242,6 +242,7 @@ struct chan_ctx {
   size_t stage_bytes = 0;
   void* h_pin = nullptr;         // pinned host staging (hipHostMalloc)
   size_t pin_bytes = 0;
+  std::vector<hipEvent_t> copy_ev;   // of the piecewise copies to the host
   bool data1_is_nl = false;      // Fortran's data1 currently holds the NL term
   // The device dt as last set or read by the host; h_dt_known is cleared by
   // every entry point that may change dt on the device without reading it back.
