@@ -209,8 +209,7 @@ void dev_div(chan_ctx* c, const double* fx, const double* fy, const double* fz, 
   const long ips = (long)g.nz2 * g.nx2, aps = (long)g.nz2 * g.kxpad, ops_ = (long)g.nxh * g.nz;
   double2* A = c->d_AB;
   double2* B = c->d_AB + (long)np * aps;
-  launch_xr2c(g, c->d_tw, fy, fx, c->ops.kx, ips, A, aps, np, c->stream);
-  launch_xr2c(g, c->d_tw, fz, nullptr, c->ops.kx, ips, B, aps, np, c->stream);
+  launch_xr2c(g, c->d_tw, fy, fx, c->ops.kx, ips, A, aps, np, c->stream, fz, B);
   launch_zfwd(g, c->d_tw, A, B, aps, c->ops.kz, out, ops_, np, 0, c->stream);
 }
 
@@ -1470,8 +1469,7 @@ int chan_compute_divergence_of_fluxes_noalloc(chan_ctx* c, const double* fx, con
     double2* B = A + (long)np * aps;
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c->stream;
     const long ips = (long)g.nz2 * g.nx2, ops_ = (long)g.nxh * g.nz;
-    launch_xr2c(g, c->d_tw, fy, fx, c->ops.kx, ips, A, aps, np, s);
-    launch_xr2c(g, c->d_tw, fz, nullptr, c->ops.kx, ips, B, aps, np, s);
+    launch_xr2c(g, c->d_tw, fy, fx, c->ops.kx, ips, A, aps, np, s, fz, B);
     launch_zfwd(g, c->d_tw, A, B, aps, c->ops.kz, (double2*)cdata, ops_, np, 0, s);
   });
 }

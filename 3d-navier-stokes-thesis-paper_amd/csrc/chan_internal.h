@@ -280,8 +280,10 @@ void launch_zinv(const XZGeom& g, const double2* tw, const double2* in, long in_
                  int poff = 0);
 void launch_xc2r(const XZGeom& g, const double2* tw, const double2* Z, long z_ps, double* out,
                  long out_ps, int nplanes, hipStream_t s);
+// fz: a second output outz = F(fz) in the same launch
 void launch_xr2c(const XZGeom& g, const double2* tw, const double* fy, const double* fx,
-                 const double* kx, long in_ps, double2* out, long out_ps, int nplanes, hipStream_t s);
+                 const double* kx, long in_ps, double2* out, long out_ps, int nplanes, hipStream_t s,
+                 const double* fz = nullptr, double2* outz = nullptr);
 // The CFL number and dt of one channel (cfl_finalize_body); on = 0: nothing to do
 struct CflBatchArgs {
   DevOps ops;

@@ -200,8 +200,14 @@ __global__ __launch_bounds__(512) void k_xr2c(XZGeom g, const double2* __restric
                                                const double* __restrict__ fy,
                                                const double* __restrict__ fx,
                                                const double* __restrict__ kxv, long in_ps,
-                                               double2* __restrict__ out, long out_ps, int rows) {
+                                               double2* __restrict__ out, long out_ps, int rows,
+                                               const double* __restrict__ fz, double2* __restrict__ outz) {
   extern __shared__ double2 lds[];
+  if (blockIdx.z) {   // the second output: F(fz) alone
+    fy = fz;
+    fx = nullptr;
+    out = outz;
+  }
   const int tid = threadIdx.x, nthr = blockDim.x;
   const int M = NC > 0 ? NC : g.nx2 / 2, ss = NC > 0 ? fft_seq_cells(NC) : M + 1;
   const long P = blockIdx.y;
@@ -573,17 +579,23 @@ void launch_xc2r(const XZGeom& g, const double2* tw, const double2* Z, long z_ps
 }
 
 void launch_xr2c(const XZGeom& g, const double2* tw, const double* fy, const double* fx,
-                 const double* kx, long in_ps, double2* out, long out_ps, int nplanes, hipStream_t s) {
+                 const double* kx, long in_ps, double2* out, long out_ps, int nplanes, hipStream_t s,
+                 const double* fz, double2* outz) {
   const int M = g.nx2 / 2;
-  const int nf = fx ? 2 : 1;
+  const int nf = fx ? 2 : 1, no = fz ? 2 : 1;
   const bool ct = fft2_split(M).n1 > 0;
   int rows = rows_for(M, g.nz2, nf, ct);
+  // A few planes: shorter workgroups, down to one point per thread of 256,
+  // until there are two per compute unit (the divergence of 8 planes of
+  // 96x96 15.0 us with them long and the second output in a launch of its own,
+  // 10.2 so).
+  while (rows % 2 == 0 && nf * rows * M > 256 && (long)(g.nz2 / rows) * nplanes * no < 512) rows /= 2;
   int nthr = std::min(512, std::max(64, ((nf * rows * M + 63) / 64) * 64));
   if (!ct) check_stage_fit(g.px, nf * rows, nthr);
-  dim3 grid(g.nz2 / rows, nplanes);
+  dim3 grid(g.nz2 / rows, nplanes, no);
   size_t lds = sizeof(double2) * (ct ? nf * rows * fft_seq_cells(M) + M : nf * rows * (M + 1));
 #define XR2C_CASE(N) \
-  hipLaunchKernelGGL(k_xr2c<N>, grid, dim3(nthr), lds, s, g, tw, fy, fx, kx, in_ps, out, out_ps, rows)
+  hipLaunchKernelGGL(k_xr2c<N>, grid, dim3(nthr), lds, s, g, tw, fy, fx, kx, in_ps, out, out_ps, rows, fz, outz)
   FFT_DISPATCH(M, XR2C_CASE)
 #undef XR2C_CASE
   LAUNCH_CHECK("k_xr2c");
