@@ -84,13 +84,21 @@ __global__ void k_ctrl_law(int npts, CtrlLaw w0, CtrlLaw w1) {
   w.out[i] = w.sgn * (w.ca * w.p2[i] + w.cb * w.p3[i] + w.add) / w.den;
 }
 
-// max |x| over n doubles into *out (bits of a nonnegative double)
-__global__ void k_absmax(long n, const double* x, unsigned long long* out) {
+// max |x| over n doubles into *out (bits of a nonnegative double).  One atomic
+// per workgroup, at most 512 of them: one per wavefront (8192 on one address)
+// took 96 us for the 1.2 million values of 64x97x64.
+__global__ __launch_bounds__(256) void k_absmax(long n, const double* __restrict__ x, unsigned long long* out) {
+  __shared__ double wm[4];
   double mx = 0.0;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    mx = fmax(mx, fabs(x[i]));
+#pragma unroll 4
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) mx = fmax(mx, fabs(x[i]));
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-  if ((threadIdx.x & 63) == 0) atomicMax(out, (unsigned long long)__double_as_longlong(mx));
+  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    mx = fmax(fmax(wm[0], wm[1]), fmax(wm[2], wm[3]));
+    atomicMax(out, (unsigned long long)__double_as_longlong(mx));
+  }
 }
 
 // Scale each (c, j) plane of a [3][ny+1][plane] complex array by the weight
@@ -164,7 +172,7 @@ void launch_ctrl_law(int npts, const CtrlLaw& w0, const CtrlLaw& w1, hipStream_t
 }
 
 void launch_absmax(long n, const double* x, unsigned long long* out, hipStream_t s) {
-  unsigned blocks = (unsigned)std::min<long>((n + 255) / 256, 2048);
+  unsigned blocks = (unsigned)std::min<long>((n + 255) / 256, 512);
   hipLaunchKernelGGL(k_absmax, dim3(blocks), dim3(256), 0, s, n, x, out);
   LAUNCH_CHECK("k_absmax");
 }
