@@ -598,11 +598,11 @@ __device__ __forceinline__ void sep_reduce(SepRow<NC>& e, double2 acl, double rb
   e.rB = pivot_rcp(e.B);
 }
 
-template <int SEG>
+template <int SEG, int MD>
 __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs& a, long bx) {
   extern __shared__ double2 sh[];
   const int tid = threadIdx.x;
-  const int s = tid / SOLVE_WG_MODES, q = tid % SOLVE_WG_MODES;
+  const int s = tid / MD, q = tid % MD;
   const long nm = (long)a.nxh * a.nz;
   const int ny = a.ny, nyp = ny + 1;
   const int ns = (nyp + SEG - 1) / SEG;   // segments
@@ -611,18 +611,18 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
   // start of the first one, whose row 0 is its row f.
   const int pad = ns * SEG - nyp, f = max(0, pad - (SEG - 3));
   const int rl = SEG - (pad - f);         // rows of the last segment
-  const int na = ns * SOLVE_WG_MODES;     // threads with rows
+  const int na = ns * MD;     // threads with rows
   const bool act = tid < na;
   double2* const E = sh;                             // exchange slots [6][na]
   double2* const NLS = sh + SOLVE_WG_SLOTS * na;     // this substep's NL rows [SEG][3][na]
   double2* const WL = NLS + 3 * SEG * na;            // wall values [u, v, w][bottom, top][8]
-  double2* const KL = WL + 6 * SOLVE_WG_MODES;       // kx, kz [8]
-  double2* const OP = KL + SOLVE_WG_MODES;           // the operators d2h .. dn as they are packed in memory
+  double2* const KL = WL + 6 * MD;       // kx, kz [8]
+  double2* const OP = KL + MD;           // the operators d2h .. dn as they are packed in memory
   const double* const d2h = reinterpret_cast<const double*>(OP);
   const double* const d2n = d2h + (ops.d2n - ops.d2h);
   const double* const dh = d2h + (ops.dh - ops.d2h);
   const double* const dn = d2h + (ops.dn - ops.d2h);
-  const long mg = bx * SOLVE_WG_MODES + q;
+  const long mg = bx * MD + q;
   const bool valid = act && mg < nm;
   const long m = (mg < nm) ? mg : nm - 1;
   const int ix = (int)(m / a.nz), iz = (int)(m - (long)ix * a.nz);
@@ -640,8 +640,8 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
   auto sel = [](bool c, double2 x, double2 y) { return make_double2(c ? x.x : y.x, c ? x.y : y.y); };
   auto put = [&](int k, double2 v) { if (act) E[k * na + tid] = v; };
   const int ti = act ? tid : 0;
-  const int tn = (act && s + 1 < ns) ? tid + SOLVE_WG_MODES : ti;   // the next segment's thread (or this one)
-  const int tp = (act && s > 0) ? tid - SOLVE_WG_MODES : ti;        // the previous segment's
+  const int tn = (act && s + 1 < ns) ? tid + MD : ti;   // the next segment's thread (or this one)
+  const int tp = (act && s > 0) ? tid - MD : ti;        // the previous segment's
   auto get = [&](int k, int t) { return E[k * na + t]; };
 
   // ---------------- every load of the kernel, none waited for before the last is issued ----------------
@@ -673,12 +673,12 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
   auto nls = [&](int c, int t) { return NLS[(t * 3 + c) * na + ti]; };
   if (first || last) {   // the segments with the wall rows fetch the wall data (cbc: top, then bottom)
     const double2* w = a.cbc + (first ? 3L : 0L) * nm + m;
-    double2* wl = WL + (first ? 0 : SOLVE_WG_MODES) + q;
+    double2* wl = WL + (first ? 0 : MD) + q;
     const double2 w0 = w[0], w1 = w[nm], w2 = w[2 * nm];
-    wl[0] = w0; wl[2 * SOLVE_WG_MODES] = w1; wl[4 * SOLVE_WG_MODES] = w2;
+    wl[0] = w0; wl[2 * MD] = w1; wl[4 * MD] = w2;
   }
   if (first) KL[q] = make_double2(kxv, kzv);
-  auto wall = [&](int c, int top) { return WL[(2 * c + top) * SOLVE_WG_MODES + q]; };
+  auto wall = [&](int c, int top) { return WL[(2 * c + top) * MD + q]; };
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wavefront's DMA rows are in LDS
   __syncthreads();                      // and the other wavefronts' operators
 
@@ -708,7 +708,7 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
       put(0, make_double2(part, 0.0));
       __syncthreads();
       double tmp = 0.0;
-      for (int k = 0; k < ns; ++k) tmp += E[k * SOLVE_WG_MODES + q].x;
+      for (int k = 0; k < ns; ++k) tmp += E[k * MD + q].x;
       __syncthreads();
       if (mean) {
         p_grad = -tmp + 0.5 * (a.dudy[ny - 1] - a.dudy[0]) / re;
@@ -846,7 +846,7 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
       __syncthreads();
       // rows past either end: the first separator's A and the last one's C
       // are zero, and stay so, so any row stands in for them
-      const int lo = (act && s >= d) ? tid - d * SOLVE_WG_MODES : ti, hi = (act && s + d < ns) ? tid + d * SOLVE_WG_MODES : ti;
+      const int lo = (act && s >= d) ? tid - d * MD : ti, hi = (act && s + d < ns) ? tid + d * MD : ti;
       const double2 rl_ = get(5, lo), rh_ = get(5, hi);
       const double2 Ghl[2] = {get(1, lo), get(2, lo)}, Ghh[2] = {get(1, hi), get(2, hi)};
       sep_reduce(eh, get(0, lo), rl_.x, Ghl, get(0, hi), rh_.x, Ghh);
@@ -927,7 +927,7 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
       __syncthreads();
       put(0, make_double2(ep.A, ep.C)); put(1, ep.G[0]); put(2, make_double2(ep.rB, 0.0));
       __syncthreads();
-      const int lo = (act && s >= d) ? tid - d * SOLVE_WG_MODES : ti, hi = (act && s + d < ns) ? tid + d * SOLVE_WG_MODES : ti;
+      const int lo = (act && s >= d) ? tid - d * MD : ti, hi = (act && s + d < ns) ? tid + d * MD : ti;
       const double2 Gl[1] = {get(1, lo)}, Gh[1] = {get(1, hi)};
       sep_reduce(ep, get(0, lo), get(2, lo).x, Gl, get(0, hi), get(2, hi).x, Gh);
     }
@@ -1092,9 +1092,13 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
   }
 }
 
-template <int SEG>
+// With four modes per workgroup the two that share 128-byte lines run on one
+// XCD (workgroups are dealt to the eight in turn), so that its L2 merges them.
+template <int SEG, int MD>
 __global__ __launch_bounds__(512) void k_solve_wg(DevOps ops, SolveArgs a) {
-  solve_wg_body<SEG>(ops, a, blockIdx.x);
+  int bx = blockIdx.x;
+  if (MD == 4 && (bx | 15) < (int)gridDim.x) bx = (bx & ~15) | ((bx & 7) << 1) | ((bx >> 3) & 1);
+  solve_wg_body<SEG, MD>(ops, a, bx);
 }
 
 // Batched form: workgroup i runs mode group it[i].bx of channel it[i].m.
@@ -1103,18 +1107,26 @@ __global__ __launch_bounds__(512) void k_solve_wg_b(const SBatchArgs* __restrict
                                                     const BatchItem* __restrict__ it) {
   const BatchItem w = it[blockIdx.x];
   const SBatchArgs& x = args[w.m];
-  solve_wg_body<SEG>(x.ops, x.a, w.bx);
+  solve_wg_body<SEG, SOLVE_WG_MODES>(x.ops, x.a, w.bx);
 }
 
 // LDS and threads of a k_solve_wg workgroup
-static size_t solve_wg_lds(int ny, int seg) {
-  const int nyp = ny + 1, na = ((nyp + seg - 1) / seg) * SOLVE_WG_MODES;
-  return sizeof(double2) * ((size_t)(SOLVE_WG_SLOTS + 3 * seg) * na + 7 * SOLVE_WG_MODES) +
+static size_t solve_wg_lds(int ny, int seg, int md = SOLVE_WG_MODES) {
+  const int nyp = ny + 1, na = ((nyp + seg - 1) / seg) * md;
+  return sizeof(double2) * ((size_t)(SOLVE_WG_SLOTS + 3 * seg) * na + 7 * md) +
          sizeof(double) * (4 * nyp + 4 * ny + 18);  // with dm(3,4) and the even padding between
 }
-static int solve_wg_threads(int ny, int seg) {
-  const int na = ((ny + seg) / seg) * SOLVE_WG_MODES;
+static int solve_wg_threads(int ny, int seg, int md = SOLVE_WG_MODES) {
+  const int na = ((ny + seg) / seg) * md;
   return (na + 63) / 64 * 64;
+}
+// Modes per workgroup of a single channel's launch: four where eight leave
+// one workgroup per compute unit and four leave two, whose load, solve and
+// store phases then overlap: 201 rows (128x200x64) 76.3 us with eight, 70.3
+// with four; 256x193x192 a whole run of 40 steps 136.1 and 133.2 ms.
+static int solve_wg_modes(int ny, int seg) {
+  auto two = [&](int md) { return solve_wg_threads(ny, seg, md) <= 256 && solve_wg_lds(ny, seg, md) <= 81920; };
+  return !two(SOLVE_WG_MODES) && two(4) ? 4 : SOLVE_WG_MODES;
 }
 
 // Rows per segment of the workgroup solve for ny+1 rows (0: none): the
@@ -1623,13 +1635,18 @@ void launch_solve(const DevOps& ops, const SolveArgs& a, hipStream_t s) {
   const bool off32 = 3.0 * (a.ny + 1) * (double)nm * 16.0 < 4.0e9;
   const int seg = a.seg ? solve_wg_seg(a.ny, a.seg) : 0;
   if (seg && off32) {
-    const dim3 gs((unsigned)((nm + SOLVE_WG_MODES - 1) / SOLVE_WG_MODES)), bs(solve_wg_threads(a.ny, seg));
-    const size_t lds = solve_wg_lds(a.ny, seg);
+    const int md = solve_wg_modes(a.ny, seg);
+    const dim3 gs((unsigned)((nm + md - 1) / md)), bs(solve_wg_threads(a.ny, seg, md));
+    const size_t lds = solve_wg_lds(a.ny, seg, md);
+#define SOLVE_CASE(S)                                                                                     \
+  if (md == 4) hipLaunchKernelGGL((k_solve_wg<S, 4>), gs, bs, lds, s, ops, a);                            \
+  else hipLaunchKernelGGL((k_solve_wg<S, SOLVE_WG_MODES>), gs, bs, lds, s, ops, a)
     switch (seg) {
-      case 3: hipLaunchKernelGGL((k_solve_wg<3>), gs, bs, lds, s, ops, a); break;
-      case 4: hipLaunchKernelGGL((k_solve_wg<4>), gs, bs, lds, s, ops, a); break;
-      default: hipLaunchKernelGGL((k_solve_wg<5>), gs, bs, lds, s, ops, a); break;
+      case 3: SOLVE_CASE(3); break;
+      case 4: SOLVE_CASE(4); break;
+      default: SOLVE_CASE(5); break;
     }
+#undef SOLVE_CASE
     LAUNCH_CHECK("k_solve_wg");
     return;   // it advances the time itself
   }
