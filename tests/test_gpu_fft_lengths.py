@@ -1,5 +1,6 @@
 """Transforms and nonlinear passes at the compile-time transform lengths with
-two or more factors of 3 (odd ones among them) against the oracle.
+two or more factors of 3 (odd ones among them) against the oracle, and two
+z-rows per wavefront where their raw rows follow each other unpadded.
 
 Bound: single calls agree to round-off as in test_gpu_parity.py (1e-12)."""
 import numpy as np
@@ -43,7 +44,8 @@ def test_transforms(nx, nx2, nz, nz2):
 @pytest.mark.parametrize("nx,nx2,nz,nz2,rows", [
     (24, 36, 18, 27, 0), (36, 54, 36, 54, 0), (36, 54, 36, 54, 1), (72, 108, 54, 81, 0), (72, 108, 36, 54, 2),
     (108, 162, 16, 24, 0), (144, 216, 108, 162, 0), (128, 256, 16, 16, 0), (216, 324, 16, 24, 0),
-    (54, 54, 18, 18, 0), (288, 432, 16, 24, 0), (324, 486, 16, 24, 0)])
+    (54, 54, 18, 18, 0), (288, 432, 16, 24, 0), (324, 486, 16, 24, 0),
+    (128, 192, 16, 24, 2), (192, 192, 16, 16, 2), (96, 144, 18, 24, 2), (144, 144, 18, 18, 2)])
 def test_nonlinear(nx, nx2, nz, nz2, rows, lin):
     g = O.make_grid(nx, 12, nz, nx2, nz2, 4.0, 2.0, 2000.0, stretch=1.5)
     rng = np.random.default_rng(nx * 1000 + nz + lin)
