@@ -251,6 +251,16 @@ __global__ __launch_bounds__(640) void k_xpass(XZGeom g, const double2* __restri
   }
 }
 
+// Two rows of 96 pairs keep the roots w_{2M}^n (n <= M) and the wavenumbers in
+// LDS tables instead of registers: of the 31 registers that went to scratch,
+// whose loads waited behind the prefetch, 5 are left.  A step at 128x129x128
+// 858 -> 827 us, 128x200x64 681 -> 665.  Level at one row of 192 pairs (17
+// registers in scratch) and two of 72 (13).
+__host__ __device__ constexpr bool xpass_tables(int M, int rw) { return rw == 2 && M == 96; }
+__host__ __device__ constexpr int xpass_table_cells(int M, int rw, int nxh) {
+  return xpass_tables(M, rw) ? M + 1 + (nxh + 1) / 2 : 0;
+}
+
 // ---------------------------------------------------------------------------
 // Wave-centric x-pass for the compile-time lengths M <= 192.  A wavefront
 // owns RW consecutive z-rows and walks a chunk of planes on its own: the
@@ -300,11 +310,18 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
   const int rawn = (RW == 1 || M < 64) ? xpass_raw_cells(M + 1) : nxh;
   double2* rl = lds;
   load_tw2<M>(rl, tw + g.px.tw, tid, 256);
+  constexpr bool TAB = xpass_tables(M, RW);
+  double2* const RT = lds + M;                                    // TAB: roots, then wavenumbers
+  double* const KX = reinterpret_cast<double*>(lds + M + M + 1);
+  if constexpr (TAB) {
+    for (int i = tid; i <= M; i += 256) RT[i] = tw[g.twx + i];
+    for (int i = tid; i < nxh; i += 256) KX[i] = ops.kx[i];
+  }
   __syncthreads();
   const int zb = (bx * 4 + wv) * RW;  // first z-row of the wavefront
   if (zb >= nz2) return;  // after the only workgroup barrier
   const long rowoff = (long)zb * kxp, prow = (long)zb * g.nx2;
-  double2* W = lds + M + wv * (4 * FS + (PF ? 3 * RW * rawn : 0));
+  double2* W = lds + M + xpass_table_cells(M, RW, nxh) + wv * (4 * FS + (PF ? 3 * RW * rawn : 0));
   double2* RAW = W + 4 * FS;
   const double2* rg = tw + g.px.tw;
   const double2* rootx = tw + g.twx;
@@ -319,7 +336,7 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
   // branch, so that the loads of a step are all issued before the first wait.
   int nq[PPL], pin[PPL], pout[PPL];
   bool vq[PPL];
-  double2 wc[PPL];
+  double2 wc[TAB ? 1 : PPL];
   auto rq = [&](int q) { return RW == 1 ? 0 : (vq[q] ? (lane + 64 * q) / M : 0); };
 #pragma unroll
   for (int q = 0; q < PPL; ++q) {
@@ -328,7 +345,7 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
     const int vv = vq[q] ? v : 0;
     const int r = RW == 1 ? 0 : vv / M, n = vv - r * M;
     nq[q] = n;
-    wc[q] = cconj(rootx[RW == 1 ? min(v, M) : n]);   // one row: also the root of output column v <= M
+    if (!TAB) wc[TAB ? 0 : q] = cconj(rootx[RW == 1 ? min(v, M) : n]);   // one row: also the root of output column v <= M
     pin[q] = r * SEQ + fft2_in_pos<M>(n);
     pout[q] = r * SEQ + fft2_out_pos<M>(n);
   }
@@ -394,12 +411,13 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
       for (int q = 0; q < PPL; ++q) {
         const int n = nq[q];
         const bool ha = n < nxh, hb = M - n < nxh, im = n != 0;
+        const double2 wq = TAB ? cconj(RT[n]) : wc[TAB ? 0 : q];
         double2 z[CB];
 #pragma unroll
         for (int c = 0; c < CB; ++c) {
           const double2 A = make_double2(ha ? ya[c][q].x : 0.0, ha && im ? ya[c][q].y : 0.0);
           const double2 B = make_double2(hb ? yb[c][q].x : 0.0, hb && im ? -yb[c][q].y : 0.0);
-          z[c] = c2r_combine(A, B, wc[q]);
+          z[c] = c2r_combine(A, B, wq);
         }
         if (vq[q]) {
 #pragma unroll
@@ -453,18 +471,22 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
   };
   auto ocol = [&](int i) { return min(lane + 64 * i, nout - 1) - orow(i) * nxh; };
   static_assert(RW > 1 || KP <= PPL, "the columns' roots are those of the pairs");
-  double2 rxl[RW == 1 ? 1 : KP];
-  double kxl[KP];
+  double2 rxl[RW == 1 || TAB ? 1 : KP];
+  double kxl[TAB ? 1 : KP];
+  if (!TAB) {
 #pragma unroll
-  for (int i = 0; i < KP; ++i) {
-    const int kq = ocol(i);
-    if (RW > 1) rxl[i] = rootx[kq];
-    kxl[i] = ops.kx[kq];
+    for (int i = 0; i < KP; ++i) {
+      const int kq = ocol(i);
+      if (RW > 1) rxl[RW == 1 || TAB ? 0 : i] = rootx[kq];
+      kxl[TAB ? 0 : i] = ops.kx[kq];
+    }
   }
   auto root_of = [&](int i, int kq) {
+    if (TAB) return RT[kq];
     if (i >= KP) return rootx[kq];
-    return RW == 1 ? cconj(wc[i < PPL ? i : 0]) : rxl[RW > 1 && i < KP ? i : 0];
+    return RW == 1 ? cconj(wc[!TAB && i < PPL ? i : 0]) : rxl[!TAB && RW > 1 && i < KP ? i : 0];
   };
+  auto kx_of = [&](int i, int kq) { return TAB ? KX[kq] : i < KP ? kxl[!TAB && i < KP ? i : 0] : ops.kx[kq]; };
   auto bufv = [&](int q) { return *reinterpret_cast<const double2*>(ops.buffer + poff(q)); };
   // Subgrid stress (LES): tau_ij is added to the flux u_i u_j wherever the
   // flux is formed, so the divergence of the fluxes carries -div(tau) with the
@@ -625,7 +647,7 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
         const int kq = ocol(i);
         const double2* S = W + orow(i) * SEQ;
         const double2 wk = root_of(i, kq);
-        const double kxv = i < KP ? kxl[i < KP ? i : 0] : ops.kx[kq];
+        const double kxv = kx_of(i, kq);
         const double2 X0 = r2c_post_nl<M>(S + 0 * FS, M, kq, wk), X1 = r2c_post_nl<M>(S + 1 * FS, M, kq, wk);
         const double2 X2 = r2c_post_nl<M>(S + 2 * FS, M, kq, wk), X3 = r2c_post_nl<M>(S + 3 * FS, M, kq, wk);
         Au[i - i0] = add_ik(X1, kxv, X0);
@@ -703,7 +725,7 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
         const int kq = ocol(i);
         const double2* S = W + orow(i) * SEQ;
         const double2 wk = root_of(i, kq);
-        const double kxv = i < KP ? kxl[i < KP ? i : 0] : ops.kx[kq];
+        const double kxv = kx_of(i, kq);
         Bw[i - i0] = r2c_post_nl<M>(S + 0 * FS, M, kq, wk);
         const double2 X5 = r2c_post_nl<M>(S + 1 * FS, M, kq, wk), X6 = r2c_post_nl<M>(S + 2 * FS, M, kq, wk);
         Av[i - i0] = add_ik(X6, kxv, X5);
@@ -775,8 +797,8 @@ static bool xpass_rw_built(int M, int rw, bool pf) {
 // with one row and two: 32x129x64 238 and 198 us, 64x97x64 244 and 238,
 // 72x81x108 356 and 335, 96x193x96 811 and 739.  Two rows of 96 pairs leave one
 // workgroup's registers and LDS twice per compute unit and pay where they
-// leave its plane ranges four planes or more: 128x65x64 296 and 304,
-// 128x200x64 724 and 713, 128x129x128 912 and 852.  With base-flow loads (lin)
+// leave its plane ranges four planes or more: 128x65x64 294 and 301,
+// 128x200x64 694 and 665, 128x129x128 912 and 827.  With base-flow loads (lin)
 // the registers set the line, 64x65x64 188 and 183, 96x97x96 421 and 426; with
 // the stress loads (les), which wait behind the prefetch, one row and its four
 // wavefronts per SIMD hide more: 48x65x48 234 and 240, 64x97x64 388 and 406.
@@ -793,7 +815,8 @@ int xpass_rows(int M, int nz2, int req, bool pf, bool lin, bool les, int nplanes
 // otherwise)
 size_t xpass_w_lds(int M, int rw, int nxh, bool pf) {
   const int rawn = rw == 1 || M < 64 ? xpass_raw_cells(M + 1) : nxh;
-  return sizeof(double2) * (M + 4 * (4 * rw * fft_seq_cells(M) + (pf ? 3 * rw * rawn : 0)));
+  return sizeof(double2) *
+         (M + xpass_table_cells(M, rw, nxh) + 4 * (4 * rw * fft_seq_cells(M) + (pf ? 3 * rw * rawn : 0)));
 }
 
 template <int N, bool PF, int RW>
