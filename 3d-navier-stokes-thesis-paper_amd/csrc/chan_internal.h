@@ -64,6 +64,16 @@ __device__ __forceinline__ T ldro(const T* p, long i) {
   return ((const __attribute__((address_space(4))) T*)p)[i];
 }
 
+// A pointer to device memory as one of the global address space.  A pointer
+// read from a table in memory is generic to the compiler: its accesses become
+// FLAT instructions, which count in vmcnt and in lgkmcnt and complete in no
+// stated order, so every wait for one is a wait for all, and a counted wait
+// behind one means nothing.
+template <class T>
+__device__ __forceinline__ T* as_global(T* p) {
+  return (T*)(__attribute__((address_space(1))) T*)(unsigned long long)p;   // a plain pair of casts is folded away
+}
+
 // Operators uploaded from the driver (layouts of the reference's globals).
 struct DevOps {
   const double* d2h;   // d2h(3, ny+1)

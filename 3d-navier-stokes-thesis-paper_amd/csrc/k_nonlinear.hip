@@ -375,7 +375,9 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
   };
   // The raw rows have landed.  Vector memory operations complete in the order
   // they were issued, so the `later` stores issued since the fetch need not
-  // have: waiting for them too would add their latency to every plane.
+  // have: waiting for them too would add their latency to every plane.  This
+  // holds for global and scratch accesses, not for FLAT ones (as_global): no
+  // pointer of this body may be generic.
   auto ready = [&](int later) {
     if constexpr (PF) {
       switch (later) {
@@ -773,11 +775,23 @@ __global__ __launch_bounds__(256, (xpass_w_waves<LIN, M, RW>())) void k_xpass_w(
 }
 
 // Batched form: workgroup i runs work-list entry it[i] of channel it[i].m.
+// The pointers of the entry go to the body as global ones: its counted waits
+// (ready) hold for global accesses only, and a FLAT load of a root or a
+// twiddle waited for the whole prefetch (60 steps of the 48-member ensemble
+// 333 ms with generic pointers, 308 so).
 template <bool LIN, int M, bool PF, int RW>
 __global__ __launch_bounds__(256, (xpass_w_waves<LIN, M, RW>())) void k_xpass_w_b(const XBatchArgs* __restrict__ args,
                                                     const BatchItem* __restrict__ it) {
   const BatchItem w = it[blockIdx.x];
-  const XBatchArgs& x = args[w.m];
+  XBatchArgs x = args[w.m];
+  x.tw = as_global(x.tw);
+  DevOps& o = x.ops;
+  for (const double** p : {&o.d2h, &o.d2n, &o.dm, &o.dh, &o.dn, &o.hn, &o.iu, &o.dyh, &o.dy, &o.kx, &o.kz, &o.buffer,
+                           &o.target, &x.a.base, &x.a.tau})
+    *p = as_global(*p);
+  x.a.Z = as_global(x.a.Z);
+  x.a.AB = as_global(x.a.AB);
+  x.a.cflbits = as_global(x.a.cflbits);
   xpass_w_body<LIN, M, PF, false, RW>(x.g, x.tw, x.ops, x.a, w.bx, w.by);
 }
 
