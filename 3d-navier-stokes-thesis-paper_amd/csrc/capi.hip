@@ -739,7 +739,7 @@ void ensemble_plan_batched(chan_ensemble* e) {
   std::map<int, int> xrw, xnxh;  // per length: rows per wavefront, largest nx/2+1
   for (chan_ctx* c : e->m) {
     const int M = c->gd.nx2 / 2;
-    const int r = e->xrows1 ? 1 : xpass_rows(M, c->gd.nz2, c->tune.xpass_rows, M <= 144, false, false, 0);
+    const int r = e->xrows1 ? 1 : xpass_batched_rows(M, c->gd.nz2, c->tune.xpass_rows);
     xrw[M] = xrw.count(M) ? std::min(xrw[M], r) : r;
     xnxh[M] = std::max(xnxh[M], c->nxh);
   }

@@ -320,6 +320,7 @@ bool xpass_batchable(int M);
 // has that kernel and nz2 is a multiple of it, otherwise the default for a
 // launch of nplanes planes
 int xpass_rows(int M, int nz2, int req, bool pf, bool lin, bool les, int nplanes);
+int xpass_batched_rows(int M, int nz2, int req);   // the same for the batched form, which has fewer
 void launch_xpass_batched(int M, bool lin, int rw, int nxh, const XBatchArgs* args, const BatchItem* items,
                           int nitems, hipStream_t s);
 long xpass_batched_resident(int M, bool lin, int rw, int nxh);

@@ -863,12 +863,21 @@ static XPassBFn xpass_wb_variant(bool lin) {
   return lin ? (XPassBFn)k_xpass_w_b<true, N, pf, RW> : (XPassBFn)k_xpass_w_b<false, N, pf, RW>;
 }
 
+// Rows per wavefront the batched form is built for: the single one's but two
+// rows of 96 pairs, which leave a compute unit one workgroup.
+static constexpr bool xpass_wb_built(int M, int rw) {
+  return rw == 1 || (rw == 2 && M <= 72) || (rw == 4 && M <= 24);
+}
+int xpass_batched_rows(int M, int nz2, int req) {
+  return xpass_rows(M, nz2, xpass_wb_built(M, req) ? req : 0, M <= 144, false, false, 0);
+}
+
 template <int N>
 static XPassBFn xpass_wb_fn(bool lin, int rw) {
-  if constexpr (N <= 24) {
+  if constexpr (xpass_wb_built(N, 4)) {
     if (rw == 4) return xpass_wb_variant<N, 4>(lin);
   }
-  if constexpr (N <= 72) {
+  if constexpr (xpass_wb_built(N, 2)) {
     if (rw == 2) return xpass_wb_variant<N, 2>(lin);
   }
   return rw == 1 ? xpass_wb_variant<N, 1>(lin) : nullptr;

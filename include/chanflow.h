@@ -254,8 +254,8 @@ int chan_jet_configure(chan_ctx* ctx, int wall, double amplitude, double radius,
  * the column fits a workgroup (ny up to about 280; keys 3, 4 and 8 then do
  * not apply), 12 z-rows per
  * wavefront of the wavefront x-pass (0, the default: by length; 1; 2 for
- * nx2/2 <= 72; 4 for nx2/2 <= 24; with the prefetch, where nz2 is a multiple;
- * otherwise the default applies; a batched ensemble takes the fewest rows its
+ * nx2/2 <= 72 and, outside a batched ensemble, 96; 4 for nx2/2 <= 24; with the
+ * prefetch, where nz2 is a multiple; otherwise the default applies; a batched ensemble takes the fewest rows its
  * members of one length choose).
  * chan_autotune times `steps` timesteps of every candidate (keys 0 and 2,
  * key 0 fixed at 1 while a subgrid closure is configured; with the wavefront

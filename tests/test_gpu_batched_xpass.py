@@ -25,6 +25,8 @@ def _member(nx, nx2, seed, rows):
     (48, 64, 2),     # 32 pairs, two rows
     (64, 64, 2),     # the same, undealiased in x: 33 columns a row
     (96, 128, 1),    # 64 pairs, one row
+    (128, 192, 2),   # 96 pairs, whose two rows only a single channel has
+    (128, 192, 4),   # and whose four rows none has
 ])
 def test_batched_against_single(nx, nx2, rows):
     mem = [_member(nx, nx2, s, rows) for s in (1, 2)]
