@@ -63,6 +63,14 @@ __device__ __forceinline__ void tile8_ts(int e, int& t, int& s) {
   s = (r & 3) | ((r >> 3) << 2);
 }
 
+// Lengths whose inter-pass twiddles the z-inverse forms in registers
+// (fft2p_rec): with no twiddle table, the 38 KB of LDS of a workgroup of 288
+// rows let four of them share a compute unit.  The products carry the root
+// table's rounding k1-fold, though: the lengths that took the runtime-planned
+// transform before, whose twiddles are all table values, keep a table, for an
+// error as small as theirs (162: 4.2e-16 with products, 2.8e-16 so).
+__host__ __device__ constexpr bool zinv_rec(int n) { return fft2_batched(n); }
+
 // (bx, by): the workgroup's kx group and plane row (blockIdx, or a work-list
 // entry of the batched form)
 template <int NC>
@@ -76,7 +84,6 @@ __device__ __forceinline__ void zinv_body(const XZGeom& g, const double2* __rest
   const long P = map_plane(pm, by);
   const int nz = g.nz, nz2 = NC > 0 ? NC : g.nz2, ss = fft_seq_cells(nz2);
   double2* rl = lds + ZT_KX * ss;
-  if constexpr (NC == 0) load_tw2<NC>(rl, tw + g.pz.tw, tid, nthr);
   const int ncol = min(ZT_KX, g.nxh - kx0);
   const double2* src = in + P * in_ps;
   const bool pad = (nz2 > nz) && !g.small;
@@ -94,9 +101,8 @@ __device__ __forceinline__ void zinv_body(const XZGeom& g, const double2* __rest
       v[i] = src[(long)(kx0 + sc) * nz + ps.idx];
       v[i] = pad_apply(v[i], ps, e < ZT_KX * NC && s < ncol);
     }
-    // the inter-pass twiddles are formed in registers (fft2p_rec): with no
-    // twiddle table, the workgroup's 38 KB of LDS let 4 workgroups share a CU
     __builtin_amdgcn_sched_barrier(0);  // keep the loads ahead of the first write
+    if constexpr (!zinv_rec(NC)) load_tw2<NC>(rl, tw + g.pz.tw, tid, nthr);
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       const int e = tid + i * nthr;
@@ -123,7 +129,8 @@ __device__ __forceinline__ void zinv_body(const XZGeom& g, const double2* __rest
     }
   }
   __syncthreads();
-  if constexpr (NC > 0) fft2p_rec<NC, 1>(lds, ss, ncol, tw + g.pz.tw, tid, nthr);  // the valid columns only
+  if constexpr (zinv_rec(NC)) fft2p_rec<NC, 1>(lds, ss, ncol, tw + g.pz.tw, tid, nthr);  // the valid columns only
+  else if constexpr (NC > 0) fft2p<NC, 1>(lds, ss, ncol, rl, tw + g.pz.tw, tid, nthr);
   else fft_run<NC, 1, FFT_MAXV>(lds, ss, ZT_KX, g.pz, tw, rl, tid, nthr);
   double2* dst = out + P * out_ps;
   for (int e = tid; e < nz2 * ZT_KX; e += nthr) {
@@ -516,7 +523,7 @@ void launch_zinv(const XZGeom& g, const double2* tw, const double2* in, long in_
   dim3 grid((g.nxh + ZT_KX - 1) / ZT_KX, nplanes);
   const int nthr = 256;
   if (!ct) check_stage_fit(g.pz, ZT_KX, nthr);
-  size_t lds = sizeof(double2) * ZT_KX * fft_seq_cells(g.nz2);  // no twiddle table (k_zinv)
+  const size_t lds = sizeof(double2) * (ZT_KX * fft_seq_cells(g.nz2) + (ct && !zinv_rec(g.nz2) ? g.nz2 : 0));
 #define ZINV_CASE(N) \
   hipLaunchKernelGGL(k_zinv<N>, grid, dim3(nthr), lds, s, g, tw, in, in_ps, out, out_ps, pm)
   FFT_DISPATCH(g.nz2, ZINV_CASE)
