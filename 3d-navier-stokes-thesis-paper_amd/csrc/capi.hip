@@ -640,10 +640,10 @@ std::string batch_ineligible(const chan_ctx* c, bool lin) {
   if (c->d_jet) return "a wall jet is configured";
   if (c->prm.ctrlu != 0.0 || c->prm.ctrlw != 0.0) return "wall feedback gains are set";
   if (lin && !c->d_base) return "no base flow (chan_set_baseflow)";
-  if (!zt_batchable(g.nz2)) return "nz2 has no compile-time transform plan";
-  if (!xpass_batchable(g.nx2 / 2)) return "nx2/2 has no wavefront x-pass";
+  if (!zt_batchable(g.nz2)) return "nz2 is none of " + batched_lengths(288);
+  if (!xpass_batchable(g.nx2 / 2)) return "nx2/2 is none of " + batched_lengths(192);
   if (g.nz > 192) return "nz above 192";
-  if (!solve_batchable(c->prm.ny)) return "ny+1 rows do not fit the segmented solve";
+  if (!solve_batchable(c->prm.ny)) return "ny+1 rows do not make 5 to 9 in each of at most 16 segments, 3 or more in the last";
   if (3.0 * c->nyp * (double)c->nmodes * 16.0 >= 4.0e9) return "the segmented solve's 32-bit offsets";
   const Tuning& t = c->tune;
   if (!(t.xpass_wave == 1 && t.zfwd_v2 == 1 && t.zinv_kx == 8 && (t.solve_seg == 1 || t.solve_seg == 3) &&

@@ -36,6 +36,14 @@ struct XZGeom {
   int twx;            // root-table offset for length nx2 (real pre/post twiddles)
 };
 
+// The lengths of fft2_batched up to `most`, for messages.
+inline std::string batched_lengths(int most) {
+  std::string s;
+  for (int n = 1; n <= most; ++n)
+    if (fft2_batched(n)) s += (s.empty() ? "" : ", ") + std::to_string(n);
+  return s;
+}
+
 // A batch of nseq transforms of the runtime-planned kind must fit the values a thread stages.
 inline void check_stage_fit(const FFTPlan& p, int nseq, int nthr) {
   for (int i = 0; i < p.nst; ++i) {

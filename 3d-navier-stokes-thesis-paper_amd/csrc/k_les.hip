@@ -463,7 +463,7 @@ int chan_les_configure(chan_ctx* c, int mode, chan_mlp* net, double beta, int ev
     if ((int)c->h_y.size() != c->prm.ny) throw chan_error("LES closure needs chan_set_coordinates");
     const XZGeom& g = c->gd;
     if (!(c->tune.xpass_wave && fft2_batched(g.nx2 / 2) && g.nx2 / 2 <= 192))
-      throw chan_error("the subgrid closure needs the wavefront x-pass (nx2/2 <= 192 of the form 2^a 3^b)");
+      throw chan_error("the subgrid closure needs the wavefront x-pass and nx2/2 one of " + batched_lengths(192));
     les_destroy(c->les);
     c->les = nullptr;
     LesState* L = new LesState();

@@ -956,7 +956,7 @@ void launch_xpass(const XZGeom& g, const double2* tw, const DevOps& ops, const X
     }
   const int nplanes = a.kb - a.ka + 1;
   if (a.tau && !(a.wave && fft2_batched(M) && M <= 192))
-    throw chan_error("the subgrid closure needs the wavefront x-pass (nx2/2 <= 192 of the form 2^a 3^b)");
+    throw chan_error("the subgrid closure needs the wavefront x-pass and nx2/2 one of " + batched_lengths(192));
   if (a.wave && ct && M <= 192) {
     const bool pf = a.prefetch && M <= 144;
     if (a.tau && a.base) throw chan_error("the subgrid closure is not defined for the linearized pass");

@@ -1169,7 +1169,9 @@ int solve_wg_seg(int ny, int solve_seg) {
 }
 
 // The columns a batched ensemble takes: ny + 1 rows in at most 16 segments of
-// 5..9 rows with 3 or more in the last one.
+// 5..9 rows with 3 or more in the last one.  The launches would take every ny
+// of solve_wg_seg (up to 269); what an ensemble accepts does not follow the
+// shape of the kernel.
 bool solve_batchable(int ny) {
   const int nyp = ny + 1;
   if (ny < 8) return false;
