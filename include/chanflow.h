@@ -251,7 +251,7 @@ int chan_jet_configure(chan_ctx* ctx, int wall, double amplitude, double radius,
  * ranges the nonlinear pass runs in turn (1..64; 1: every kernel over all
  * planes), 11 segmented column solve (1 on, the y column of a mode in segments
  * of 3, 4 or 5 rows by its length; 2 on with 5 rows; 3 as 1; 0 off) wherever
- * the column fits a workgroup (ny up to about 280; keys 3, 4 and 8 then do
+ * the column fits a workgroup (ny up to 269; keys 3, 4 and 8 then do
  * not apply), 12 z-rows per
  * wavefront of the wavefront x-pass (0, the default: by length; 1; 2 for
  * nx2/2 <= 72 and, outside a batched ensemble, 96; 4 for nx2/2 <= 24; with the
