@@ -281,8 +281,9 @@ __host__ __device__ constexpr int xpass_table_cells(int M, int rw, int nxh) {
 // LDS buffer by direct global-to-LDS loads (global_load_lds_dwordx4: lane i
 // writes cells base + i) as soon as the current rows have been consumed, so
 // their latency overlaps a whole plane of work instead of stalling the
-// wavefront at the start of every plane.  A raw row takes nxh cells (M + 1
-// with one row per wavefront, or below 64 pairs) rounded up to 64.
+// wavefront at the start of every plane.  A raw row takes M + 1 cells rounded
+// up to 64 with one row per wavefront or below 64 pairs, otherwise nxh cells:
+// the next row follows, so the lanes past a row's end are masked.
 //
 // What bounds it: LDS round trips and vector issue in turn (M = 144: two
 // wavefronts per SIMD, a forward transform phase of 2900 cycles of which
@@ -291,7 +292,7 @@ __host__ __device__ constexpr int xpass_table_cells(int M, int rw, int nxh) {
 // masked, which lets every load of a step issue before the first wait, and
 // the wait for the next raw rows leaves the stores behind them in flight.
 // x-pass at 256x193x192 (M = 192, rows read in place): 796 us with a branch
-// per cell and one wavefront per SIMD, 442 now; 32x65x32 16.6 and 14.8.
+// per cell and one wavefront per SIMD, 388 now; 32x65x32 16.6 and 15.5.
 //
 // (bx, by): the workgroup's group of 4*RW z-rows and its plane range
 // (blockIdx, or a work-list entry of the batched form)
@@ -764,7 +765,7 @@ __device__ __forceinline__ void xpass_w_body(const XZGeom& g, const double2* __r
 // scratch at M = 192 and two rows of 72), but one for the linearized pass of
 // 128 and more pairs, whose base flow would go there.  Three at two rows of
 // 36 or 48 cost 20 registers of scratch: 337 against 334 ms for 60 steps of
-// the 48-member ensemble.
+// the 48-member ensemble (with the generic pointers its kernels had then).
 template <bool LIN, int M, int RW>
 constexpr int xpass_w_waves() { return LIN && RW * M >= 128 ? 1 : 2; }
 
@@ -825,8 +826,7 @@ int xpass_rows(int M, int nz2, int req, bool pf, bool lin, bool les, int nplanes
 
 // LDS of a wavefront x-pass workgroup: the root table and, per wavefront, 4*rw
 // sequences and (with the prefetch) 3*rw raw rows (of M + 1 cells rounded up
-// to 64 for one row per wavefront and below 64 pairs, of nxh cells rounded up
-// otherwise)
+// to 64 for one row per wavefront and below 64 pairs, of nxh cells otherwise)
 size_t xpass_w_lds(int M, int rw, int nxh, bool pf) {
   const int rawn = rw == 1 || M < 64 ? xpass_raw_cells(M + 1) : nxh;
   return sizeof(double2) *

@@ -465,9 +465,9 @@ __device__ __forceinline__ double2 shfl2(double2 v, int src) {
 //  - Row accesses of 8 modes are whole 128-byte lines.  A copy of this
 //    kernel's loads and stores alone takes 109 us with 8 modes per row piece,
 //    147 us with 4 (64-byte pieces), 95 us with 16, whose workgroups are too
-//    large for the arithmetic's registers.  The whole kernel takes 139 us
-//    (3.9 TB/s); a form with 4 modes and 16 nine-row segments in one
-//    wavefront took 206 us.  201 rows (128x200x64) take 75 us, 334 us with
+//    large for the arithmetic's registers.  The whole kernel takes 136 us
+//    (4.0 TB/s); a form with 4 modes and 16 nine-row segments in one
+//    wavefront took 206 us.  201 rows (128x200x64) take 70 us, 334 us with
 //    the sweep-based k_solve3 that served columns above 144 rows before.
 //  - Two workgroups of four wavefronts share a compute unit (256 registers,
 //    75 KB of LDS each), so that one's loads and stores run beside the
@@ -501,11 +501,12 @@ __device__ __forceinline__ double2 quot(double2 g, double b, double rb) {
 
 // Rounding.  A column passes five or six reduction levels where sweeps pass
 // rows, so every sum takes its small terms first (for the low diffusion numbers
-// of the Helmholtz systems they round by little) and the quotients are corrected
-// (quot).  Against extended precision a substep's u, v, w, register and pressure
+// of the Helmholtz systems they round by little) and the quotients of the
+// Helmholtz systems are corrected (quot; in the Poisson system it changes no
+// error).  Against extended precision a substep's u, v, w, register and pressure
 // are then off by 0.97, 0.96, 0.96, 0.96 and 0.94 of what the sweeps are off (1.03,
-// 1.01, 1.02, 1.01 and 1.01 with the terms in their order and plain products),
-// for 0.5 to 1 % of a step's time at 64x97x64, none at 192x129x192.
+// 1.01, 1.02, 1.01 and 1.01 with the terms in their order and plain products).
+// A launch at 64x97x64 takes 21.3 us so and took 20.9, at 192x129x192 136 and 139.
 //
 // Partitioned solve of NC right-hand sides X[c][0..SEG) that share one
 // matrix, in pieces so that independent systems can be interleaved:
@@ -520,7 +521,7 @@ struct SegSys {
   double VL, VR;
 };
 
-template <int SEG, int NC, class CoefF>
+template <bool QUOT, int SEG, int NC, class CoefF>
 __device__ __forceinline__ void seg_eliminate(double2 (&X)[NC][SEG], SegSys<SEG, NC>& S, CoefF coef, bool last) {
   S.aT = 0.0; S.bT = 1.0; S.cT = 0.0;
 #pragma unroll
@@ -535,8 +536,10 @@ __device__ __forceinline__ void seg_eliminate(double2 (&X)[NC][SEG], SegSys<SEG,
     S.cp[t] = c_ * inv;
     S.gp[t] = (t == 0) ? (-a_) * inv : (-(a_ * S.gp[t - 1])) * inv;
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
-      X[c][t] = (t == 0) ? quot(X[c][t], bp, inv) : quot(csub(X[c][t], rmul(a_, X[c][t - 1])), bp, inv);
+    for (int c = 0; c < NC; ++c) {
+      const double2 g = (t == 0) ? X[c][t] : csub(X[c][t], rmul(a_, X[c][t - 1]));
+      X[c][t] = QUOT ? quot(g, bp, inv) : rmul(inv, g);
+    }
   }
   // the separator row itself: x = 0 + 0 * xl - (-1) * xr
   if (!last) {
@@ -829,7 +832,7 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
   {
     SegSys<SEG, 2> SH;
     SegSys<SEG, 1> SN;
-    seg_eliminate(UW, SH, [&](int t, double& a_, double& b_, double& c_) {
+    seg_eliminate<true>(UW, SH, [&](int t, double& a_, double& b_, double& c_) {
       const int j = j0 + t, jc = rowc(j);
       const bool wall = (j <= 0 || j >= ny);
       const double w = wall ? 0.0 : vis_imp;
@@ -837,7 +840,7 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
       b_ = -w * d2h[3 * jc + 1] + (wall ? 1.0 : alpha);
       c_ = -w * d2h[3 * jc + 2];
     }, !eq);
-    seg_eliminate(V, SN, [&](int t, double& a_, double& b_, double& c_) {
+    seg_eliminate<true>(V, SN, [&](int t, double& a_, double& b_, double& c_) {
       const int j = j0 + t, jv = min(rowc(j), ny - 1);
       const bool wall = (j <= 0 || j >= ny - 1);
       const double w = wall ? 0.0 : vis_imp;
@@ -918,7 +921,7 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
   const double alp = mean ? -1.0 : -k2;  // the mean mode has no pressure correction
   {
     SegSys<SEG, 1> SP;
-    seg_eliminate(PH, SP, [&](int t, double& a_, double& b_, double& c_) {
+    seg_eliminate<false>(PH, SP, [&](int t, double& a_, double& b_, double& c_) {
       const int jc = rowc(j0 + t);
       a_ = d2h[3 * jc]; b_ = d2h[3 * jc + 1] + alp; c_ = d2h[3 * jc + 2];
       // the Neumann rows 0, 1 and ny-1, ny, and identity rows beyond them
@@ -947,7 +950,7 @@ __device__ __forceinline__ void solve_wg_body(const DevOps& ops, const SolveArgs
       const double2 Gl[1] = {get(1, lo)}, Gh[1] = {get(1, hi)};
       sep_reduce(ep, get(0, lo), get(2, lo).x, Gl, get(0, hi), get(2, hi).x, Gh);
     }
-    ep.G[0] = quot(ep.G[0], ep.B, ep.rB);
+    ep.G[0] = rmul(ep.rB, ep.G[0]);
     put(3, ep.G[0]);
     __syncthreads();
     const double2 xl[1] = {get(3, tp)};
@@ -1138,8 +1141,8 @@ static int solve_wg_threads(int ny, int seg, int md = SOLVE_WG_MODES) {
 }
 // Modes per workgroup of a single channel's launch: four where eight leave
 // one workgroup per compute unit and four leave two, whose load, solve and
-// store phases then overlap: 201 rows (128x200x64) 76.3 us with eight, 70.3
-// with four; 256x193x192 a whole run of 40 steps 136.1 and 133.2 ms.
+// store phases then overlap: 201 rows (128x200x64) 79.8 us with eight, 70.0
+// with four; 256x193x192 369 and 352.
 static int solve_wg_modes(int ny, int seg) {
   auto two = [&](int md) { return solve_wg_threads(ny, seg, md) <= 256 && solve_wg_lds(ny, seg, md) <= 81920; };
   return !two(SOLVE_WG_MODES) && two(4) ? 4 : SOLVE_WG_MODES;
@@ -1148,11 +1151,11 @@ static int solve_wg_modes(int ny, int seg) {
 // Rows per segment of the workgroup solve for ny+1 rows (0: none): the
 // shortest of 3, 4, 5 that leaves room for two workgroups of at most 256
 // threads on a compute unit, else the longest that fits one.  A shorter
-// segment is a shorter serial chain: 66 rows take 16.4 us with 3 rows, 17.8
-// with 5 (64x65x64), 98 rows 20.5 with 4, 20.8 with 5 (64x97x64).  But 130
-// rows of 4 make 264 threads, one workgroup per compute unit: 197 us against
-// 155 (192x129x192, an earlier form of the kernel; its 6 rows took 233 us,
-// for want of registers).  The padding rows (pad) must leave 3 rows in the
+// segment is a shorter serial chain: 66 rows take 17.3 us with 3 rows, 18.7
+// with 5 (64x65x64), 98 rows 21.5 with 4, 22.3 with 5 (64x97x64).  But 130
+// rows of 4 make 264 threads with eight modes, so that only four share a
+// workgroup: 186 us against 136 (192x129x192; 6 rows 179, for want of
+// registers).  The padding rows (pad) must leave 3 rows in the
 // first and in the last segment, which 5 rows always do.
 int solve_wg_seg(int ny, int solve_seg) {
   if (ny < 8) return 0;

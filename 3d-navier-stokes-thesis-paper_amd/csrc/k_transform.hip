@@ -594,8 +594,8 @@ void launch_xr2c(const XZGeom& g, const double2* tw, const double* fy, const dou
   int rows = rows_for(M, g.nz2, nf, ct);
   // A few planes: shorter workgroups, down to one point per thread of 256,
   // until there are two per compute unit (the divergence of 8 planes of
-  // 96x96 15.0 us with them long and the second output in a launch of its own,
-  // 10.2 so).
+  // 96x96 14.6 us with them long and the second output in a launch of its own,
+  // 11.3 so).
   while (rows % 2 == 0 && nf * rows * M > 256 && (long)(g.nz2 / rows) * nplanes * no < 512) rows /= 2;
   int nthr = std::min(512, std::max(64, ((nf * rows * M + 63) / 64) * 64));
   if (!ct) check_stage_fit(g.px, nf * rows, nthr);
