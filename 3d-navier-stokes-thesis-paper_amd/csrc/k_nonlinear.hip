@@ -779,7 +779,7 @@ __global__ __launch_bounds__(256, (xpass_w_waves<LIN, M, RW>())) void k_xpass_w(
 // The pointers of the entry go to the body as global ones: its counted waits
 // (ready) hold for global accesses only, and a FLAT load of a root or a
 // twiddle waited for the whole prefetch (60 steps of the 48-member ensemble
-// 333 ms with generic pointers, 308 so).
+// 333 ms with generic pointers, 311 so).
 template <bool LIN, int M, bool PF, int RW>
 __global__ __launch_bounds__(256, (xpass_w_waves<LIN, M, RW>())) void k_xpass_w_b(const XBatchArgs* __restrict__ args,
                                                     const BatchItem* __restrict__ it) {

@@ -465,8 +465,8 @@ __device__ __forceinline__ double2 shfl2(double2 v, int src) {
 //  - Row accesses of 8 modes are whole 128-byte lines.  A copy of this
 //    kernel's loads and stores alone takes 109 us with 8 modes per row piece,
 //    147 us with 4 (64-byte pieces), 95 us with 16, whose workgroups are too
-//    large for the arithmetic's registers.  The whole kernel takes 136 us
-//    (4.0 TB/s); a form with 4 modes and 16 nine-row segments in one
+//    large for the arithmetic's registers.  The whole kernel takes 139 us
+//    (3.9 TB/s); a form with 4 modes and 16 nine-row segments in one
 //    wavefront took 206 us.  201 rows (128x200x64) take 70 us, 334 us with
 //    the sweep-based k_solve3 that served columns above 144 rows before.
 //  - Two workgroups of four wavefronts share a compute unit (256 registers,
@@ -506,7 +506,7 @@ __device__ __forceinline__ double2 quot(double2 g, double b, double rb) {
 // error).  Against extended precision a substep's u, v, w, register and pressure
 // are then off by 0.97, 0.96, 0.96, 0.96 and 0.94 of what the sweeps are off (1.03,
 // 1.01, 1.02, 1.01 and 1.01 with the terms in their order and plain products).
-// A launch at 64x97x64 takes 21.3 us so and took 20.9, at 192x129x192 136 and 139.
+// A launch at 64x97x64 takes 21.4 us so and took 20.9, at 192x129x192 139 either way.
 //
 // Partitioned solve of NC right-hand sides X[c][0..SEG) that share one
 // matrix, in pieces so that independent systems can be interleaved:
