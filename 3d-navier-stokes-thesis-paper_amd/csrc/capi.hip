@@ -1755,7 +1755,7 @@ int chan_plane_moments(chan_ctx* c, double* out) {
     if ((size_t)3 * cs * sizeof(double) > (size_t)2 * 3 * nyp * c->gd.nz2 * c->gd.kxpad * sizeof(double2))
       throw chan_error("plane_moments: physical planes do not fit the transform buffer");
     const size_t b = sizeof(double) * 15 * nyp;
-    if (!plane_moments_fused(g)) {
+    if (!plane_moments_fused(g, nyp)) {
       double* d = (double*)stage(c, b);
       dev_c2r(c, g, c->d_vel, 3 * nyp, (double*)c->d_AB);
       launch_plane_moments_points((const double*)c->d_AB, ps, cs, nyp, d, c->stream);

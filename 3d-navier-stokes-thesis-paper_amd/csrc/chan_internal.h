@@ -375,7 +375,7 @@ void launch_l2_modes(const XZGeom& g, const double2* vel, int nyp, const double*
 void launch_l2_final(const double* part, int n, double npts, const double* dudy, int ny, double* out, hipStream_t s);
 void launch_mass_flux(const double2* vel, long nm, int nyp, const double* dyh, double* out, hipStream_t s);
 void launch_mode_energy(const DevOps& ops, int ny, int nxh, int nz, const double2* vel, double* ke, hipStream_t s);
-bool plane_moments_fused(const XZGeom& g);
+bool plane_moments_fused(const XZGeom& g, int nyp);
 long plane_moments_part(const XZGeom& g, int nyp);
 void launch_plane_moments_points(const double* phys, long ps, long cs, int nyp, double* out, hipStream_t s);
 void launch_plane_moments(const XZGeom& g, const double2* tw, const double2* Z, long z_ps, int nyp, const double2* vel,

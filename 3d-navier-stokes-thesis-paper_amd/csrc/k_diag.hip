@@ -245,7 +245,8 @@ __global__ __launch_bounds__(64) void k_moments_final(const double* __restrict__
 }
 
 // The same from the points in memory, one workgroup per plane: for rows too
-// long for three of them in LDS (nx/2 above 2048).
+// long for three of them in LDS (nx/2 above 2048) and for many short ones
+// (plane_moments_fused).
 __global__ __launch_bounds__(256) void k_plane_moments(const double* __restrict__ phys, long ps, long cs, int nyp,
                                                        double* __restrict__ out) {
   __shared__ double red[4];
@@ -322,7 +323,15 @@ static int moments_rows(const XZGeom& g) {
     if (g.nz2 % d == 0 && d * M <= cap) best = d;
   return best;
 }
-bool plane_moments_fused(const XZGeom& g) { return g.nx2 / 2 <= 2048; }
+// Rows below 16 pairs take the runtime-planned transform, whose workgroups run
+// one to a compute unit: up to one round of them the fused form is 7 to 30 %
+// ahead, from the second on the points in memory are.  A call at nx = 16: 31.2 us
+// fused and 34.8 through memory at 66 planes of 32 rows (132 workgroups), 38.6 and
+// 34.9 at 130 (260), 68.2 and 57.4 at 501 (1002).
+bool plane_moments_fused(const XZGeom& g, int nyp) {
+  const int M = g.nx2 / 2;
+  return M <= 2048 && (M >= 16 || (long)nyp * (g.nz2 / moments_rows(g)) <= 256);
+}
 // Workgroups per plane: about a thousand in all, each with the same number of row groups but the last
 static int moments_blocks(const XZGeom& g, int nyp) {
   const int ng = g.nz2 / moments_rows(g), want = std::min(ng, std::max(1, 1024 / nyp)), per = (ng + want - 1) / want;
