@@ -1711,6 +1711,7 @@ int chan_l2_norm(chan_ctx* c, double* l2, double* drag) {
       lam[j] = 1.0 - yy * yy;
     }
     const bool modes = g.nx2 > c->prm.nx && g.nz2 > c->prm.nz;   // Parseval on a dealiased grid (k_l2_modes)
+    if (modes) check_c2r(g);   // no transform here, but no norm of a grid that has none
     const int np = modes ? l2_modes_parts(nyp) : 3 * nyp;
     char* s = (char*)stage(c, sizeof(double) * (nyp + np + 2) + 64);
     double* d_lam = (double*)s;

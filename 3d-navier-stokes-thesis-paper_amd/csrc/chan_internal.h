@@ -296,6 +296,7 @@ void xz_geom_init(XZGeom& g, int nx, int nz, int nx2, int nz2, int small, std::v
 void launch_zinv(const XZGeom& g, const double2* tw, const double2* in, long in_ps, double2* out,
                  long out_ps, int nplanes, hipStream_t s, int kx = 8, int pcnt = 0, int pstride = 0,
                  int poff = 0);
+void check_c2r(const XZGeom& g);
 void launch_xc2r(const XZGeom& g, const double2* tw, const double2* Z, long z_ps, double* out,
                  long out_ps, int nplanes, hipStream_t s);
 // fz: a second output outz = F(fz) in the same launch

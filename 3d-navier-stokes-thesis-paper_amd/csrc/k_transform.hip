@@ -570,12 +570,22 @@ static int rows_for(int M, int nz2, int nf, bool ct) {
   return best;
 }
 
+static int xc2r_threads(int M, int rows) { return std::min(512, std::max(64, ((rows * M + 63) / 64) * 64)); }
+
+// Refuses a grid whose transform to its points does not fit the workgroups of
+// launch_zinv and launch_xc2r.
+void check_c2r(const XZGeom& g) {
+  const int M = g.nx2 / 2, rows = rows_for(M, g.nz2, 1, false);
+  if (fft2_split(g.nz2).n1 == 0) check_stage_fit(g.pz, ZT_KX, 256);
+  if (fft2_split(M).n1 == 0) check_stage_fit(g.px, rows, xc2r_threads(M, rows));
+}
+
 void launch_xc2r(const XZGeom& g, const double2* tw, const double2* Z, long z_ps, double* out,
                  long out_ps, int nplanes, hipStream_t s) {
   const int M = g.nx2 / 2;
   const bool ct = fft2_split(M).n1 > 0;
   int rows = rows_for(M, g.nz2, 1, ct);
-  int nthr = std::min(512, std::max(64, ((rows * M + 63) / 64) * 64));
+  const int nthr = xc2r_threads(M, rows);
   if (!ct) check_stage_fit(g.px, rows, nthr);
   dim3 grid(g.nz2 / rows, nplanes);
   size_t lds = sizeof(double2) * (ct ? rows * fft_seq_cells(M) + M : rows * (M + 1));

@@ -1,5 +1,5 @@
 """What a batched ensemble and the subgrid closure refuse, and that the message
-says what they take."""
+says what they take; the diagnostics of a grid that no transform fits."""
 import pytest
 
 from helpers import chanflow, make_channel
@@ -29,4 +29,14 @@ def test_closure():
     ch = _channel(nx=36)
     with pytest.raises(chanflow().ChanError, match="needs the wavefront x-pass and nx2/2 one of " + LENGTHS):
         ch.les_configure("dynamic")
+    ch.close()
+
+
+@pytest.mark.parametrize("nz", [512, 486])
+def test_norm_of_a_grid_without_transforms(nz):
+    """The l2 norm needs no transform, but nothing else works on these grids."""
+    ch = _channel(ny=9, nz=nz)
+    for call in (ch.l2_norm, ch.initialize_flow, lambda: ch.step(1)):
+        with pytest.raises(chanflow().ChanError, match="FFT batch too large for workgroup"):
+            call()
     ch.close()
