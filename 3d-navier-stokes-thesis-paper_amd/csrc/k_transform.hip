@@ -68,7 +68,7 @@ __device__ __forceinline__ void tile8_ts(int e, int& t, int& s) {
 // rows let four of them share a compute unit.  The products carry the root
 // table's rounding k1-fold, though: the lengths that took the runtime-planned
 // transform before, whose twiddles are all table values, keep a table, for an
-// error as small as theirs (162: 4.2e-16 with products, 2.8e-16 so).
+// error as small as theirs (162: 4.2e-16 with products, 2.6e-16 so).
 __host__ __device__ constexpr bool zinv_rec(int n) { return fft2_batched(n); }
 
 // (bx, by): the workgroup's kx group and plane row (blockIdx, or a work-list
